@@ -1,0 +1,63 @@
+"""The one-workgroup SCF iteration (n <= 64) and its neighbour, the multi-launch form, against the CPU
+oracle's SCF, at sizes on both sides of the 16-wide tile edges: n = 7, 14, 28, 35, 49, 56, 63 (one workgroup)
+and 70 (multi-launch), with DIIS histories that take the register LU (up to 8), the LDS one (12) and none, and
+GHF at n = 14.  Bars: the energy to 1e-10 Eh (a converged SCF's error is second order in the density error,
+far below 1e-10 at the 1e-8 threshold), the orbitals as eigenvectors of the returned Fock matrix to 1e-9."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from zinq_amd import hip
+    c = hip.Context(0)
+    yield c
+    c.close()
+
+
+def _water(k):
+    from zinq_amd.molecules import water_system
+    s = water_system(k, basis="builtin:sto-3g")
+    return s, s.hcore(), s.overlap(), s.coulomb(), s.nrep()
+
+
+@pytest.mark.parametrize("k,diis", [(1, 8), (2, 8), (4, 8), (5, 3), (7, 8), (8, 12), (9, 8), (10, 8)])
+def test_scf_step_sizes(ctx, k, diis):
+    s, H, S, g, VN = _water(k)
+    o = s.nel // 2
+    ctx.eri_load_packed(s.coulomb_packed(), s.nbf)
+    ro = O.scf(H, S, g, VN, o, diis=diis, threshold=1e-8)
+    for fock in ("fp64", "fp32"):
+        r = ctx.scf(H, S, VN, o, diis=diis, threshold=1e-8, device=True, fock_precision=fock)
+        assert ctx.last_scf_driver() == "device"
+        print(f"n={s.nbf} diis={diis} {fock}: dE {r['E'] - ro['E']:+.1e} it {r['iterations']}/{ro['iterations']}", flush=True)
+        assert r["E"] == pytest.approx(ro["E"], abs=1e-10)
+        C, e = r["C"], r["e"]
+        np.testing.assert_allclose(C.T @ S @ C, np.eye(s.nbf), atol=1e-10)
+        np.testing.assert_allclose(r["F"] @ C, S @ C * e, atol=1e-9)
+
+
+@pytest.mark.parametrize("k", [1, 6])
+def test_scf_step_without_diis(ctx, k):
+    s, H, S, g, VN = _water(k)
+    o = s.nel // 2
+    ctx.eri_load_packed(s.coulomb_packed(), s.nbf)
+    ro = O.scf(H, S, g, VN, o, diis=None, threshold=1e-8)
+    r = ctx.scf(H, S, VN, o, diis=None, threshold=1e-8, device=True)
+    assert ctx.last_scf_driver() == "device" and r["iterations"] == ro["iterations"]
+    assert r["E"] == pytest.approx(ro["E"], abs=1e-10)
+
+
+def test_scf_step_ghf(ctx):
+    from zinq_amd.system import spin_block_1e, spin_block_2e
+    s, H, S, g, VN = _water(1)
+    Hs, Ss, gs = spin_block_1e(H), spin_block_1e(S), spin_block_2e(g)
+    ctx.eri_load(gs)
+    r = ctx.scf(Hs, Ss, VN, s.nel, generalized=True, device=True)
+    ro = O.scf(H, S, g, VN, s.nel // 2)
+    assert ctx.last_scf_driver() == "device"
+    assert r["E"] == pytest.approx(ro["E"], abs=1e-10)

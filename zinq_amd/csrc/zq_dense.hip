@@ -44,32 +44,13 @@
 #include <algorithm>
 
 #include "zq_internal.h"
+#include "zq_step.h"
 #include "zq_tile.h"
 
 namespace {
 
 using namespace zqt;
-
-// Sp2Bufs::est, in doubles: the fold bookkeeping kept across the SP2 runs of one device SCF.
-enum : int {
-  kEstValid = 0,      // 1: ref holds F' of a settled plain run, and kEstHomo / kEstLumo bound its HOMO / LUMO
-  kEstHomo = 1,       // upper bound of that run's HOMO energy
-  kEstLumo = 2,       // lower bound of its LUMO energy
-  kEstLastPlain = 3,  // 1: the last run was plain: ref holds its F', its traces are in the history
-  kEstLastLo = 4,     // and its Gershgorin interval
-  kEstLastHi = 5,
-  kEstFold = 6,       // this run folds, with the bounds kEstA0 (virtual) and kEstB0 (occupied) in X_0's scale
-  kEstA0 = 7,
-  kEstB0 = 8,
-  kEstSteps = 9,      // steps the last run recorded, and whether it settled
-  kEstSettled = 10,
-  kEstRuns = 11,      // since the SCF's first density: densities, folded ones, SP2 steps in all
-  kEstFolds = 12,
-  kEstStepSum = 13,
-  kEstRefSel = 14,    // which of the two n x n reference buffers holds F'_ref
-  kEstHist = 16,      // history[k] = {tr X_k, tr X_k^2, 1 for a down step, fold point}
-  kEstSize = kEstHist + 4 * kSp2MaxSteps
-};
+using namespace zqs;
 
 template <bool VEC>
 __global__ __launch_bounds__(64) void k_gemm_nt(const double *__restrict__ A, int lda, const double *__restrict__ B,
@@ -99,28 +80,6 @@ __device__ inline void tile_of(int t, int T, int &ti, int &tj) {
   tj = ti + t;
 }
 
-// HOMO (upper bound) and LUMO (lower bound) energies of the last plain run (steps steps, Gershgorin
-// interval [lo, hi]) from its trace history h (a copy in LDS of est + kEstHist).
-__device__ bool sp2_estimate(int steps, double lo, double hi, const double *h, int nocc, double &eh, double &el) {
-  int ks = -1;
-  for (int k = 0; k < steps && ks < 0; ++k)
-    if (h[4 * k] - h[4 * k + 1] < 1e-3) ks = k;
-  if (ks < 0) return false;
-  const double idem = h[4 * ks] - h[4 * ks + 1], d = h[4 * ks] - double(nocc), r = 4.0 * idem * idem + 1e-12;
-  double xl = fmin(fmax(0.5 * (idem + d) + r, 0.0), 1.0), xh = fmin(fmax(1.0 - (0.5 * (idem - d) + r), 0.0), 1.0);
-  for (int k = ks - 1; k >= 0; --k) {
-    if (h[4 * k + 2] != 0.0) {
-      xl = sqrt(xl), xh = sqrt(xh);
-    } else {
-      xl = 1.0 - sqrt(fmax(1.0 - xl, 0.0)), xh = 1.0 - sqrt(fmax(1.0 - xh, 0.0));
-    }
-  }
-  const double inv = 1.0 / fmax(hi - lo, 1e-10 * fmax(1.0, fabs(hi)));
-  eh = hi - xh / inv;
-  el = hi - xl / inv;
-  return el > eh;
-}
-
 // Gershgorin bounds of the symmetric n x n F (ld n): scal[0] = min_i (F_ii - R_i), scal[1] = max_i (F_ii + R_i).
 // kGershBlocks workgroups of 4 waves, one wave per row (global wave g takes rows g, g + 4 kGershBlocks,
 // ...): the lanes read the row coalesced and sum it with a butterfly.  Each workgroup leaves its
@@ -142,17 +101,9 @@ __global__ __launch_bounds__(256) void k_gershgorin(const double *__restrict__ F
   if (skip && *skip) return;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // the bookkeeping scalars are read before the rows, so that their latency hides behind the sums
-  double e_valid = 0.0, e_homo = 0.0, e_lumo = 0.0, e_lo = 0.0, e_hi = 0.0, e_runs = 0.0, e_folds = 0.0;
-  int e_steps = 0, sel = 0;
-  bool last_plain = false, pending = false;
-  if (track) {
-    e_valid = est[kEstValid], e_homo = est[kEstHomo], e_lumo = est[kEstLumo];
-    e_lo = est[kEstLastLo], e_hi = est[kEstLastHi], e_steps = int(est[kEstSteps]);
-    sel = int(est[kEstRefSel]) & 1;
-    e_runs = est[kEstRuns], e_folds = est[kEstFolds];
-    last_plain = est[kEstLastPlain] != 0.0;
-    pending = track == 2 && last_plain && est[kEstSettled] != 0.0;
-  }
+  FoldBook book{};
+  if (track) book = fold_book(est, track);
+  const int sel = book.sel;
   const double *rold = ref + size_t(sel) * n * n;
   double *rnew = ref + size_t(sel ^ 1) * n * n;
   double lo = 1e300, hi = -1e300, dd = 0.0, dm = 0.0;  // dm: the largest row sum of |F' - F'_ref|
@@ -174,7 +125,7 @@ __global__ __launch_bounds__(256) void k_gershgorin(const double *__restrict__ F
         const int j = j0 + 64 * u + lane;
         rsum += fabs(f[u]);
         const double df = f[u] - r[u];
-        if (track == 2) dd += df * df, rdif += fabs(df);
+        if (track == 2) dd = fma(df, df, dd), rdif += fabs(df);
         if (track && j < n) rnew[size_t(i) * n + j] = f[u];
       }
     }
@@ -198,8 +149,8 @@ __global__ __launch_bounds__(256) void k_gershgorin(const double *__restrict__ F
   if (!last_s) return;
   __threadfence();
   // the last plain run's history into LDS for the estimate
-  if (pending)
-    for (int e = threadIdx.x; e < 4 * e_steps; e += blockDim.x) hist_s[e] = est[kEstHist + e];
+  if (book.pending)
+    for (int e = threadIdx.x; e < 4 * book.steps; e += blockDim.x) hist_s[e] = est[kEstHist + e];
   __syncthreads();
   if (threadIdx.x == 0) {
     *gcount = 0u;
@@ -212,38 +163,10 @@ __global__ __launch_bounds__(256) void k_gershgorin(const double *__restrict__ F
     const double emin = glo - pad, emax = ghi + pad;
     scal[0] = emin;
     scal[1] = emax;
-    int fold = 0;
     if (track) {
-      double valid = track == 1 ? 0.0 : e_valid, eh = e_homo, el = e_lumo;
-      if (track == 2 && last_plain) {
-        // ref holds the last run's F': its history gives the bounds, when it settled
-        valid = 0.0;
-        if (pending && sp2_estimate(e_steps, e_lo, e_hi, hist_s, nocc, eh, el)) {
-          est[kEstHomo] = eh, est[kEstLumo] = el;
-          valid = 1.0;
-        }
-      }
-      est[kEstValid] = valid;
-      if (valid != 0.0) {
-        // ||F' - F'_ref||_2 is at most its Frobenius norm and at most its largest absolute row sum
-        // (F' symmetric); the row sum is often the smaller one early in an SCF.  A relative pad covers
-        // the rounding of both sums.
-        const double D = fmin(sqrt(dsum), dmax) * (1.0 + 1e-12);
-        const double lumo = el - D, homo = eh + D;
-        if (lumo - homo > 0.5 * (el - eh)) {
-          const double inv = 1.0 / fmax(emax - emin, 1e-10 * fmax(1.0, fabs(emax)));
-          fold = 1;
-          est[kEstA0] = fmin(fmax((emax - lumo) * inv, 0.0), 1.0);
-          est[kEstB0] = fmin(fmax((emax - homo) * inv, 0.0), 1.0);
-        }
-      }
-      est[kEstFold] = fold;
-      est[kEstLastPlain] = fold ? 0.0 : 1.0;
-      if (!fold) est[kEstRefSel] = double(sel ^ 1);
-      if (track == 1) e_runs = 0.0, e_folds = 0.0, est[kEstStepSum] = 0.0;
-      est[kEstRuns] = e_runs + 1.0;
-      est[kEstFolds] = e_folds + fold;
-      if (!fold) est[kEstLastLo] = emin, est[kEstLastHi] = emax;
+      double eh = 0.0, el = 0.0, a0, b0;
+      const bool found = book.pending && sp2_estimate(book.steps, book.lo, book.hi, hist_s, nocc, eh, el);
+      fold_decide(est, book, track, found, eh, el, emin, emax, dsum, dmax, a0, b0);
     }
   }
 }
@@ -255,7 +178,7 @@ __device__ inline void tile_partials(const double v[4], int ti, int tj, int i0, 
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     if (ti == tj && i0 + 4 * j + q == j0 + r) s1 += v[j];
-    s2 += v[j] * v[j];
+    s2 = fma(v[j], v[j], s2);
   }
   s1 = wave_sum(s1);
   s2 = wave_sum(s2);
@@ -330,12 +253,6 @@ __device__ inline void sp2_load(Sp2Ops<PRE> &o, const double *__restrict__ Xin, 
 // X_out tile = alpha X_in^2 + beta X_in + gamma I, stored with its mirror, and its partial traces in
 // pout[t].  Every wave of the workgroup calls it; PRE sums the waves' partial products in LDS, in wave
 // order, and wave 0 finishes the tile.
-// The polynomial of one step, X_(k+1) = alpha X_k^2 + beta X_k + gamma I; s is the fold point (0 plain).
-struct Sp2Map {
-  double alpha, beta, gamma, s;
-  bool down;
-};
-
 template <bool PRE>
 __device__ inline void sp2_finish(const Sp2Ops<PRE> &o, const double *__restrict__ Xin, double *__restrict__ Xout, int m,
                                   int ti, int tj, const Sp2Map &p, double2 *__restrict__ pout, int t) {
@@ -373,36 +290,6 @@ __device__ inline void sp2_finish(const Sp2Ops<PRE> &o, const double *__restrict
     if (ti != tj) Xout[size_t(col) * m + row] = v[j];
   }
   tile_partials(v, ti, tj, i0, j0, pout, t);
-}
-
-// The stop rule and the step's map from the summed partials (t1 = tr X_k, t2 = tr X_k^2 over the m x m
-// grid): count < 0 before idem < tol was first seen, then the number of steps taken since; the step that
-// brings count to 2 produces the settled projector.  Plain: X^2 or 2X - X^2, whichever keeps the trace
-// closer to N.  Folding (bounds a < b carried in a, b): the folded map of the side whose bound lags,
-// down when a > 1 - b, else up; both bounds go through it.  (The trace rule cannot choose between
-// folded maps: a folded down step lifts every eigenvalue near 0, the zero padding included, to
-// s^2/(1-s)^2, which makes its trace look worse than it is and keeps the iteration going up.)
-__device__ inline Sp2Map sp2_map(double t1, double t2, double tol, int nocc, int &count, bool fold, double &a,
-                                 double &b) {
-  const double N = double(nocc);
-  if (count < 0 && t1 - t2 < tol) count = 0;
-  if (count >= 0) ++count;
-  Sp2Map p;
-  if (!fold || !(b > a)) {
-    p.down = fabs(t2 - N) <= fabs(2.0 * t1 - t2 - N);
-    p.alpha = p.down ? 1.0 : -1.0, p.beta = p.down ? 0.0 : 2.0, p.gamma = 0.0, p.s = 0.0;
-    return p;
-  }
-  const double sd = 0.5 * a, su = 0.5 * (1.0 - b);
-  const double cd = 1.0 / (1.0 - sd), cu = 1.0 / (1.0 - su);
-  p.down = a > 1.0 - b;
-  if (p.down)
-    p.alpha = cd * cd, p.beta = -2.0 * sd * cd * cd, p.gamma = sd * sd * cd * cd, p.s = sd;
-  else
-    p.alpha = -cu * cu, p.beta = 2.0 * cu, p.gamma = 0.0, p.s = su;
-  a = p.alpha * a * a + p.beta * a + p.gamma;
-  b = p.alpha * b * b + p.beta * b + p.gamma;
-  return p;
 }
 
 __device__ inline void sum_partials(const double2 *__restrict__ pin, int ntiles, double &t1, double &t2) {

@@ -35,9 +35,12 @@
 #include "../../include/zinq_scf.h"
 #include "zq_internal.h"
 #include "zq_linalg.h"
+#include "zq_step.h"
 #include "zq_tile.h"
 
 namespace {
+
+using namespace zqs;
 
 constexpr int kRedBlocks = 64;
 
@@ -252,42 +255,6 @@ int sync_read(zq_ctx *ctx, const double *dsrc, double *host, size_t cnt) {
 // kernel of an iteration returns at once when state.done != 0, so the host can enqueue iteration k+1
 // before it has seen whether iteration k converged; it reads the state one iteration late.
 
-constexpr int kMaxHist = 16;
-
-struct ScfState {
-  int done;       // 0 running, 1 converged, 2 iteration limit reached, 3 SP2 did not settle in its budget
-  int it;         // iterations completed
-  int sp2_steps;  // SP2 steps of the last density
-  int sp2_max;    // most SP2 steps of any density so far
-  int hist_n, cur, combine;
-  int resets;          // singular DIIS systems met (the history reset to the current entry)
-  int hist[kMaxHist];  // DIIS slots, oldest first
-  int sp2[6];          // SP2 {count, steps} pairs, the settled buffer's parity, the abort flag
-  double e_old, e_new, rms, dE;
-  double coef[kMaxHist + 1];
-  double B[kMaxHist * kMaxHist];  // B[slot][slot] = <err_slot, err_slot'>
-};
-
-// Slot of the next iteration's error/Fock pair: the oldest when the history is full, else the lowest
-// free.  Taken at the end of the previous iteration (k_converge) or by k_state_init for the first.
-__device__ void diis_next_slot(ScfState *st, int diis) {
-  int slot;
-  if (st->hist_n >= diis) {
-    slot = st->hist[0];
-    for (int k = 1; k < st->hist_n; ++k) st->hist[k - 1] = st->hist[k];
-    --st->hist_n;
-  } else {
-    slot = 0;
-    for (bool used = true; used; ) {
-      used = false;
-      for (int k = 0; k < st->hist_n; ++k) used |= st->hist[k] == slot;
-      if (used) ++slot;
-    }
-  }
-  st->hist[st->hist_n++] = slot;
-  st->cur = slot;
-}
-
 __global__ void k_state_init(ScfState *st, double VN, int diis) {
   if (threadIdx.x != 0) return;
   st->done = 0, st->it = 0, st->sp2_steps = 0, st->sp2_max = 0;
@@ -328,67 +295,6 @@ __global__ __launch_bounds__(256) void k_dots_state(const double *__restrict__ h
     __syncthreads();
   }
   if (threadIdx.x == 0) part[blockIdx.y * kRedBlocks + blockIdx.x] = red[0];
-}
-
-// LU with partial pivoting and the triangular solves of the host zq::getrf/getrs, on one wave: row i
-// of A (n <= kLuMax) in LDS at A[i * kLuLd], b[i] in lane i's register.  Every element sees the same
-// operations in the same order as in the serial steps: the same pivot (the first row with the largest
-// |A[i][k]|), the same multipliers and updates, the forward sums in ascending j, the backward sums in
-// ascending j.  The rows of b are swapped as the pivots are found, which permutes b exactly as applying
-// the swaps afterwards does.  The loops run to n, not to kLuMax: the code stays small, which matters for
-// a kernel that runs once per iteration with its instructions not in the cache.  Returns false, on every
-// lane, for a zero pivot; otherwise lane i < n holds x[i] in b.
-constexpr int kLuMax = kMaxHist + 1;
-constexpr int kLuLd = kLuMax + 1;  // row stride of A in LDS
-
-// lane src's v on every lane; src is wave-uniform, so this is two v_readlane, not an LDS permute
-__device__ inline double lane_bcast(double v, int src) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), src),
-                          __builtin_amdgcn_readlane(__double2loint(v), src));
-}
-
-__device__ bool lu_solve_lds(int n, double *A, double &b) {
-  const int lane = threadIdx.x & 63;
-  for (int k = 0; k < n; ++k) {
-    // pivot: every lane scans column k in row order, so all find the same row
-    int p = k;
-    double best = fabs(A[k * kLuLd + k]);
-    for (int i = k + 1; i < n; ++i) {
-      const double v = fabs(A[i * kLuLd + k]);
-      if (v > best) best = v, p = i;
-    }
-    if (best == 0.0) return false;
-    p = __builtin_amdgcn_readfirstlane(p);
-    if (p != k) {
-      if (lane < n) {  // lane j swaps column j of rows k and p
-        const double rk = A[k * kLuLd + lane], rp = A[p * kLuLd + lane];
-        A[k * kLuLd + lane] = rp;
-        A[p * kLuLd + lane] = rk;
-      }
-      const double bk = lane_bcast(b, k), bp = lane_bcast(b, p);
-      b = lane == k ? bp : (lane == p ? bk : b);
-      __syncthreads();
-    }
-    if (lane > k && lane < n) {
-      const double f = A[lane * kLuLd + k] / A[k * kLuLd + k];
-      A[lane * kLuLd + k] = f;
-      for (int j = k + 1; j < n; ++j) A[lane * kLuLd + j] -= f * A[k * kLuLd + j];
-    }
-    __syncthreads();
-  }
-  for (int j = 0; j < n; ++j) {
-    const double bj = lane_bcast(b, j);
-    if (lane > j && lane < n) b -= A[lane * kLuLd + j] * bj;
-  }
-  for (int i = n - 1; i >= 0; --i) {
-    double acc = b;
-    for (int j = i + 1; j < n; ++j) {
-      const double bj = lane_bcast(b, j);
-      if (lane < n) acc -= A[lane * kLuLd + j] * bj;
-    }
-    if (lane == i) b = acc / A[i * kLuLd + i];
-  }
-  return true;
 }
 
 // E = sum of the energy partials + V_NN; DIIS: the new row of B, the bordered system, its LU solve
@@ -450,7 +356,7 @@ __global__ __launch_bounds__(64) void k_diis_solve(const double *__restrict__ pa
       Alu[lane * kLuLd + j] = lane < m ? (j < m ? Bs[lane * kMaxHist + j] : -1.0) : (j < m ? -1.0 : 0.0);
   double c = lane == m ? -1.0 : 0.0;
   __syncthreads();
-  if (lu_solve_lds(m + 1, Alu, c)) {
+  if (lu_solve(m + 1, Alu, c)) {
     if (lane < m) st->coef[lane] = c;
     if (lane == 0) st->combine = 1;
   } else if (lane == 0) {
@@ -554,6 +460,43 @@ int density_async(Dev &d, const double *A, int nocc, double factor, int nsteps, 
   return ZQ_OK;
 }
 
+// The one-workgroup form takes molecules up to n = 64.  A whole run, multi-launch / one workgroup, ms: n = 7
+// 1.24 / 0.66, n = 24 2.73 / 1.37, n = 48 3.27 / 2.20, n = 56 2.91 / 2.44.  Beyond that the FP64 matrix rate of
+// one compute unit costs what the launches did: n = 72 4.21 / 4.16, n = 96 5.27 / 6.76.
+constexpr int kStepMaxTiles = 4;
+bool step_fits(int n) { return n <= 16 * kStepMaxTiles; }
+
+// The fused form's workgroup: 512 threads, so that two waves share each SIMD and a wave may keep 256
+// registers (its tiles and its share of the matrices).
+constexpr int kStepThreads = 512;
+
+// scf_step of one molecule; an iteration whose state is already done only hands its mark to the host.
+template <int T>
+__global__ __launch_bounds__(kStepThreads) void k_scf_step(StepArgs a) {
+  extern __shared__ __attribute__((aligned(16))) double step_lds[];
+  __shared__ StepShared sh;
+  if (a.mode == kStepIter && a.st->done) {
+    if (threadIdx.x == 0) *a.done_out = a.st->done;
+    return;
+  }
+  StepBody<kStepThreads, T>::run(a, step_lds, sh);
+}
+
+int launch_step(zq_ctx *ctx, const StepArgs &a) {
+  const int T = (a.n + 15) / 16;
+  const size_t lds = step_lds_bytes(16 * T);
+  zq_prof_begin(ctx, "scf_step");
+  switch (T) {
+    case 1: hipLaunchKernelGGL(k_scf_step<1>, dim3(1), dim3(kStepThreads), lds, ctx->stream, a); break;
+    case 2: hipLaunchKernelGGL(k_scf_step<2>, dim3(1), dim3(kStepThreads), lds, ctx->stream, a); break;
+    case 3: hipLaunchKernelGGL(k_scf_step<3>, dim3(1), dim3(kStepThreads), lds, ctx->stream, a); break;
+    default: hipLaunchKernelGGL(k_scf_step<kStepMaxTiles>, dim3(1), dim3(kStepThreads), lds, ctx->stream, a); break;
+  }
+  zq_prof_end(ctx);
+  ZQ_LAUNCH_CHECK(ctx, "k_scf_step");
+  return ZQ_OK;
+}
+
 // Destroys the context's captured iterations.
 void drop_graphs(zq_ctx *ctx) {
   for (auto &kv : ctx->scf_graphs)
@@ -566,6 +509,8 @@ struct Run {
   double x_exch, factor, VN;
   const zq_scf_options *opt;
   bool mixed;  // incremental Fock builds from the FP32 ERI copy
+  bool fused = false;  // the iteration after the Fock build as one workgroup (scf_step)
+  StepArgs step{};     // its arguments
 };
 
 // Uploads S, X = L^-T, X^T, H; zeroes P.
@@ -586,6 +531,24 @@ int setup(Dev &d, const double *H, const double *S) {
   return ZQ_OK;
 }
 
+// Arguments of scf_step that do not change over the run, and its buffers.
+int step_args(const Dev &d, Run &r, ScfState *st) {
+  zq_ctx *ctx = d.ctx;
+  StepArgs &a = r.step;
+  a.st = st;
+  a.H = ctx->d_H, a.F = ctx->d_F, a.ldh = r.n;
+  a.P = ctx->d_P, a.dP = r.mixed ? d.dP : nullptr, a.ldp = r.np;
+  a.S = d.S, a.X = d.X, a.XT = d.XT, a.W = d.W, a.ldm = r.n;
+  a.Fh = d.Fh, a.Eh = d.Eh;
+  a.epart = d.epart, a.nep = ctx->Nb;
+  a.ref = (double *)zq_scratch(ctx, "sp2_ref", 2 * d.nn * sizeof(double));
+  a.est = (double *)zq_scratch(ctx, "sp2_est", kEstSize * sizeof(double));
+  if (!a.ref || !a.est) return zq_fail(ctx, ZQ_ERR_OOM, "SCF step buffers");
+  a.n = r.n, a.nocc = r.nocc, a.diis = r.opt->diis, a.maxit = r.opt->iterations;
+  a.factor = r.factor, a.VN = r.VN, a.thr = r.opt->threshold, a.err_scale = ctx->diis_err_scale;
+  return ZQ_OK;
+}
+
 // The kernels of one SCF iteration; every one of them returns at once while state.done != 0.
 int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *part_rms, int *host_done) {
   zq_ctx *ctx = d.ctx;
@@ -593,6 +556,14 @@ int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *pa
   const size_t nn = d.nn;
   const int gblocks = int(std::min<size_t>(1024, (nn + 255) / 256));
   const int *skip = &st->done;
+  if (r.fused) {
+    const int rc = r.mixed ? zq_fock_jk_device(ctx, d.dP, ctx->d_F, r.x_exch, ctx->d_F, skip, true, d.epart)
+                           : zq_fock_jk_device(ctx, ctx->d_P, ctx->d_H, r.x_exch, ctx->d_F, skip, false, d.epart);
+    if (rc) return rc;
+    StepArgs a = r.step;
+    a.mode = kStepIter, a.nsteps = budget, a.done_out = host_done;
+    return launch_step(ctx, a);
+  }
   // the reduce also leaves the energy partials (getEnergy) in d.epart; the DIIS slot of this iteration
   // was taken by the previous one's k_converge (or k_state_init)
   if (r.mixed) {
@@ -621,7 +592,7 @@ int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *pa
 // The asynchronous SCF.  Returns ZQ_OK with *status = state.done (1 converged, 2 iteration limit,
 // 3 SP2 budget exceeded: the caller reruns the synchronised driver), the final energy and iteration
 // count, and W = the last diagonalised Fock matrix.
-int scf_async(Dev &d, const Run &r, int *status, double *energy, int *iterations) {
+int scf_async(Dev &d, Run &r, int *status, double *energy, int *iterations) {
   zq_ctx *ctx = d.ctx;
   const int n = d.n, nocc = r.nocc;
   const size_t nn = d.nn;
@@ -644,12 +615,19 @@ int scf_async(Dev &d, const Run &r, int *status, double *energy, int *iterations
     if (!d.dP) return zq_fail(ctx, ZQ_ERR_OOM, "SCF dP");
     ZQ_TRY(ctx, hipMemsetAsync(d.dP, 0, size_t(r.np) * r.np * sizeof(double), ctx->stream));
   }
-  hipLaunchKernelGGL(k_state_init, dim3(1), dim3(64), 0, ctx->stream, st, r.VN, r.opt->diis);
   // core-Hamiltonian guess, src/hartree_fock.zig:425-431; W = H until the first iteration replaces it
-  ZQ_TRY(ctx, hipMemcpyAsync(d.W, ctx->d_H, nn * 8, hipMemcpyDeviceToDevice, ctx->stream));
-  if (int rc = density_async(d, ctx->d_H, nocc, r.factor, ctx->sp2_guess_budget, st, part_rms,
-                             r.mixed ? d.dP : nullptr, true))
-    return rc;
+  if (r.fused) {
+    if (int rc = step_args(d, r, st)) return rc;
+    StepArgs a = r.step;
+    a.mode = kStepGuess, a.nsteps = ctx->sp2_guess_budget;
+    if (int rc = launch_step(ctx, a)) return rc;
+  } else {
+    hipLaunchKernelGGL(k_state_init, dim3(1), dim3(64), 0, ctx->stream, st, r.VN, r.opt->diis);
+    ZQ_TRY(ctx, hipMemcpyAsync(d.W, ctx->d_H, nn * 8, hipMemcpyDeviceToDevice, ctx->stream));
+    if (int rc = density_async(d, ctx->d_H, nocc, r.factor, ctx->sp2_guess_budget, st, part_rms,
+                               r.mixed ? d.dP : nullptr, true))
+      return rc;
+  }
   // the incremental builds start from F = H (dP = P_0 after the guess)
   if (r.mixed) ZQ_TRY(ctx, hipMemcpyAsync(ctx->d_F, ctx->d_H, nn * 8, hipMemcpyDeviceToDevice, ctx->stream));
   const int budget = ctx->sp2_budget;
@@ -842,6 +820,7 @@ extern "C" int zq_scf_run_device(zq_ctx *ctx, size_t n_, size_t nocc_, const dou
   const int n = int(n_), nocc = int(nocc_), np = ctx->npad;
   const bool generalized = opt->generalized != 0;
   Run r{n, nocc, np, generalized ? 1.0 : 0.5, generalized ? 1.0 : 2.0, VN, opt, opt->fock_precision == ZQ_PREC_FP32};
+  r.fused = step_fits(n);
   const int maxh = opt->diis > 0 ? opt->diis : 1;
   Dev d;
   if (int rc = alloc(ctx, d, n, std::max(maxh, kMaxHist))) return rc;
