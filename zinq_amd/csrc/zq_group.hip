@@ -8,9 +8,10 @@
 //     F' = X^T F_ext X, SP2 purification -> D, P = 2 X D X^T       (geigh + getDensity, :621-640)
 //     rms(dP), |dE|, convergence test                            (:853-870)
 //   k_batch_count: molecules done, read by the host one iteration late.
+// The step is scf_step of zq_step.h, the one the device SCF of a small molecule runs, certified folds included.
 // Every per-molecule matrix lives in one workspace with leading dimension mp = n rounded up to 16 and
-// zero padding, so the small GEMMs (zq_tile.h, A B^T on FP64 MFMA, one wave per 16 x 16 tile) never
-// need bounds checks.  After convergence: F' of the last extrapolated F for each molecule, rocSOLVER
+// zero padding, so the small GEMMs of the eigenpair stage (zq_tile.h, A B^T on FP64 MFMA, one wave per
+// 16 x 16 tile) never need bounds checks.  After convergence: F' of the last extrapolated F for each molecule, rocSOLVER
 // dsyevd_strided_batched per distinct n, C = X V, and the MP2 energy from the OVOV transform of
 // zq_transform.hip through a context that views the molecule's resident quartets.
 
@@ -31,60 +32,34 @@
 #include "../../include/zinq_batch.h"
 #include "zq_internal.h"
 #include "zq_linalg.h"
+#include "zq_step.h"
 #include "zq_tile.h"
 
 using namespace zqt;
+using namespace zqs;
 
 namespace {
 
 constexpr int kMaxN = 96;
 constexpr int kHist = 8;
-constexpr int kMats = 13;
-enum { M_H, M_F, M_P, M_S, M_X, M_XT, M_W, M_T, M_FP, M_FPS, M_FPR, M_XS, M_X2 };
-enum { MODE_GUESS = 0, MODE_ITER = 1 };
+constexpr int kMats = 10;
+enum { M_H, M_F, M_P, M_S, M_X, M_XT, M_W, M_T, M_FP, M_FPR };
+// matrices of mp x mp in a molecule's workspace: the above, the DIIS history of F and of the error, and the
+// two buffers of the SP2 fold reference
+constexpr int kWsMats = kMats + 2 * kHist + 2;
+static_assert(kMaxN <= 16 * kStepTiles && kHist <= kMaxHist, "the step's limits");
 
 struct BMol {
-  long long ws;  // workspace offset (doubles): kMats + 2 kHist matrices of mp x mp
+  long long ws;  // workspace offset (doubles): kWsMats matrices of mp x mp
   int n, mp, nocc, pad;
   double VN;
 };
 
-struct BState {
-  int done, it, status, hist_n, cur, combine, sp2_steps, pad;
-  int hist[kHist];
-  double e_old, e_new, rms, dE;
-  double coef[kHist + 1];
-  double B[kHist * kHist];
+// What a run returns of a molecule's state.
+struct BResult {
+  double energy;
+  int it, done;  // done: 1 converged, 2 iteration limit, 3 an SP2 density did not settle
 };
-
-template <int NT>
-__device__ double block_sum(double v, double *red) {
-  v = wave_sum(v);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  __syncthreads();
-  if (lane == 0) red[w] = v;
-  __syncthreads();
-  double s = 0.0;
-#pragma unroll
-  for (int k = 0; k < NT / 64; ++k) s += red[k];
-  return s;
-}
-
-template <int NT>
-__device__ void block_minmax(double &lo, double &hi, double *red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = fmin(lo, __shfl_xor(lo, o, 64));
-    hi = fmax(hi, __shfl_xor(hi, o, 64));
-  }
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  __syncthreads();
-  if (lane == 0) red[w] = lo, red[NT / 64 + w] = hi;
-  __syncthreads();
-  lo = red[0], hi = red[NT / 64];
-#pragma unroll
-  for (int k = 1; k < NT / 64; ++k) lo = fmin(lo, red[k]), hi = fmax(hi, red[NT / 64 + k]);
-}
 
 // C = alpha A B^T, all mp x mp with leading dimension mp (mp a multiple of 16); the workgroup's waves
 // take the 16 x 16 tiles in turn.  Ends with a barrier.
@@ -101,270 +76,44 @@ __device__ void wg_gemm_nt(const double *A, const double *B, double *C, int mp, 
   __syncthreads();
 }
 
-// The 16 x 16 tile (i0, j0) of X X^T for the symmetric mp x mp X held in LDS (leading dimension ld):
-// lane l (r = l % 16, q = l / 16) supplies X[i0 + r][k + q] and X[j0 + r][k + q] to each
-// v_mfma_f64_16x16x4f64; accumulator element j is row i0 + 4 j + q, column j0 + r.
-__device__ inline d4 lds_tile_sq(const double *Xl, int ld, int mp, int i0, int j0) {
-  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-  const double *a = Xl + (i0 + r) * ld + q, *b = Xl + (j0 + r) * ld + q;
-  d4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int k = 0; k < mp; k += 4) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], b[k], acc, 0, 0, 0);
-  return acc;
-}
-
-// Bordered DIIS system (m + 1) x (m + 1) by LU with partial pivoting, the steps of zq::getrf/getrs.
-__device__ bool lu_solve(int n, double *A, double *b) {
-  int piv[kHist + 1];
-  for (int k = 0; k < n; ++k) {
-    int p = k;
-    double best = fabs(A[k * n + k]);
-    for (int i = k + 1; i < n; ++i)
-      if (fabs(A[i * n + k]) > best) best = fabs(A[i * n + k]), p = i;
-    piv[k] = p;
-    if (best == 0.0) return false;
-    if (p != k)
-      for (int j = 0; j < n; ++j) {
-        const double t = A[k * n + j];
-        A[k * n + j] = A[p * n + j], A[p * n + j] = t;
-      }
-    for (int i = k + 1; i < n; ++i) {
-      const double f = A[i * n + k] / A[k * n + k];
-      A[i * n + k] = f;
-      for (int j = k + 1; j < n; ++j) A[i * n + j] -= f * A[k * n + j];
-    }
-  }
-  for (int k = 0; k < n; ++k)
-    if (piv[k] != k) {
-      const double t = b[k];
-      b[k] = b[piv[k]], b[piv[k]] = t;
-    }
-  for (int i = 0; i < n; ++i)
-    for (int j = 0; j < i; ++j) b[i] -= A[i * n + j] * b[j];
-  for (int i = n - 1; i >= 0; --i) {
-    for (int j = i + 1; j < n; ++j) b[i] -= A[i * n + j] * b[j];
-    b[i] /= A[i * n + i];
-  }
-  return true;
-}
-
-// One SCF step (MODE_ITER) or the core-Hamiltonian guess (MODE_GUESS) of molecule order[blockIdx.x].
-// The SP2 iterate X lives in dynamic LDS (mp x (mp + 1) doubles, sized for the batch's largest mp) for
-// the whole step loop: each wave computes its 16 x 16 tiles of X^2 from LDS into registers, and after a
-// barrier writes its tiles' next X back in place.
+// One SCF step (kStepIter) or the core-Hamiltonian guess (kStepGuess) of molecule order[blockIdx.x]: scf_step
+// on its matrices.  Against the form before it (products on operands in L2, a serial DIIS solve, all tiles of
+// X^2 and no folds), per iteration of 96 molecules, n <= 72: 401 -> 198 us.
 template <int NT>
 __global__ __launch_bounds__(NT) void k_batch_step(double *__restrict__ ws, const BMol *__restrict__ mols,
-                                                   const int *__restrict__ order, BState *__restrict__ st,
-                                                   int *__restrict__ done, int mode, int diis, double thr, int maxit) {
-  __shared__ double red[2 * (NT / 64)];
-  extern __shared__ double Xl[];
-  __shared__ double Am[(kHist + 1) * (kHist + 1)], c[kHist + 1];  // the bordered DIIS system (thread 0)
-  const int mi = order[blockIdx.x], tid = threadIdx.x;
-  if (mode == MODE_ITER && done[mi]) return;
+                                                   const int *__restrict__ order, ScfState *__restrict__ st,
+                                                   double *__restrict__ est, int *__restrict__ done, int mode, int diis,
+                                                   double thr, int maxit) {
+  extern __shared__ __attribute__((aligned(16))) double step_lds[];
+  __shared__ StepShared sh;
+  const int mi = order[blockIdx.x];
+  if (mode == kStepIter && done[mi]) return;
   const BMol M = mols[mi];
-  BState &S = st[mi];
-  const int n = M.n, mp = M.mp;
-  const size_t mm = size_t(mp) * mp;
+  const size_t mm = size_t(M.mp) * M.mp;
   double *base = ws + M.ws;
-  double *H = base + M_H * mm, *F = base + M_F * mm, *P = base + M_P * mm, *Sm = base + M_S * mm;
-  double *X = base + M_X * mm, *XT = base + M_XT * mm, *W = base + M_W * mm, *T = base + M_T * mm;
-  double *FP = base + M_FP * mm, *FPS = base + M_FPS * mm, *Fpr = base + M_FPR * mm, *Xs = base + M_XS * mm;
-  double *Fh = base + kMats * mm, *Eh = Fh + kHist * mm;
-  const double *A = H;
+  StepArgs a{};
+  a.st = st + mi;
+  a.H = base + M_H * mm, a.F = base + M_F * mm, a.ldh = M.mp;
+  a.P = base + M_P * mm, a.ldp = M.mp;
+  a.S = base + M_S * mm, a.X = base + M_X * mm, a.XT = base + M_XT * mm, a.W = base + M_W * mm, a.ldm = M.mp;
+  a.Fh = base + kMats * mm, a.Eh = a.Fh + kHist * mm, a.ref = a.Eh + kHist * mm;
+  a.est = est + size_t(mi) * kEstSize;
+  a.done_out = done + mi;
+  a.n = M.n, a.nocc = M.nocc, a.diis = diis, a.maxit = maxit, a.nsteps = 100, a.mode = mode;
+  a.factor = 2.0, a.VN = M.VN, a.thr = thr, a.err_scale = 1.0;
+  switch (M.mp >> 4) {
+    case 1: StepBody<NT, 1>::run(a, step_lds, sh); break;
+    case 2: StepBody<NT, 2>::run(a, step_lds, sh); break;
+    case 3: StepBody<NT, 3>::run(a, step_lds, sh); break;
+    case 4: StepBody<NT, 4>::run(a, step_lds, sh); break;
+    case 5: StepBody<NT, 5>::run(a, step_lds, sh); break;
+    default: StepBody<NT, 6>::run(a, step_lds, sh); break;
+  }
+}
 
-  if (mode == MODE_GUESS) {
-    if (tid == 0) {
-      S.done = 0, S.it = 0, S.status = 0, S.hist_n = 0, S.cur = 0, S.combine = 0, S.sp2_steps = 0;
-      S.e_old = M.VN, S.e_new = M.VN, S.rms = 0.0, S.dE = 0.0;
-      done[mi] = 0;
-    }
-  } else {
-    // energy of P and F (F = H + G(P) from the grouped J/K)
-    double e = 0.0;
-    for (int x = tid; x < n * n; x += NT) {
-      const int i = x / n, j = x - i * n;
-      const size_t o = size_t(i) * mp + j;
-      e += 0.5 * P[o] * (H[o] + F[o]);
-    }
-    e = block_sum<NT>(e, red) + M.VN;
-    if (diis > 0) {
-      if (tid == 0) {
-        int slot;
-        if (S.hist_n >= diis) {
-          slot = S.hist[0];
-          for (int k = 1; k < S.hist_n; ++k) S.hist[k - 1] = S.hist[k];
-          --S.hist_n;
-        } else {
-          slot = 0;
-          for (bool used = true; used;) {
-            used = false;
-            for (int k = 0; k < S.hist_n; ++k) used |= S.hist[k] == slot;
-            if (used) ++slot;
-          }
-        }
-        S.hist[S.hist_n++] = slot;
-        S.cur = slot;
-      }
-      wg_gemm_nt<NT>(F, P, FP, mp, 1.0);    // F P   (P symmetric)
-      wg_gemm_nt<NT>(FP, Sm, FPS, mp, 1.0);  // F P S (S symmetric)
-      const int cur = S.cur, hn = S.hist_n;
-      double *Ec = Eh + cur * mm, *Fc = Fh + cur * mm;
-      for (size_t x = tid; x < mm; x += NT) {
-        const int i = int(x / mp), j = int(x - size_t(i) * mp);
-        Ec[x] = FPS[x] - FPS[size_t(j) * mp + i];
-        Fc[x] = F[x];
-      }
-      __syncthreads();
-      for (int k = 0; k < hn; ++k) {
-        const double *Ek = Eh + S.hist[k] * mm;
-        double d = 0.0;
-        for (size_t x = tid; x < mm; x += NT) d += Ec[x] * Ek[x];
-        d = block_sum<NT>(d, red);
-        if (tid == 0) S.B[cur * kHist + S.hist[k]] = S.B[S.hist[k] * kHist + cur] = d;
-      }
-      __syncthreads();
-      if (tid == 0) {
-        S.combine = 0;
-        if (hn >= 2) {
-          const int dd = hn + 1;
-          for (int i = 0; i < dd * dd; ++i) Am[i] = 0.0;
-          for (int i = 0; i < dd; ++i) c[i] = 0.0;
-          for (int i = 0; i < hn; ++i)
-            for (int j = 0; j < hn; ++j) Am[i * dd + j] = S.B[S.hist[i] * kHist + S.hist[j]];
-          for (int i = 0; i < hn; ++i) Am[i * dd + hn] = Am[hn * dd + i] = -1.0;
-          c[hn] = -1.0;
-          if (lu_solve(dd, Am, c)) {
-            for (int i = 0; i < hn; ++i) S.coef[i] = c[i];
-            S.combine = 1;
-          } else {
-            S.hist[0] = cur;
-            S.hist_n = 1;
-          }
-        }
-      }
-      __syncthreads();
-    }
-    const int comb = diis > 0 ? S.combine : 0, hn = S.hist_n;
-    for (size_t x = tid; x < mm; x += NT) {
-      const int i = int(x / mp), j = int(x - size_t(i) * mp);
-      if (!comb) {
-        W[x] = F[x];
-      } else if (j >= i) {
-        double a = 0.0, b = 0.0;
-        for (int k = 0; k < hn; ++k) {
-          const double *Fk = Fh + S.hist[k] * mm;
-          a += S.coef[k] * Fk[size_t(i) * mp + j];
-          b += S.coef[k] * Fk[size_t(j) * mp + i];
-        }
-        const double avg = (a + b) / 2;
-        W[size_t(i) * mp + j] = avg;
-        W[size_t(j) * mp + i] = avg;
-      }
-    }
-    if (tid == 0) S.e_new = e;
-    __syncthreads();
-    A = W;
-  }
-
-  // F' = X^T A X
-  wg_gemm_nt<NT>(XT, A, T, mp, 1.0);
-  wg_gemm_nt<NT>(T, XT, Fpr, mp, 1.0);
-  // SP2 on F' (Gershgorin bounds, trace-correcting steps; see zq_dense.hip)
-  double lo = 1e300, hi = -1e300;
-  for (int i = tid; i < n; i += NT) {
-    double rs = 0.0;
-    for (int j = 0; j < n; ++j) rs += fabs(Fpr[size_t(j) * mp + i]);
-    const double dgl = Fpr[size_t(i) * mp + i];
-    rs -= fabs(dgl);
-    lo = fmin(lo, dgl - rs), hi = fmax(hi, dgl + rs);
-  }
-  block_minmax<NT>(lo, hi, red);
-  const double pad = 1e-12 * fmax(fabs(lo), fabs(hi));
-  lo -= pad, hi += pad;
-  const double inv = 1.0 / fmax(hi - lo, 1e-10 * fmax(1.0, fabs(hi)));
-  const int ld = mp + 1;  // odd: the 16 rows of a tile fall in distinct LDS banks
-  double t1 = 0.0, t2 = 0.0;
-  for (size_t x = tid; x < mm; x += NT) {
-    const int i = int(x / mp), j = int(x - size_t(i) * mp);
-    double v = 0.0;
-    if (i < n && j < n) v = ((i == j ? hi : 0.0) - 0.5 * (Fpr[x] + Fpr[size_t(j) * mp + i])) * inv;
-    Xl[i * ld + j] = v;
-    t1 += (i == j) ? v : 0.0;
-    t2 += v * v;
-  }
-  t1 = block_sum<NT>(t1, red);
-  t2 = block_sum<NT>(t2, red);
-  const double N = double(M.nocc);
-  constexpr int NW = NT / 64, kTiles = (kMaxN / 16) * (kMaxN / 16), kPer = (kTiles + NW - 1) / NW;
-  const int Tt = mp >> 4, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q16 = lane >> 4;
-  int count = -1, steps = 0;
-  for (; steps < 100; ++steps) {
-    if (count >= 2) break;
-    if (count < 0 && t1 - t2 < 1e-9) count = 0;
-    if (count >= 0) ++count;
-    const bool sq = fabs(t2 - N) <= fabs(2.0 * t1 - t2 - N);
-    d4 acc[kPer];
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int t = wave + u * NW;
-      if (t < Tt * Tt) acc[u] = lds_tile_sq(Xl, ld, mp, (t / Tt) * 16, (t % Tt) * 16);
-    }
-    __syncthreads();  // every tile of X^2 is formed before X is overwritten
-    double a1 = 0.0, a2 = 0.0;
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int t = wave + u * NW;
-      if (t < Tt * Tt) {
-        const int ti = t / Tt, tj = t % Tt;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = ti * 16 + 4 * j + q16, c = tj * 16 + r16;
-          const double x2 = acc[u][j];
-          const double v = sq ? x2 : 2.0 * Xl[i * ld + c] - x2;
-          Xl[i * ld + c] = v;
-          a1 += (i == c) ? v : 0.0;
-          a2 += v * v;
-        }
-      }
-    }
-    t1 = block_sum<NT>(a1, red);  // its barriers also order the writes before the next step's reads
-    t2 = block_sum<NT>(a2, red);
-  }
-  if (count < 2) {  // no gap at the Fermi level: this molecule stops here
-    if (tid == 0) S.status = 3, S.done = 1, done[mi] = 1;
-    return;
-  }
-  for (size_t x = tid; x < mm; x += NT) {
-    const int i = int(x / mp), j = int(x - size_t(i) * mp);
-    Xs[x] = Xl[i * ld + j];
-  }
-  __syncthreads();
-  // P = 2 X D X^T, rms(dP)
-  wg_gemm_nt<NT>(X, Xs, T, mp, 1.0);
-  wg_gemm_nt<NT>(T, X, FP, mp, 2.0);
-  double s = 0.0;
-  for (size_t x = tid; x < mm; x += NT) {
-    const double dlt = FP[x] - P[x];
-    s += dlt * dlt;
-    P[x] = FP[x];
-  }
-  s = block_sum<NT>(s, red);
-  if (tid == 0) {
-    S.sp2_steps = steps;
-    if (mode == MODE_ITER) {
-      const double rms = sqrt(s / (double(n) * n));
-      const double dE = fabs(S.e_new - S.e_old);
-      S.e_old = S.e_new;
-      S.rms = rms, S.dE = dE;
-      const bool conv = S.it > 0 && dE < thr && rms < thr;
-      ++S.it;
-      if (conv) {
-        S.done = 1, S.status = 1;
-      } else if (S.it >= maxit) {
-        S.done = 1, S.status = 2;
-      }
-      done[mi] = S.done;
-    }
-  }
+__global__ void k_batch_result(const ScfState *__restrict__ st, int m, BResult *__restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < m) out[i] = BResult{st[i].e_new, st[i].it, st[i].done};
 }
 
 __global__ void k_batch_count(const int *__restrict__ done, int m, int *__restrict__ out) {
@@ -442,7 +191,9 @@ struct zq_batch {
   double *eri = nullptr, *ws = nullptr, *rec = nullptr;
   BMol *d_mols = nullptr;
   int *d_order = nullptr;  // molecules by descending padded size: the step kernel's workgroup order
-  BState *d_state = nullptr;
+  ScfState *d_state = nullptr;
+  double *d_est = nullptr;  // fold bookkeeping, kEstSize per molecule
+  BResult *d_res = nullptr;
   int *d_done = nullptr, *d_count = nullptr, *d_ptr = nullptr, *d_idx = nullptr;
   JKItem *d_items = nullptr;
   JKMol *d_jkm = nullptr;
@@ -450,7 +201,7 @@ struct zq_batch {
   int nitems = 0, nblk = 0;
   std::vector<long long> eri_off, ws_off;
   size_t eri_count = 0;  // doubles in eri
-  int mp_max = 16;       // largest padded size of the batch (the SP2 iterate's LDS)
+  int mp_max = 16;       // largest padded size of the batch (the step's LDS)
   int *h_count = nullptr;
   hipGraphExec_t graph = nullptr;
   std::string graph_key;
@@ -562,10 +313,11 @@ void free_all(zq_batch *b) {
   free_plan(b);
   free_eig(b);
   for (void *p : {(void *)b->eri, (void *)b->ws, (void *)b->d_mols, (void *)b->d_order, (void *)b->d_state,
-                  (void *)b->d_done, (void *)b->d_count, (void *)b->d_jkm, (void *)b->eri32, b->mp2_ws})
+                  (void *)b->d_est, (void *)b->d_res, (void *)b->d_done, (void *)b->d_count, (void *)b->d_jkm,
+                  (void *)b->eri32, b->mp2_ws})
     if (p) (void)hipFree(p);
   b->eri = nullptr, b->ws = nullptr, b->d_mols = nullptr, b->d_order = nullptr, b->d_state = nullptr;
-  b->d_done = nullptr;
+  b->d_est = nullptr, b->d_res = nullptr, b->d_done = nullptr;
   b->d_count = nullptr, b->d_jkm = nullptr, b->eri32 = nullptr, b->mp2_ws = nullptr, b->mp2_ws_bytes = 0;
   b->uploaded = false;
 }
@@ -637,7 +389,7 @@ int upload(zq_batch *b) {
     b->eri_off[m] = (long long)eri_total;
     b->ws_off[m] = (long long)ws_total;
     eri_total += nq * ZQ_QUARTET;
-    ws_total += (kMats + 2 * kHist) * mm;
+    ws_total += kWsMats * mm;
     canon_max = std::max(canon_max, h.eri.size());
     bm[m] = BMol{(long long)b->ws_off[m], h.n, mp, h.nocc, 0, h.VN};
     b->mp_max = std::max(b->mp_max, mp);
@@ -649,7 +401,9 @@ int upload(zq_batch *b) {
   BTRY(b, hipMalloc(&b->ws, ws_total * sizeof(double)));
   BTRY(b, hipMalloc(&b->d_mols, M * sizeof(BMol)));
   BTRY(b, hipMalloc(&b->d_order, M * sizeof(int)));
-  BTRY(b, hipMalloc(&b->d_state, M * sizeof(BState)));
+  BTRY(b, hipMalloc(&b->d_state, M * sizeof(ScfState)));
+  BTRY(b, hipMalloc(&b->d_est, M * kEstSize * sizeof(double)));
+  BTRY(b, hipMalloc(&b->d_res, M * sizeof(BResult)));
   BTRY(b, hipMalloc(&b->d_done, M * sizeof(int)));
   BTRY(b, hipMalloc(&b->d_count, sizeof(int)));
   BTRY(b, hipMalloc(&b->d_jkm, M * sizeof(JKMol)));
@@ -710,19 +464,19 @@ int upload(zq_batch *b) {
 
 void launch_step(zq_batch *b, int mode, int diis, double thr, int maxit) {
   const dim3 grid(unsigned(b->mols.size()));
-  const size_t lds = size_t(b->mp_max) * (b->mp_max + 1) * sizeof(double);  // the SP2 iterate
+  const size_t lds = step_lds_bytes(b->mp_max);
   if (b->nt == 512)
     hipLaunchKernelGGL(k_batch_step<512>, grid, dim3(512), lds, b->stream, b->ws, b->d_mols, b->d_order, b->d_state,
-                       b->d_done, mode, diis, thr, maxit);
+                       b->d_est, b->d_done, mode, diis, thr, maxit);
   else
     hipLaunchKernelGGL(k_batch_step<256>, grid, dim3(256), lds, b->stream, b->ws, b->d_mols, b->d_order, b->d_state,
-                       b->d_done, mode, diis, thr, maxit);
+                       b->d_est, b->d_done, mode, diis, thr, maxit);
 }
 
 int enqueue_iteration(zq_batch *b, int diis, double thr, int maxit) {
   BTRY(b, zq_jk_group(b->stream, b->eri, b->d_items, b->nitems, b->ws, 0.5, b->rec, b->d_jkm, b->d_done, b->d_ptr,
                       b->d_idx, b->d_blk, b->nblk, b->ws, b->ws));
-  launch_step(b, MODE_ITER, diis, thr, maxit);
+  launch_step(b, kStepIter, diis, thr, maxit);
   hipLaunchKernelGGL(k_batch_count, dim3(1), dim3(256), 0, b->stream, b->d_done, int(b->mols.size()), b->d_count);
   BTRY(b, hipGetLastError());
   return ZQ_OK;
@@ -842,7 +596,7 @@ int zq_batch_autotune(zq_batch *b, int chosen[2]) {
   best = 1e30f;
   for (int nt : {256, 512}) {
     b->nt = nt;
-    const float ms = time_it([&] { launch_step(b, MODE_GUESS, 8, 1e-8, 100); });
+    const float ms = time_it([&] { launch_step(b, kStepGuess, 8, 1e-8, 100); });
     if (ms < best) best = ms, best_nt = nt;
   }
   (void)hipEventDestroy(e0);
@@ -869,7 +623,7 @@ int zq_batch_run(zq_batch *b, const zq_scf_options *opt, int mp2_precision, doub
   };
 
   // core-Hamiltonian guess, then the captured iteration until every molecule is done
-  launch_step(b, MODE_GUESS, opt->diis, opt->threshold, opt->iterations);
+  launch_step(b, kStepGuess, opt->diis, opt->threshold, opt->iterations);
   char key[128];
   snprintf(key, sizeof key, "%d/%d/%d/%a/%d/%p", b->nt, b->chunk, opt->diis, opt->threshold, opt->iterations,
            (void *)b->d_items);
@@ -906,8 +660,9 @@ int zq_batch_run(zq_batch *b, const zq_scf_options *opt, int mp2_precision, doub
   BTRY(b, hipStreamSynchronize(b->stream));
   (void)hipEventDestroy(ev[0]);
   (void)hipEventDestroy(ev[1]);
-  std::vector<BState> hs(M);
-  BTRY(b, hipMemcpyAsync(hs.data(), b->d_state, M * sizeof(BState), hipMemcpyDeviceToHost, b->stream));
+  std::vector<BResult> hs(M);
+  hipLaunchKernelGGL(k_batch_result, dim3(unsigned((M + 255) / 256)), dim3(256), 0, b->stream, b->d_state, M, b->d_res);
+  BTRY(b, hipMemcpyAsync(hs.data(), b->d_res, M * sizeof(BResult), hipMemcpyDeviceToHost, b->stream));
   BTRY(b, hipStreamSynchronize(b->stream));
   b->stage_ms[0] = since(t0);
   const auto t1 = std::chrono::steady_clock::now();
@@ -1017,7 +772,7 @@ int zq_batch_run(zq_batch *b, const zq_scf_options *opt, int mp2_precision, doub
     std::vector<ZqGroupMol> gm;
     std::vector<int> which;
     for (int m = 0; m < M; ++m) {
-      if (hs[m].status != 1 && hs[m].status != 2) continue;
+      if (hs[m].done != 1 && hs[m].done != 2) continue;
       gm.push_back(ZqGroupMol{b->eri + b->eri_off[m], f32 ? b->eri32 + b->eri_off[m] : nullptr, b->mols[m].n,
                               b->mols[m].nocc, d_c + coff[m], d_w + woff[m]});
       which.push_back(m);
@@ -1047,7 +802,7 @@ int zq_batch_run(zq_batch *b, const zq_scf_options *opt, int mp2_precision, doub
         ZqGate gate;
         (void)hipSetDevice(b->device);
         for (int m; (m = next.fetch_add(1)) < M;) {
-          if (hs[m].status != 1 && hs[m].status != 2) continue;
+          if (hs[m].done != 1 && hs[m].done != 2) continue;
           bind_view(views[w], b, m);
           rc_m[m] = zq_mp2_device(views[w], b->h_c + coff[m], b->h_w + woff[m], b->mols[m].nocc, mp2_precision,
                                   &E_corr[m]);
@@ -1066,9 +821,9 @@ int zq_batch_run(zq_batch *b, const zq_scf_options *opt, int mp2_precision, doub
   for (int s = 0; s < M; ++s) info[order[s]] = b->h_info[s] ? 1 : 0;
   b->stage_ms[3] = since(t0);
   for (int m = 0; m < M; ++m) {
-    E_rhf[m] = hs[m].e_new;
+    E_rhf[m] = hs[m].energy;
     iterations[m] = hs[m].it;
-    status[m] = hs[m].status == 1 ? ZQ_OK : hs[m].status == 2 ? ZQ_ERR_NOT_CONVERGED : ZQ_ERR_LAPACK;
+    status[m] = hs[m].done == 1 ? ZQ_OK : hs[m].done == 2 ? ZQ_ERR_NOT_CONVERGED : ZQ_ERR_LAPACK;
     if (info[m] && status[m] == ZQ_OK) status[m] = ZQ_ERR_LAPACK;
     if (rc_m[m] != ZQ_OK && status[m] == ZQ_OK) status[m] = rc_m[m];
   }
