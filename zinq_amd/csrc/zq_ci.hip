@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -284,6 +285,7 @@ std::vector<Det> gen_dets(int nel, int nsp, const int *exc, size_t nexc, size_t 
 
 // The spin-orbital setting of one call: the FULL transform of the resident ERIs with C on the device.
 struct SoSetup {
+  ZqStage stage;  // C on its way to the device
   SoInts I{};
   int nel = 0;
 };
@@ -298,7 +300,7 @@ int so_setup(zq_ctx *ctx, const double *C, int nocc, int generalized, SoSetup &s
   void *d = nullptr;
   int dims[4];
   bool f32 = false;
-  if (int rc = zq_transform_device(ctx, C, 0, ZQ_BLOCK_FULL, ZQ_PREC_FP64, &d, dims, &f32)) return rc;
+  if (int rc = zq_transform_device(ctx, s.stage, C, 0, ZQ_BLOCK_FULL, ZQ_PREC_FP64, &d, dims, &f32)) return rc;
   s.I.g = (const double *)d;
   s.I.n = n, s.I.nsp = nsp, s.I.so = generalized ? 0 : 1;
   s.nel = nel;
@@ -336,14 +338,23 @@ extern "C" int zq_ao2mo_pp(zq_ctx *ctx, size_t n_, const double *A, const double
   auto *dT = (double *)zq_scratch(ctx, "pp_T", nn * 8, nullptr, false);
   auto *dO = (double *)zq_scratch(ctx, "pp_O", nn * 8, nullptr, false);
   if (!dA || !dC || !dT || !dO) return zq_fail(ctx, ZQ_ERR_OOM, "zq_ao2mo_pp buffers");
-  ZQ_TRY(ctx, hipMemcpyAsync(dA, A, nn * 8, hipMemcpyHostToDevice, ctx->stream));
-  ZQ_TRY(ctx, hipMemcpyAsync(dC, C, nn * 8, hipMemcpyHostToDevice, ctx->stream));
+  ZqStage st;
+  if (2 * nn <= kZqStageMax) {
+    if (int rc = st.take(ctx, 2 * nn)) return rc;
+    std::memcpy(st.host, A, nn * 8);
+    std::memcpy(st.host + nn, C, nn * 8);
+    zq_pad(ctx, st.dev, 1, n, n, dA);
+    zq_pad(ctx, st.dev + nn, 1, n, n, dC);
+  } else {
+    ZQ_TRY(ctx, hipMemcpyAsync(dA, A, nn * 8, hipMemcpyHostToDevice, ctx->stream));
+    ZQ_TRY(ctx, hipMemcpyAsync(dC, C, nn * 8, hipMemcpyHostToDevice, ctx->stream));
+  }
   // T[mu][q] = sum_nu A[mu][nu] C[nu][q]; out[p][q] = sum_mu C[mu][p] T[mu][q]
   if (int rc = zq_dgemm(ctx, dA, n, 1, dC, n, 1, dT, n, 1, n, n, n, "ao2mo_pp")) return rc;
   if (int rc = zq_dgemm(ctx, dC, 1, n, dT, n, 1, dO, n, 1, n, n, n, "ao2mo_pp")) return rc;
-  ZQ_TRY(ctx, hipMemcpyAsync(out, dO, nn * 8, hipMemcpyDeviceToHost, ctx->stream));
-  ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  return ZQ_OK;
+  const int rc = zq_read_back(ctx, dO, out, nn);
+  if (rc == ZQ_OK) st.done();
+  return rc;
 }
 
 extern "C" int zq_ci(zq_ctx *ctx, const double *H, const double *C, size_t nocc, int generalized, const int *excitations,
@@ -389,6 +400,7 @@ extern "C" int zq_ci(zq_ctx *ctx, const double *H, const double *C, size_t nocc,
   ZQ_TRY(ctx, hipMemcpyAsync(hw.data(), w, size_t(nd) * 8, hipMemcpyDeviceToHost, ctx->stream));
   ZQ_TRY(ctx, hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  s.stage.done();
   if (hinfo != 0) return zq_fail(ctx, ZQ_ERR_LAPACK, "zq_ci: eigensolver did not converge");
   for (size_t k = 0; k < nstates && k < size_t(nd); ++k) energies[k] = hw[k] + VN;
   return ZQ_OK;
@@ -449,6 +461,7 @@ extern "C" int zq_mp(zq_ctx *ctx, const double *C, const double *e, size_t nocc,
   double e00 = 0.0;
   ZQ_TRY(ctx, hipMemcpyAsync(&e00, E0, 8, hipMemcpyDeviceToHost, ctx->stream));
   ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  s.stage.done();
   hE[0] = e00;
   for (int k = 0; k <= order; ++k) energies[k] = hE[k];
   return ZQ_OK;

@@ -7,6 +7,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <thread>
 
 #include <shared_mutex>
@@ -87,6 +89,157 @@ void *zq_pinned(zq_ctx *ctx, const std::string &name, size_t bytes) {
   }
   b.bytes = bytes;
   return b.ptr;
+}
+
+namespace {
+// The pinned pool: free buffers by size (powers of two from 64 KB).
+struct PinPool {
+  std::mutex mu;
+  std::multimap<size_t, void *> free;
+  size_t kept = 0;
+  int users = 0;
+};
+constexpr size_t kPinKeep = size_t(64) << 20;
+PinPool &pin_pool() {
+  static PinPool *p = new PinPool;  // never destroyed: the runtime may be gone by the time statics are
+  return *p;
+}
+
+__global__ __launch_bounds__(256) void k_push(const double *__restrict__ src, size_t cnt, double *__restrict__ dst) {
+  for (size_t i = blockIdx.x * size_t(256) + threadIdx.x; i < cnt; i += size_t(gridDim.x) * 256) dst[i] = src[i];
+}
+}  // namespace
+
+void zq_stage_pool_users(int change) {
+  PinPool &p = pin_pool();
+  std::lock_guard<std::mutex> lock(p.mu);
+  p.users += change;
+  if (p.users > 0) return;
+  for (auto &kv : p.free) (void)hipHostFree(kv.second);
+  p.free.clear();
+  p.kept = 0;
+}
+
+int ZqStage::take(zq_ctx *c, size_t cnt) {
+  size_t want = size_t(64) << 10;
+  while (want < cnt * sizeof(double)) want <<= 1;
+  PinPool &p = pin_pool();
+  void *ptr = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(p.mu);
+    auto it = p.free.find(want);
+    if (it != p.free.end()) {
+      ptr = it->second;
+      p.free.erase(it);
+      p.kept -= want;
+    }
+  }
+  if (!ptr && hipHostMalloc(&ptr, want, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    return zq_fail(c, ZQ_ERR_OOM, "pinned host buffer");
+  }
+  ctx = c, bytes = want, host = (double *)ptr;
+  ZQ_TRY(c, hipHostGetDevicePointer((void **)&dev, ptr, 0));
+  return ZQ_OK;
+}
+
+ZqStage::~ZqStage() {
+  if (!host) return;
+  if (!idle) (void)hipStreamSynchronize(ctx->stream);
+  PinPool &p = pin_pool();
+  {
+    std::lock_guard<std::mutex> lock(p.mu);
+    if (p.kept + bytes <= kPinKeep && p.users > 0) {
+      p.free.emplace(bytes, host);
+      p.kept += bytes;
+      return;
+    }
+  }
+  (void)hipHostFree(host);
+}
+
+// Kernels write 1 MB chunks over the link into a ring of four (19 us each) while the host copies earlier ones
+// on.  One core reads freshly written memory at 28 GB/s, half the link's rate, so up to four threads each copy
+// a slice of every chunk.  22.5 MB: 1.30 ms as one runtime copy into touched pages, 0.92 ms with one copying
+// thread, 0.57 ms with four.
+int zq_read_back(zq_ctx *ctx, const double *src, double *out, size_t cnt) {
+  constexpr size_t kChunk = size_t(1) << 17, kRing = 4, kMaxCopiers = 4;
+  const size_t chunk = std::min(cnt, kChunk), chunks = cnt ? (cnt + chunk - 1) / chunk : 0, ring = std::min(chunks, kRing);
+  ZqStage st;
+  if (chunks)
+    if (int rc = st.take(ctx, ring * chunk)) return rc;
+  if (chunks <= 1) {
+    if (chunks) {
+      hipLaunchKernelGGL(k_push, dim3(unsigned(std::min<size_t>(256, (cnt + 255) / 256))), dim3(256), 0, ctx->stream, src, cnt,
+                         st.dev);
+      ZQ_LAUNCH_CHECK(ctx, "zq_read_back");
+    }
+    ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    st.done();
+    if (chunks) std::memcpy(out, st.host, cnt * sizeof(double));
+    return ZQ_OK;
+  }
+  for (hipEvent_t &e : ctx->copy_events)
+    if (!e) ZQ_TRY(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  // copier t takes slice t of every chunk; ready chunks are published in order, copied[t] counts its slices
+  std::atomic<size_t> ready{0};
+  std::atomic<size_t> copied[kMaxCopiers];
+  size_t copiers = std::min<size_t>(kMaxCopiers, std::max(1u, std::thread::hardware_concurrency() / 2));
+  for (auto &c : copied) c.store(0);
+  constexpr size_t kAbort = ~size_t(0);
+  std::vector<std::thread> th;
+  auto slice = [&](size_t c, size_t t, size_t of) {
+    const size_t len = std::min(chunk, cnt - c * chunk), a = len * t / of, b = len * (t + 1) / of;
+    std::memcpy(out + c * chunk + a, st.host + (c % ring) * chunk + a, (b - a) * sizeof(double));
+    copied[t].store(c + 1, std::memory_order_release);
+  };
+  // the slices depend on the number of copiers, which is known once their threads have been made
+  std::atomic<size_t> of{0};
+  for (size_t t = 1; t < copiers; ++t) try {
+      th.emplace_back([&, t] {
+        while (!of.load(std::memory_order_acquire)) std::this_thread::yield();
+        for (size_t c = 0; c < chunks; ++c) {
+          size_t r;
+          for (unsigned spins = 0; (r = ready.load(std::memory_order_acquire)) <= c;)
+            if (++spins > 4000) std::this_thread::yield();
+          if (r == kAbort) return;
+          slice(c, t, of.load());
+        }
+      });
+    } catch (...) {
+      break;  // fewer threads
+    }
+  copiers = th.size() + 1;
+  of.store(copiers, std::memory_order_release);
+  auto stop = [&](int rc) {
+    if (rc) ready.store(kAbort, std::memory_order_release);
+    for (auto &x : th) x.join();
+    return rc;
+  };
+  size_t launched = 0;
+  for (size_t c = 0; c < chunks; ++c) {
+    for (;;) {  // refill the ring: a buffer is free once every copier has left it
+      size_t left = chunks;
+      for (size_t t = 0; t < copiers; ++t) left = std::min(left, copied[t].load(std::memory_order_acquire));
+      for (; launched < chunks && launched < left + ring; ++launched) {
+        const size_t len = std::min(chunk, cnt - launched * chunk);
+        hipLaunchKernelGGL(k_push, dim3(unsigned(std::min<size_t>(256, (len + 255) / 256))), dim3(256), 0, ctx->stream,
+                           src + launched * chunk, len, st.dev + (launched % ring) * chunk);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipEventRecord(ctx->copy_events[launched % ring], ctx->stream);
+        if (e != hipSuccess) return stop(zq_check(ctx, e, "zq_read_back"));
+      }
+      if (launched > c) break;
+      std::this_thread::yield();
+    }
+    if (hipError_t e = hipEventSynchronize(ctx->copy_events[c % ring])) return stop(zq_check(ctx, e, "zq_read_back"));
+    ready.store(c + 1, std::memory_order_release);
+    slice(c, 0, copiers);
+  }
+  stop(ZQ_OK);
+  ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  st.done();
+  return ZQ_OK;
 }
 
 void zq_prof_begin(zq_ctx *ctx, const char *name) {
@@ -219,6 +372,7 @@ zq_ctx *zq_create(int device) {
     delete ctx;
     return nullptr;
   }
+  zq_stage_pool_users(1);
   return ctx;
 }
 
@@ -238,6 +392,7 @@ void zq_destroy(zq_ctx *ctx) {
     if (kv.second.ptr) (void)hipHostFree(kv.second.ptr);
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
+  zq_stage_pool_users(-1);
 }
 
 const char *zq_last_error(const zq_ctx *ctx) { return ctx ? ctx->err.c_str() : "null context"; }

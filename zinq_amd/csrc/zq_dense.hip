@@ -502,7 +502,7 @@ int sp2_bufs(zq_ctx *ctx, int n, Sp2Bufs &b) {
   b.part = (double2 *)zq_scratch(ctx, "sp2_part", size_t(kSp2MaxSteps + 1) * b.ntiles * sizeof(double2));
   b.scal = (double *)zq_scratch(ctx, "sp2_scal", 2 * sizeof(double));
   b.sync = (unsigned *)zq_scratch(ctx, "sp2_sync", 2 * kSp2MaxSteps * sizeof(unsigned));
-  b.est = (double *)zq_scratch(ctx, "sp2_est", kEstSize * sizeof(double));
+  b.est = zq_sp2_est(ctx);
   b.ref = (double *)zq_scratch(ctx, "sp2_ref", 2 * size_t(n) * n * sizeof(double));
   b.gpart = (double *)zq_scratch(ctx, "sp2_gpart", 4 * kGershBlocks * sizeof(double));
   bool fresh = false;  // the Gershgorin arrival count starts at zero and its last workgroup clears it again
@@ -563,15 +563,7 @@ int zq_sp2_enqueue(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, i
   return ZQ_OK;
 }
 
-int zq_sp2_tracked_stats(zq_ctx *ctx, int out[3]) {
-  auto *est = (const double *)zq_scratch(ctx, "sp2_est", kEstSize * sizeof(double));
-  if (!est) return zq_fail(ctx, ZQ_ERR_OOM, "SP2 buffers");
-  double h[3] = {0.0, 0.0, 0.0};
-  ZQ_TRY(ctx, hipMemcpyAsync(h, est + kEstRuns, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-  ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  for (int k = 0; k < 3; ++k) out[k] = int(h[k]);
-  return ZQ_OK;
-}
+double *zq_sp2_est(zq_ctx *ctx) { return (double *)zq_scratch(ctx, "sp2_est", kEstSize * sizeof(double)); }
 
 int zq_sp2_density(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, int max_steps, int *steps_hint,
                    const double **dD, int *ld, int *steps) {

@@ -23,6 +23,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <algorithm>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -378,6 +379,20 @@ int zq_syev_rows(zq_ctx *ctx, double *A, int n, double *w, double *offd, int *in
   return zq_gemm_nt(ctx, Z, n, Qm, n, A, n, n, n, n, 1.0, "scf_eig");
 }
 
+namespace {
+// out[i n + k] = V[k n + i] (16 x 16 tiles through LDS), then w (n) and info, into pinned memory.
+__global__ __launch_bounds__(256) void k_eigh_out(const double *__restrict__ V, const double *__restrict__ w,
+                                                  const int *__restrict__ info, int n, double *__restrict__ out) {
+  __shared__ double t[16][17];
+  const int x = threadIdx.x & 15, y = threadIdx.x >> 4, i0 = blockIdx.y * 16, k0 = blockIdx.x * 16;
+  if (k0 + y < n && i0 + x < n) t[y][x] = V[size_t(k0 + y) * n + i0 + x];
+  __syncthreads();
+  if (i0 + y < n && k0 + x < n) out[size_t(i0 + y) * n + k0 + x] = t[x][y];
+  if (blockIdx.y == 0 && threadIdx.x < 16 && k0 + x < n) out[size_t(n) * n + k0 + x] = w[k0 + x];
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) out[size_t(n) * n + n] = *info;
+}
+}  // namespace
+
 extern "C" int zq_eigh(zq_ctx *ctx, size_t n, const double *A, double *W, double *U) {
   ZqGate _gate;
   if (!ctx || !A || !W || !U || n < 1) return zq_fail(ctx, ZQ_ERR_INVALID, "zq_eigh: null argument or n = 0");
@@ -388,6 +403,23 @@ extern "C" int zq_eigh(zq_ctx *ctx, size_t n, const double *A, double *W, double
   auto *dw = (double *)zq_scratch(ctx, "eigh_w", 2 * n * sizeof(double));
   auto *dinfo = (int *)zq_scratch(ctx, "eigh_info", sizeof(int));
   if (!dA || !dw || !dinfo) return zq_fail(ctx, ZQ_ERR_OOM, "zq_eigh buffers");
+  if (nn <= kZqStageMax) {
+    // A through pinned memory; U (the transpose of the eigenvector rows), W and info back in it
+    ZqStage st;
+    if (int rc = st.take(ctx, nn + n + 1)) return rc;
+    std::memcpy(st.host, A, nn * sizeof(double));
+    zq_pad(ctx, st.dev, 1, int(n), int(n), dA);
+    if (int rc = zq_syev_rows(ctx, dA, int(n), dw, dw + n, dinfo)) return rc;
+    hipLaunchKernelGGL(k_eigh_out, dim3(unsigned((n + 15) / 16), unsigned((n + 15) / 16)), dim3(256), 0, ctx->stream, dA,
+                       dw, dinfo, int(n), st.dev);
+    ZQ_LAUNCH_CHECK(ctx, "k_eigh_out");
+    ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    st.done();
+    if (st.host[nn + n] != 0.0) return zq_fail(ctx, ZQ_ERR_LAPACK, "zq_eigh: tridiagonal eigensolver did not converge");
+    std::memcpy(U, st.host, nn * sizeof(double));
+    std::memcpy(W, st.host + nn, n * sizeof(double));
+    return ZQ_OK;
+  }
   ZQ_TRY(ctx, hipMemcpyAsync(dA, A, nn * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
   if (int rc = zq_syev_rows(ctx, dA, int(n), dw, dw + n, dinfo)) return rc;
   std::vector<double> V(nn);

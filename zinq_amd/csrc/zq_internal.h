@@ -136,7 +136,7 @@ struct zq_ctx {
   int scf_replays = 0;   // iterations the asynchronous driver enqueued in the last device SCF
   int scf_driver = 0;    // driver that finished the last device SCF: 1 device-decided, 2 host-synchronised
   int scf_sp2[3] = {0, 0, 0};  // its SP2 densities, folded ones, steps (device-decided driver only)
-  hipEvent_t scf_events[2] = {nullptr, nullptr};  // the asynchronous SCF's lagged state reads
+  hipEvent_t copy_events[4] = {nullptr, nullptr, nullptr, nullptr};  // zq_read_back's buffers
 
   // named scratch buffers (grow-only)
   std::map<std::string, DevBuf> scratch;
@@ -191,6 +191,36 @@ int zq_check(zq_ctx *ctx, hipError_t e, const char *what);
 // captured, pass false).
 void *zq_scratch(zq_ctx *ctx, const std::string &name, size_t bytes, bool *fresh = nullptr, bool captured = true);
 void *zq_pinned(zq_ctx *ctx, const std::string &name, size_t bytes);
+// Host arrays at the boundary.  A caller's arrays are pageable: a copy of one goes through the runtime's
+// staging and costs 20 us at 5 KB, 125 us at 300 KB, and 2-D copies one of these per few rows.  So they
+// are copied to or from pinned buffers here, which kernels read and write in place over the link (55 GB/s).
+//
+// ZqStage: a pinned buffer for the length of one call, and its device address.  The buffers come from a pool of
+// the process, because the host's first touch of pinned pages costs 0.4 ms per MB: a new context takes pages
+// that an earlier call has touched.  The pool keeps at most 64 MB and is emptied with the last context.  A
+// buffer goes back when its holder has waited for the stream (done()); without that (an error return) the
+// destructor waits first, so no kernel can still be reading or writing a buffer that another thread takes.
+struct ZqStage {
+  double *host = nullptr, *dev = nullptr;
+  ZqStage() = default;
+  ~ZqStage();
+  ZqStage(const ZqStage &) = delete;
+  ZqStage &operator=(const ZqStage &) = delete;
+  int take(zq_ctx *ctx, size_t cnt);  // cnt doubles; ZQ_OK or ZQ_ERR_OOM
+  void done() { idle = true; }        // the stream has been waited for
+
+ private:
+  zq_ctx *ctx = nullptr;
+  size_t bytes = 0;
+  bool idle = false;
+};
+void zq_stage_pool_users(int change);  // contexts alive: +1 / -1
+// Largest array (doubles) that is staged whole: 8 MB.  Larger ones take the runtime's copies.
+constexpr size_t kZqStageMax = size_t(1) << 20;
+// cnt doubles from the device into the caller's array, in order on ctx's stream, which is idle on return.
+int zq_read_back(zq_ctx *ctx, const double *src, double *out, size_t cnt);
+// nd matrices n x n (contiguous, device or pinned) into np x np slots, zero padded (zq_jk.hip).
+void zq_pad(zq_ctx *ctx, const double *src, size_t nd, int n, int np, double *dst);
 void zq_free_eri(zq_ctx *ctx);
 void zq_prof_begin(zq_ctx *ctx, const char *name);
 void zq_prof_end(zq_ctx *ctx);
@@ -219,7 +249,8 @@ int zq_mp2_grouped(hipStream_t stream, const std::vector<ZqGroupMol> &mols, int 
                    double *e_corr, std::string &err);
 // Q1..Q4 of the resident ERIs into context scratch (zq_transform.hip): *d_out = out[i][j][a][b] with dims
 // m1 x m2 x m3 x m4 (FULL: n^4, <pq|rs>; OVOV: o o v v), double or (*is_f32) float.
-int zq_transform_device(zq_ctx *ctx, const double *C, int nocc, int block, int precision, void **d_out, int dims[4],
+// st: the caller's stage for C, held until it has waited for the stream.
+int zq_transform_device(zq_ctx *ctx, ZqStage &st, const double *C, int nocc, int block, int precision, void **d_out, int dims[4],
                         bool *is_f32);
 // Devices whose static no-allocation scratch address is kept (zq_transform.hip).
 constexpr int kZqMaxDevices = 64;
@@ -261,8 +292,8 @@ constexpr int kSp2MaxSteps = 128;
 int zq_syev_rows(zq_ctx *ctx, double *A, int n, double *w, double *offd, int *info);  // zq_eigen.hip
 int zq_sp2_enqueue(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, int nsteps, const int *skip, int *state6,
                    const double **dX, long long *stride, int *ld, int track);  // zq_dense.hip
-// {densities, folded densities, SP2 steps} of the tracked runs since the last track = 1 run (synchronous).
-int zq_sp2_tracked_stats(zq_ctx *ctx, int out[3]);  // zq_dense.hip
+// The fold bookkeeping of the tracked runs (kEstSize doubles); null on failure.
+double *zq_sp2_est(zq_ctx *ctx);  // zq_dense.hip
 
 #define ZQ_TRY(ctx, call)                                \
   do {                                                   \

@@ -210,27 +210,65 @@ int sygv(int n, double *A, double *B, double *w) {
 
 int chol_inv_t(int n, const double *S, double *X) {
   // S = U^T U with U = L^T upper (row-major), right-looking: row j of U, then the trailing update
-  // A[i][i..] -= U[j][i] U[j][i..], all on contiguous row segments (vectorised axpys)
+  // A[i][i..] -= U[j][i] U[j][i..], all on contiguous row segments (vectorised axpys).  Four rows of U are
+  // formed before the trailing rows take them in one pass, each element still in ascending j, so the values
+  // are those of one row at a time; it loads and stores the trailing block a quarter as often.
   std::vector<double> U(S, S + size_t(n) * n);
-  for (int j = 0; j < n; ++j) {
-    double *Uj = U.data() + size_t(j) * n;
-    if (Uj[j] <= 0.0) return 1;
-    const double d = std::sqrt(Uj[j]), inv = 1.0 / d;
-    Uj[j] = d;
-    for (int k = j + 1; k < n; ++k) Uj[k] *= inv;
-    for (int i = j + 1; i < n; ++i) {
+  for (int j0 = 0; j0 < n; j0 += 4) {
+    const int j1 = j0 + 4 < n ? j0 + 4 : n;
+    for (int j = j0; j < j1; ++j) {
+      double *Uj = U.data() + size_t(j) * n;
+      if (Uj[j] <= 0.0) return 1;
+      const double d = std::sqrt(Uj[j]), inv = 1.0 / d;
+      Uj[j] = d;
+      for (int k = j + 1; k < n; ++k) Uj[k] *= inv;
+      for (int i = j + 1; i < j1; ++i) {
+        double *__restrict__ Ai = U.data() + size_t(i) * n;
+        const double *__restrict__ uj = Uj;
+        const double f = uj[i];
+        for (int k = i; k < n; ++k) Ai[k] -= f * uj[k];
+      }
+    }
+    if (j1 - j0 < 4) break;  // the last rows: nothing trails them
+    const double *__restrict__ u0 = U.data() + size_t(j0) * n, *__restrict__ u1 = u0 + n, *__restrict__ u2 = u1 + n,
+                             *__restrict__ u3 = u2 + n;
+    for (int i = j1; i < n; ++i) {
       double *__restrict__ Ai = U.data() + size_t(i) * n;
-      const double *__restrict__ uj = Uj;
-      const double f = uj[i];
-      for (int k = i; k < n; ++k) Ai[k] -= f * uj[k];
+      const double f0 = u0[i], f1 = u1[i], f2 = u2[i], f3 = u3[i];
+      for (int k = i; k < n; ++k) {
+        double a = Ai[k];
+        a -= f0 * u0[k];
+        a -= f1 * u1[k];
+        a -= f2 * u2[k];
+        a -= f3 * u3[k];
+        Ai[k] = a;
+      }
     }
   }
-  // X = L^-T = U^-1 (upper), by rows from the bottom: X[i][i..] = (e_i - sum_{k>i} U[i][k] X[k][i..]) / U[i][i]
+  // X = L^-T = U^-1 (upper), by rows from the bottom: X[i][i..] = (e_i - sum_{k>i} U[i][k] X[k][i..]) / U[i][i], the
+  // rows k taken four at a time from the column where all four have begun, again in ascending k
   for (int i = n - 1; i >= 0; --i) {
     double *__restrict__ Xi = X + size_t(i) * n;
     const double *Ui = U.data() + size_t(i) * n;
     for (int c = 0; c < n; ++c) Xi[c] = c == i ? 1.0 : 0.0;
-    for (int k = i + 1; k < n; ++k) {
+    int k = i + 1;
+    for (; k + 4 <= n; k += 4) {
+      const double f0 = Ui[k], f1 = Ui[k + 1], f2 = Ui[k + 2], f3 = Ui[k + 3];
+      const double *__restrict__ x0 = X + size_t(k) * n, *__restrict__ x1 = x0 + n, *__restrict__ x2 = x1 + n,
+                               *__restrict__ x3 = x2 + n;
+      Xi[k] -= f0 * x0[k];
+      Xi[k + 1] -= f0 * x0[k + 1], Xi[k + 1] -= f1 * x1[k + 1];
+      Xi[k + 2] -= f0 * x0[k + 2], Xi[k + 2] -= f1 * x1[k + 2], Xi[k + 2] -= f2 * x2[k + 2];
+      for (int c = k + 3; c < n; ++c) {
+        double a = Xi[c];
+        a -= f0 * x0[c];
+        a -= f1 * x1[c];
+        a -= f2 * x2[c];
+        a -= f3 * x3[c];
+        Xi[c] = a;
+      }
+    }
+    for (; k < n; ++k) {
       const double f = Ui[k];
       const double *__restrict__ Xk = X + size_t(k) * n;
       for (int c = k; c < n; ++c) Xi[c] -= f * Xk[c];

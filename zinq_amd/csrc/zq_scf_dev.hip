@@ -30,6 +30,7 @@
 #include <cstring>
 #include <deque>
 #include <memory>
+#include <thread>
 #include <vector>
 
 #include "../../include/zinq_scf.h"
@@ -171,6 +172,7 @@ struct Dev {
   double *dP = nullptr;     // P_k - P_(k-1), npad x npad zero padded (mixed Fock path only)
   double *epart = nullptr;  // energy partials of the J/K reduce, one per output block
   int *slots, *info;
+  ZqStage in;               // S, X and H on their way to the device
   int sp2_hint = 24;  // SP2 steps of the previous density, the first convergence check comes after it
   int sp2_steps = 0, sp2_calls = 0, sp2_fallbacks = 0;
 };
@@ -402,14 +404,14 @@ __global__ void k_sp2_check(int parity, ScfState *__restrict__ st) {
 }
 
 // The end of an iteration: the SP2 check of k_sp2_check (parity of its step budget), then rms(dP) and
-// the convergence test of src/hartree_fock.zig:853-870 (one wave, butterfly sum).  The state's done
-// word also goes to *host_done (host memory the device writes), which the host reads one iteration late.
+// the convergence test of src/hartree_fock.zig:853-870 (one wave, butterfly sum), and the report to the host,
+// which reads it one iteration late.
 __global__ __launch_bounds__(64) void k_converge(const double *__restrict__ part, int n, double thr, int maxit,
-                                                 ScfState *__restrict__ st, int parity, int *__restrict__ host_done,
+                                                 ScfState *st, int parity, const double *est, ScfProgress *progress,
                                                  int diis) {
   if (st->done) {
     // set before this iteration (the guess density's SP2 check): the host stops replaying as well
-    if (threadIdx.x == 0) *host_done = st->done;
+    if (threadIdx.x == 0) report(st, est, progress);
     return;
   }
   const double s = zqt::wave_sum(part[threadIdx.x]);
@@ -419,22 +421,21 @@ __global__ __launch_bounds__(64) void k_converge(const double *__restrict__ part
   st->sp2_max = max(st->sp2_max, fin[1]);
   if (fin[0] < 2 || st->sp2[5] != 0) {  // SP2 did not settle: the P of this iteration is not used
     st->done = 3;
-    *host_done = 3;
-    return;
+  } else {
+    const double rms = sqrt(s / (double(n) * n));
+    const double dE = fabs(st->e_new - st->e_old);
+    st->e_old = st->e_new;
+    st->rms = rms, st->dE = dE;
+    const bool conv = st->it > 0 && dE < thr && rms < thr;
+    ++st->it;
+    if (conv)
+      st->done = 1;
+    else if (st->it >= maxit)
+      st->done = 2;
+    else if (diis > 0)
+      diis_next_slot(st, diis);
   }
-  const double rms = sqrt(s / (double(n) * n));
-  const double dE = fabs(st->e_new - st->e_old);
-  st->e_old = st->e_new;
-  st->rms = rms, st->dE = dE;
-  const bool conv = st->it > 0 && dE < thr && rms < thr;
-  ++st->it;
-  if (conv)
-    st->done = 1;
-  else if (st->it >= maxit)
-    st->done = 2;
-  else if (diis > 0)
-    diis_next_slot(st, diis);
-  *host_done = st->done;
+  report(st, est, progress);
 }
 
 // P from the symmetric Fock matrix A by SP2 with a fixed step budget, without host synchronisation.
@@ -470,13 +471,13 @@ bool step_fits(int n) { return n <= 16 * kStepMaxTiles; }
 // registers (its tiles and its share of the matrices).
 constexpr int kStepThreads = 512;
 
-// scf_step of one molecule; an iteration whose state is already done only hands its mark to the host.
+// scf_step of one molecule; an iteration whose state is already done only reports it to the host.
 template <int T>
 __global__ __launch_bounds__(kStepThreads) void k_scf_step(StepArgs a) {
   extern __shared__ __attribute__((aligned(16))) double step_lds[];
   __shared__ StepShared sh;
   if (a.mode == kStepIter && a.st->done) {
-    if (threadIdx.x == 0) *a.done_out = a.st->done;
+    if (threadIdx.x == 0) report(a.st, a.est, a.progress);
     return;
   }
   StepBody<kStepThreads, T>::run(a, step_lds, sh);
@@ -513,21 +514,53 @@ struct Run {
   StepArgs step{};     // its arguments
 };
 
-// Uploads S, X = L^-T, X^T, H; zeroes P.
+// S, X, H from pinned memory to the device, X^T beside X, and a zeroed density.
+__global__ __launch_bounds__(256) void k_scf_in(const double *__restrict__ in, int n, int np, double *__restrict__ S,
+                                                double *__restrict__ X, double *__restrict__ XT, double *__restrict__ H,
+                                                double *__restrict__ P) {
+  const size_t nn = size_t(n) * n, pp = size_t(np) * np;
+  for (size_t x = blockIdx.x * size_t(256) + threadIdx.x; x < pp; x += size_t(gridDim.x) * 256) {
+    P[x] = 0.0;
+    if (x >= nn) continue;
+    const int i = int(x / unsigned(n)), j = int(x - size_t(i) * n);
+    const double s = in[x], v = in[nn + x], h = in[2 * nn + x];
+    S[x] = s, X[x] = v, XT[size_t(j) * n + i] = v, H[x] = h;
+  }
+}
+
+// The results into pinned memory: C, P (without its padding), the diagonalised Fock matrix, e, and *energy (if
+// given).
+__global__ __launch_bounds__(256) void k_scf_out(const double *__restrict__ C, const double *__restrict__ P, int n, int np,
+                                                 const double *__restrict__ W, const double *__restrict__ e,
+                                                 const double *__restrict__ energy, double *__restrict__ out) {
+  const size_t nn = size_t(n) * n;
+  for (size_t x = blockIdx.x * size_t(256) + threadIdx.x; x < nn; x += size_t(gridDim.x) * 256) {
+    const int i = int(x / unsigned(n)), j = int(x - size_t(i) * n);
+    out[x] = C[x], out[nn + x] = P[size_t(i) * np + j], out[2 * nn + x] = W[x];
+    if (x < size_t(n)) out[3 * nn + x] = e[x];
+    if (x == 0 && energy) out[3 * nn + n] = *energy;
+  }
+}
+
+unsigned io_blocks(size_t cnt) { return unsigned(std::min<size_t>(1024, (cnt + 255) / 256)); }
+
+// Uploads S, X = L^-T, X^T, H; zeroes P.  (A second call, of the host-synchronised restart, finds the first one's
+// copies long done: iterations have run behind them.)
 int setup(Dev &d, const double *H, const double *S) {
   zq_ctx *ctx = d.ctx;
   const int n = d.n, np = ctx->npad;
   const size_t nn = d.nn;
-  std::vector<double> hX(nn), hXT(nn);
-  if (zq::chol_inv_t(n, S, hX.data())) return zq_fail(ctx, ZQ_ERR_LAPACK, "overlap matrix not positive definite");
-  for (int i = 0; i < n; ++i)
-    for (int j = 0; j < n; ++j) hXT[size_t(j) * n + i] = hX[size_t(i) * n + j];
-  ZQ_TRY(ctx, hipMemcpyAsync(d.S, S, nn * 8, hipMemcpyHostToDevice, ctx->stream));
-  ZQ_TRY(ctx, hipMemcpyAsync(d.X, hX.data(), nn * 8, hipMemcpyHostToDevice, ctx->stream));
-  ZQ_TRY(ctx, hipMemcpyAsync(d.XT, hXT.data(), nn * 8, hipMemcpyHostToDevice, ctx->stream));
-  ZQ_TRY(ctx, hipMemcpyAsync(ctx->d_H, H, nn * 8, hipMemcpyHostToDevice, ctx->stream));
-  ZQ_TRY(ctx, hipMemsetAsync(ctx->d_P, 0, size_t(np) * np * 8, ctx->stream));
-  ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));  // the host vectors go out of scope
+  if (!d.in.host)
+    if (int rc = d.in.take(ctx, 3 * nn)) return rc;
+  ZqStage &st = d.in;
+  std::vector<double> X(nn);  // built in ordinary memory: its rows are read back many times
+  if (zq::chol_inv_t(n, S, X.data())) return zq_fail(ctx, ZQ_ERR_LAPACK, "overlap matrix not positive definite");
+  std::memcpy(st.host, S, nn * sizeof(double));
+  std::memcpy(st.host + nn, X.data(), nn * sizeof(double));
+  std::memcpy(st.host + 2 * nn, H, nn * sizeof(double));
+  hipLaunchKernelGGL(k_scf_in, dim3(io_blocks(size_t(np) * np)), dim3(256), 0, ctx->stream, st.dev, n, np, d.S, d.X, d.XT,
+                     ctx->d_H, ctx->d_P);
+  ZQ_LAUNCH_CHECK(ctx, "k_scf_in");
   return ZQ_OK;
 }
 
@@ -542,7 +575,7 @@ int step_args(const Dev &d, Run &r, ScfState *st) {
   a.Fh = d.Fh, a.Eh = d.Eh;
   a.epart = d.epart, a.nep = ctx->Nb;
   a.ref = (double *)zq_scratch(ctx, "sp2_ref", 2 * d.nn * sizeof(double));
-  a.est = (double *)zq_scratch(ctx, "sp2_est", kEstSize * sizeof(double));
+  a.est = zq_sp2_est(ctx);
   if (!a.ref || !a.est) return zq_fail(ctx, ZQ_ERR_OOM, "SCF step buffers");
   a.n = r.n, a.nocc = r.nocc, a.diis = r.opt->diis, a.maxit = r.opt->iterations;
   a.factor = r.factor, a.VN = r.VN, a.thr = r.opt->threshold, a.err_scale = ctx->diis_err_scale;
@@ -550,7 +583,7 @@ int step_args(const Dev &d, Run &r, ScfState *st) {
 }
 
 // The kernels of one SCF iteration; every one of them returns at once while state.done != 0.
-int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *part_rms, int *host_done) {
+int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *part_rms, ScfProgress *progress) {
   zq_ctx *ctx = d.ctx;
   const int n = d.n, maxh = r.opt->diis > 0 ? r.opt->diis : 1;
   const size_t nn = d.nn;
@@ -561,7 +594,7 @@ int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *pa
                            : zq_fock_jk_device(ctx, ctx->d_P, ctx->d_H, r.x_exch, ctx->d_F, skip, false, d.epart);
     if (rc) return rc;
     StepArgs a = r.step;
-    a.mode = kStepIter, a.nsteps = budget, a.done_out = host_done;
+    a.mode = kStepIter, a.nsteps = budget, a.progress = progress;
     return launch_step(ctx, a);
   }
   // the reduce also leaves the energy partials (getEnergy) in d.epart; the DIIS slot of this iteration
@@ -583,10 +616,31 @@ int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *pa
   hipLaunchKernelGGL(k_diis_solve, dim3(1), dim3(64), 0, ctx->stream, d.part, d.epart, ctx->Nb, r.opt->diis, r.VN, st);
   hipLaunchKernelGGL(k_combine_state, dim3(gblocks), dim3(256), 0, ctx->stream, d.Fh, ctx->d_F, n, d.W, st);
   if (int rc = density_async(d, d.W, r.nocc, r.factor, budget, st, part_rms, r.mixed ? d.dP : nullptr, false)) return rc;
+  const double *est = zq_sp2_est(ctx);
+  if (!est) return zq_fail(ctx, ZQ_ERR_OOM, "SP2 buffers");
   hipLaunchKernelGGL(k_converge, dim3(1), dim3(64), 0, ctx->stream, part_rms, n, r.opt->threshold, r.opt->iterations, st,
-                     budget & 1, host_done, r.opt->diis);
+                     budget & 1, est, progress, r.opt->diis);
   ZQ_LAUNCH_CHECK(ctx, "scf iteration");
   return ZQ_OK;
+}
+
+// Waits until the device has reported its-th iterations or a set done mark, on the pinned word itself: an event
+// per iteration costs the stream about 5 us between iterations.  A stream that has gone idle without the
+// report (a failed launch) ends the wait.
+int wait_progress(zq_ctx *ctx, const ScfProgress *p, unsigned its, unsigned long long &word) {
+  auto reported = [&] {
+    word = __atomic_load_n(&p->word, __ATOMIC_ACQUIRE);
+    return (word >> 32) != 0 || unsigned(word) >= its;
+  };
+  for (unsigned spins = 1;; ++spins) {
+    if (reported()) return ZQ_OK;
+    if (spins > 2000) std::this_thread::yield();
+    if (spins % (1u << 20) == 0) {
+      const hipError_t e = hipStreamQuery(ctx->stream);
+      if (e != hipSuccess && e != hipErrorNotReady) return zq_check(ctx, e, "device SCF");
+      if (e == hipSuccess && !reported()) return zq_fail(ctx, ZQ_ERR_LAUNCH, "device SCF: the stream ended without a report");
+    }
+  }
 }
 
 // The asynchronous SCF.  Returns ZQ_OK with *status = state.done (1 converged, 2 iteration limit,
@@ -598,17 +652,13 @@ int scf_async(Dev &d, Run &r, int *status, double *energy, int *iterations) {
   const size_t nn = d.nn;
   std::unique_ptr<ZqGate> gate(new ZqGate);  // set-up allocates; released before the replay loop
   auto *st = (ScfState *)zq_scratch(ctx, "scf_state", sizeof(ScfState));
-  auto *hdone = (int *)zq_pinned(ctx, "scf_done", sizeof(int));
-  if (!st || !hdone || !zq_pinned(ctx, "scf_state_full", sizeof(ScfState))) return zq_fail(ctx, ZQ_ERR_OOM, "SCF state");
-  int *ddone = nullptr;  // the same host word as the kernels address it
-  ZQ_TRY(ctx, hipHostGetDevicePointer((void **)&ddone, hdone, 0));
+  auto *hprog = (ScfProgress *)zq_pinned(ctx, "scf_progress", sizeof(ScfProgress));
+  if (!st || !hprog) return zq_fail(ctx, ZQ_ERR_OOM, "SCF state");
+  ScfProgress *dprog = nullptr;  // the same host memory as the kernels address it
+  ZQ_TRY(ctx, hipHostGetDevicePointer((void **)&dprog, hprog, 0));
   double *part_rms = d.part + (1 + kMaxHist) * kRedBlocks;
   d.epart = (double *)zq_scratch(ctx, "scf_epart", size_t(ctx->Nb) * sizeof(double));
   if (!d.epart) return zq_fail(ctx, ZQ_ERR_OOM, "SCF energy partials");
-  hipEvent_t *ev = ctx->scf_events;
-  if (!ev[0]) ZQ_TRY(ctx, hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
-  if (!ev[1]) ZQ_TRY(ctx, hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
-
   if (r.mixed) {
     if (int rc = zq_eri32(ctx)) return rc;
     d.dP = (double *)zq_scratch(ctx, "scf_dP", size_t(r.np) * r.np * sizeof(double));
@@ -638,7 +688,7 @@ int scf_async(Dev &d, Run &r, int *status, double *energy, int *iterations) {
   char key[256];
   snprintf(key, sizeof key, "%d/%d/%d/%d/%d/%a/%a/%a/%a/%a/%c%llu/%p/%p/%d", n, nocc, budget, r.opt->diis,
            r.opt->iterations, r.x_exch, r.factor, r.VN, r.opt->threshold, ctx->diis_err_scale, ctx->set_id ? 's' : 'g',
-           ctx->set_id ? ctx->set_id : (unsigned long long)ctx->eri_gen, (void *)st, (void *)ddone, int(r.mixed));
+           ctx->set_id ? ctx->set_id : (unsigned long long)ctx->eri_gen, (void *)st, (void *)dprog, int(r.mixed));
   if (ctx->scf_graphs_gen != ctx->scratch_gen || ctx->scf_graphs.size() >= 64) {
     drop_graphs(ctx);
     ctx->scf_graphs_gen = ctx->scratch_gen;
@@ -648,7 +698,7 @@ int scf_async(Dev &d, Run &r, int *status, double *energy, int *iterations) {
   if (use_graph && !graph_exec) {
     ZqCaptureWindow window;  // no allocation or synchronous call in any thread while capturing
     ZQ_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    const int rc = enqueue_iteration(d, r, budget, st, part_rms, ddone);
+    const int rc = enqueue_iteration(d, r, budget, st, part_rms, dprog);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(ctx->stream, &graph);
     if (rc) {
@@ -664,34 +714,40 @@ int scf_async(Dev &d, Run &r, int *status, double *energy, int *iterations) {
     ++ctx->scf_captures;
     graph_exec = exec;
   }
-  // the stream is idle here (the previous run ended with a synchronisation), so no kernel writes it now
-  *(volatile int *)hdone = 0;
+  // the stream holds only the guess density, which does not write the progress word
+  __atomic_store_n(&hprog->word, 0ULL, __ATOMIC_RELEASE);
   ctx->scf_replays = 0;
-  int k = 0;
-  for (; k < r.opt->iterations; ++k) {
+  unsigned long long word = 0;
+  for (int k = 0; k < r.opt->iterations; ++k) {
     ++ctx->scf_replays;
     if (use_graph) {
       ZQ_TRY(ctx, hipGraphLaunch(graph_exec, ctx->stream));
-    } else if (int rc = enqueue_iteration(d, r, budget, st, part_rms, ddone)) {
+    } else if (int rc = enqueue_iteration(d, r, budget, st, part_rms, dprog)) {
       return rc;
     }
-    ZQ_TRY(ctx, hipEventRecord(ev[k & 1], ctx->stream));
+    // done after iteration k-1 (or a later one: done never goes back to 0); iteration k is already queued
+    // behind it
     if (k >= 1) {
-      // done after iteration k-1 (or a later one: done never goes back to 0); iteration k is already
-      // queued behind it
-      ZQ_TRY(ctx, hipEventSynchronize(ev[(k - 1) & 1]));
-      if (*(volatile int *)hdone != 0) break;
+      if (int rc = wait_progress(ctx, hprog, unsigned(k), word)) return rc;
+      if (word >> 32) break;
     }
   }
-  auto *hs_p = (ScfState *)zq_pinned(ctx, "scf_state_full", sizeof(ScfState));
-  if (!hs_p) return zq_fail(ctx, ZQ_ERR_OOM, "SCF state");
-  ZQ_TRY(ctx, hipMemcpyAsync(hs_p, st, sizeof(ScfState), hipMemcpyDeviceToHost, ctx->stream));
-  ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  const ScfState hs = *hs_p;
-  *status = hs.done == 0 ? 2 : hs.done;
-  *energy = hs.e_new;
-  *iterations = hs.it;
-  ctx->scf_diis_resets = hs.resets;
+  if (r.opt->iterations < 1) {  // no iteration, no report: the guess density's state
+    ScfState hs;
+    ZQ_TRY(ctx, hipMemcpyAsync(&hs, st, sizeof(ScfState), hipMemcpyDeviceToHost, ctx->stream));
+    ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    *status = hs.done == 0 ? 2 : hs.done;
+    *energy = hs.e_new, *iterations = hs.it;
+    return ZQ_OK;
+  }
+  // a run that used its last iteration has not seen that one's report yet
+  if (!(word >> 32))
+    if (int rc = wait_progress(ctx, hprog, unsigned(r.opt->iterations), word)) return rc;
+  *status = int(word >> 32);
+  *energy = hprog->energy;
+  *iterations = hprog->it;
+  ctx->scf_diis_resets = hprog->resets;
+  for (int x = 0; x < 3; ++x) ctx->scf_sp2[x] = *status == 3 ? 0 : hprog->sp2[x];
   return ZQ_OK;
 }
 
@@ -797,7 +853,7 @@ void zq_release_solver(zq_ctx *ctx) {
     ctx->solver = nullptr;
   }
   drop_graphs(ctx);
-  for (hipEvent_t &e : ctx->scf_events)
+  for (hipEvent_t &e : ctx->copy_events)
     if (e) (void)hipEventDestroy(e), e = nullptr;
   for (hipEvent_t &e : ctx->eig_events)
     if (e) (void)hipEventDestroy(e), e = nullptr;
@@ -831,6 +887,8 @@ extern "C" int zq_scf_run_device(zq_ctx *ctx, size_t n_, size_t nocc_, const dou
   if (int rc = setup(d, H, S)) return rc;
   ctx->scf_replays = 0;
   ctx->scf_diis_resets = 0;
+  ctx->scf_sp2[0] = ctx->scf_sp2[1] = ctx->scf_sp2[2] = 0;
+  const double *d_energy = nullptr;  // an energy still on the device
   if (opt->diis <= kMaxHist) {
     gate.reset();
     const int rc = scf_async(d, r, &status, &energy, &iterations);
@@ -839,9 +897,6 @@ extern "C" int zq_scf_run_device(zq_ctx *ctx, size_t n_, size_t nocc_, const dou
   }
   if (status == 3) ctx->sp2_budget = std::min(kSp2MaxSteps, ctx->sp2_budget + 16);
   ctx->scf_driver = (status == 0 || status == 3) ? 2 : 1;
-  ctx->scf_sp2[0] = ctx->scf_sp2[1] = ctx->scf_sp2[2] = 0;
-  if (ctx->scf_driver == 1)
-    if (int rc = zq_sp2_tracked_stats(ctx, ctx->scf_sp2)) return rc;
   if (status == 0 || status == 3) {
     // DIIS history beyond the device bookkeeping, or an SP2 budget too small: synchronised driver
     // (FP64 Fock builds throughout)
@@ -854,9 +909,7 @@ extern "C" int zq_scf_run_device(zq_ctx *ctx, size_t n_, size_t nocc_, const dou
     hipLaunchKernelGGL(k_energy_part, dim3(kRedBlocks), dim3(256), 0, ctx->stream, ctx->d_P, np, ctx->d_H, ctx->d_F, n,
                        d.part, nullptr);
     hipLaunchKernelGGL(k_finish, dim3(1), dim3(64), 0, ctx->stream, d.part, 1, d.scal);
-    double h = 0.0;
-    if (int rc = sync_read(ctx, d.scal, &h, 1)) return rc;
-    energy = h + VN;
+    d_energy = d.scal;
     ++iterations;
     ZQ_TRY(ctx, hipMemcpyAsync(d.W, ctx->d_F, nn * 8, hipMemcpyDeviceToDevice, ctx->stream));
   }
@@ -865,13 +918,19 @@ extern "C" int zq_scf_run_device(zq_ctx *ctx, size_t n_, size_t nocc_, const dou
   if (int rc = to_orthonormal(d, d.W)) return rc;
   if (int rc = diag_orthonormal(d, d.C)) return rc;
   hipLaunchKernelGGL(k_density, dim3(kRedBlocks), dim3(256), 0, ctx->stream, d.C, n, nocc, r.factor, ctx->d_P, np, d.part);
-  std::vector<double> hP(size_t(np) * np);
-  ZQ_TRY(ctx, hipMemcpyAsync(C, d.C, nn * 8, hipMemcpyDeviceToHost, ctx->stream));
-  ZQ_TRY(ctx, hipMemcpyAsync(e, d.eig, size_t(n) * 8, hipMemcpyDeviceToHost, ctx->stream));
-  ZQ_TRY(ctx, hipMemcpyAsync(hP.data(), ctx->d_P, hP.size() * 8, hipMemcpyDeviceToHost, ctx->stream));
-  ZQ_TRY(ctx, hipMemcpyAsync(F, d.W, nn * 8, hipMemcpyDeviceToHost, ctx->stream));
+  ZqStage out;
+  if (int rc = out.take(ctx, 3 * nn + n + 1)) return rc;
+  hipLaunchKernelGGL(k_scf_out, dim3(io_blocks(nn)), dim3(256), 0, ctx->stream, d.C, ctx->d_P, n, np, d.W, d.eig, d_energy,
+                     out.dev);
+  ZQ_LAUNCH_CHECK(ctx, "k_scf_out");
   ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  for (int i = 0; i < n; ++i) std::memcpy(P + size_t(i) * n, hP.data() + size_t(i) * np, n * sizeof(double));
+  out.done();
+  d.in.done();
+  std::memcpy(C, out.host, nn * sizeof(double));
+  std::memcpy(P, out.host + nn, nn * sizeof(double));
+  std::memcpy(F, out.host + 2 * nn, nn * sizeof(double));
+  std::memcpy(e, out.host + 3 * nn, size_t(n) * sizeof(double));
+  if (d_energy) energy = out.host[3 * nn + n] + VN;
   res->energy = energy;
   res->iterations = iterations;
   if (status != 1) return zq_fail(ctx, ZQ_ERR_NOT_CONVERGED, "SCF did not converge");

@@ -173,6 +173,25 @@ struct ScfState {
   double B[kMaxHist * kMaxHist];  // B[slot][slot] = <err_slot, err_slot'>
 };
 
+// The host's view of a device SCF, in pinned memory: word holds done << 32 | iterations completed and is
+// written last, once per iteration; the rest is valid once done is set.
+struct ScfProgress {
+  unsigned long long word;
+  double energy;
+  int it, resets;
+  int sp2[3];  // densities, folded ones, SP2 steps
+};
+
+// One thread, at the end of an iteration (or of one that found done already set).
+__device__ inline void report(const ScfState *st, const double *est, ScfProgress *p) {
+  if (st->done) {
+    p->energy = st->e_new, p->it = st->it, p->resets = st->resets;
+    for (int k = 0; k < 3; ++k) p->sp2[k] = int(est[kEstRuns + k]);
+  }
+  __hip_atomic_store(&p->word, (unsigned long long)(st->done) << 32 | unsigned(st->it), __ATOMIC_RELEASE,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Slot of the next iteration's error/Fock pair: the oldest when the history is full, else the lowest
 // free.  Taken at the end of the previous iteration (k_converge) or by k_state_init for the first.
 __device__ inline void diis_next_slot(ScfState *st, int diis) {
@@ -372,6 +391,7 @@ struct StepArgs {
   double *est;          // fold bookkeeping
   const double *epart;  // energy partials of the J/K reduce; null: the energy is summed here
   int *done_out;        // receives st->done at the end (may be null)
+  ScfProgress *progress;  // the host's view of the run (may be null)
   int nep, ldh, ldp, ldm, n, nocc, diis, maxit, nsteps, mode;
   double factor, VN, thr, err_scale;
 };
@@ -865,6 +885,7 @@ struct StepBody {
       if (!settled) {  // no gap at the Fermi level within the budget: this density is not used
         st->done = 3;
         if (a.done_out) *a.done_out = 3;
+        if (a.progress) report(st, a.est, a.progress);
       }
     }
     if (!settled) return;
@@ -916,6 +937,7 @@ struct StepBody {
         diis_next_slot(st, a.diis);
     }
     if (a.done_out) *a.done_out = st->done;
+    if (a.progress) report(st, a.est, a.progress);
   }
 };
 

@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <type_traits>
 
@@ -952,6 +953,12 @@ __global__ void zq_c_slices(const double *__restrict__ C, int n, int np, int m1,
   c_slices_body<T>(C, n, np, m1, m2, m3, off3, c1, c2t, c3, blockIdx.x);  // one workgroup per row mu < np
 }
 
+// y = x (n doubles; x may be pinned host memory)
+__global__ void zq_take(const double *__restrict__ x, int n, double *__restrict__ y) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) y[i] = x[i];
+}
+
 // BF16X3 Q1 operand: C1 split into bf16 hi + lo and transposed, [i][mu] with leading dimension ldt.
 __global__ void zq_c1_split(const double *__restrict__ C, int n, int m1, int ldt, bf16 *__restrict__ hh,
                             bf16 *__restrict__ hl) {
@@ -977,7 +984,7 @@ struct Dims {
 // terms of the dual transform.
 struct Coefs {
   const double *q[4];
-  bool dev = false;  // q[] are device pointers (one matrix: the context's resident SCF orbitals)
+  bool dev = false;  // q[] are addresses a kernel may read (one matrix: resident orbitals, or pinned memory)
 };
 
 // Bytes run_chain carves from a static arena for these dimensions and one coefficient matrix (a
@@ -1037,8 +1044,8 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
       hipLaunchKernelGGL(zq_c1_split, dim3(unsigned(m1)), dim3(256), 0, ctx->stream, dC, n, m1, ldt, d1h, d1l);
     ZQ_LAUNCH_CHECK(ctx, "zq_c_slices");
   } else if (cf.dev) {
-    // C already on the device: the slices are cut there, as above, into the buffers the host staging
-    // below fills
+    // C readable by kernels: the slices are cut on the device, as above, into the buffers the host staging
+    // of the dual transform's matrices below fills
     d1 = (T *)zq_scratch(ctx, "C1", size_t(np) * m1 * sizeof(T), nullptr, false);
     d2t = (T *)zq_scratch(ctx, "C2T", size_t(m2) * np * sizeof(T), nullptr, false);
     d3 = (T *)zq_scratch(ctx, "C3", size_t(np) * m3 * sizeof(T), nullptr, false);
@@ -1238,12 +1245,16 @@ int transform_in(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, Are
 }
 }  // namespace
 
-int zq_transform_device(zq_ctx *ctx, const double *C, int nocc, int block, int precision, void **d_out, int dims[4],
-                        bool *is_f32) {
+int zq_transform_device(zq_ctx *ctx, ZqStage &st, const double *C, int nocc, int block, int precision, void **d_out,
+                        int dims[4], bool *is_f32) {
   Dims d;
   if (int rc = make_dims(ctx, nocc, block, precision, d)) return rc;
+  // C in pinned memory, from where the slices are cut on the device
+  const size_t nn = size_t(ctx->n) * ctx->n;
+  if (int rc = st.take(ctx, nn)) return rc;
+  std::memcpy(st.host, C, nn * sizeof(double));
   Arena ar{ctx};
-  return transform_in(ctx, Coefs{{C, C, C, C}}, d, precision, ar, d_out, dims, is_f32);
+  return transform_in(ctx, Coefs{{st.dev, st.dev, st.dev, st.dev}, true}, d, precision, ar, d_out, dims, is_f32);
 }
 
 extern "C" int zq_ao2mo(zq_ctx *ctx, const double *C, size_t nocc, int block, int precision, double *out) {
@@ -1253,7 +1264,8 @@ extern "C" int zq_ao2mo(zq_ctx *ctx, const double *C, size_t nocc, int block, in
   void *d = nullptr;
   int dims[4];
   bool f32 = false;
-  if (int rc = zq_transform_device(ctx, C, int(nocc), block, precision, &d, dims, &f32)) return rc;
+  ZqStage st;
+  if (int rc = zq_transform_device(ctx, st, C, int(nocc), block, precision, &d, dims, &f32)) return rc;
   const size_t cnt = size_t(dims[0]) * dims[1] * dims[2] * dims[3];
   const double *src = (const double *)d;
   if (f32) {
@@ -1263,9 +1275,9 @@ extern "C" int zq_ao2mo(zq_ctx *ctx, const double *C, size_t nocc, int block, in
     ZQ_LAUNCH_CHECK(ctx, "zq_widen");
     src = wide;
   }
-  ZQ_TRY(ctx, hipMemcpyAsync(out, src, cnt * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  return ZQ_OK;
+  const int rc = zq_read_back(ctx, src, out, cnt);
+  if (rc == ZQ_OK) st.done();
+  return rc;
 }
 
 namespace {
@@ -1279,25 +1291,44 @@ int mp2_in(zq_ctx *ctx, const double *C, const double *e, int nocc, int precisio
   void *T = nullptr;
   int dims[4];
   bool f32 = false, packed = false;
-  if (int rc = transform_in(ctx, Coefs{{C, C, C, C}, dev}, dm, precision, ar, &T, dims, &f32, &packed)) return rc;
+  // host C and e go through pinned memory (but for the entry point that allocates nothing), and the energy
+  // comes back in it
+  const size_t nn = size_t(ctx->n) * ctx->n;
+  const bool fixed = ar.base != nullptr;
+  ZqStage st;
+  if (!fixed) {
+    if (int rc = st.take(ctx, nn + ctx->n + 1)) return rc;
+    if (!dev) {
+      std::memcpy(st.host, C, nn * sizeof(double));
+      std::memcpy(st.host + nn, e, size_t(ctx->n) * sizeof(double));
+      C = st.dev;
+    }
+  }
+  if (int rc = transform_in(ctx, Coefs{{C, C, C, C}, !fixed}, dm, precision, ar, &T, dims, &f32, &packed)) return rc;
   const int o = dims[0], v = dims[2], nij = packed ? o * (o + 1) / 2 : o * o;
   double *de = (double *)ar.get("mp2_e", size_t(ctx->n) * 8);
   double *part = (double *)ar.get("mp2_part", size_t(o) * o * 8 + 8);
-  if (!de || !part) return zq_fail(ctx, ar.base ? ZQ_ERR_INVALID : ZQ_ERR_OOM, "mp2 scratch");
-  ZQ_TRY(ctx, hipMemcpyAsync(de, e, size_t(ctx->n) * 8, dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
-                             ctx->stream));
+  if (!de || !part) return zq_fail(ctx, fixed ? ZQ_ERR_INVALID : ZQ_ERR_OOM, "mp2 scratch");
+  const double *ev = dev ? e : de;
+  if (fixed)
+    ZQ_TRY(ctx, hipMemcpyAsync(de, e, size_t(ctx->n) * 8, hipMemcpyHostToDevice, ctx->stream));
+  else if (!dev)
+    hipLaunchKernelGGL(zq_take, dim3(unsigned((ctx->n + 255) / 256)), dim3(256), 0, ctx->stream, st.dev + nn, ctx->n, de);
+  double *sum = fixed ? part + nij : st.dev + nn + ctx->n;
   zq_prof_begin(ctx, "mp2_energy");
   if (f32)
-    hipLaunchKernelGGL(zq_mp2_pairs<float>, dim3(unsigned(nij)), dim3(256), 0, ctx->stream, (const float *)T, de, o, v,
+    hipLaunchKernelGGL(zq_mp2_pairs<float>, dim3(unsigned(nij)), dim3(256), 0, ctx->stream, (const float *)T, ev, o, v,
                        part, int(packed));
   else
-    hipLaunchKernelGGL(zq_mp2_pairs<double>, dim3(unsigned(nij)), dim3(256), 0, ctx->stream, (const double *)T, de, o, v,
+    hipLaunchKernelGGL(zq_mp2_pairs<double>, dim3(unsigned(nij)), dim3(256), 0, ctx->stream, (const double *)T, ev, o, v,
                        part, int(packed));
-  hipLaunchKernelGGL(zq_sum_wave, dim3(1), dim3(64), 0, ctx->stream, part, nij, part + nij);
+  hipLaunchKernelGGL(zq_sum_wave, dim3(1), dim3(64), 0, ctx->stream, part, nij, sum);
   zq_prof_end(ctx);
   ZQ_LAUNCH_CHECK(ctx, "zq_mp2_pairs");
-  ZQ_TRY(ctx, hipMemcpyAsync(e_corr, part + nij, 8, hipMemcpyDeviceToHost, ctx->stream));
+  if (fixed) ZQ_TRY(ctx, hipMemcpyAsync(e_corr, sum, 8, hipMemcpyDeviceToHost, ctx->stream));
   ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  st.done();
+  if (!fixed) *e_corr = st.host[nn + ctx->n];
   return ZQ_OK;
 }
 
@@ -1628,8 +1659,7 @@ extern "C" int zq_ao2mo_dual(zq_ctx *ctx, zq_eri_set *dset, const double *C, con
     const int rc = transform_in(ctx, terms[t], d, ZQ_PREC_FP64, ar, &dv, dims, &f32);
     ctx->eri = own;
     if (rc) return rc;
-    ZQ_TRY(ctx, hipMemcpyAsync(dst, dv, cnt * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    if (int rc2 = zq_read_back(ctx, (const double *)dv, dst, cnt)) return rc2;
     if (t >= 2)
       for (size_t k = 0; k < cnt; ++k) dout[k] += part[k];
   }

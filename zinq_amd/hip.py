@@ -215,7 +215,7 @@ class Context:
 
     def fock_jk(self, H, P, x_exch=0.5):
         H, P = _f64(H), _f64(P)
-        F = np.zeros_like(H)
+        F = np.empty_like(H)
         self._check(self._L.zq_fock_jk(self._h, ptr(H), ptr(P), float(x_exch), ptr(F)))
         return F
 
@@ -223,7 +223,7 @@ class Context:
         """F[d] = H + G(P[d]) for a stack of densities in one ERI pass (H=None: bare G(P[d]))."""
         Ps = _f64(Ps)
         nd, n = Ps.shape[0], Ps.shape[1]
-        F = np.zeros_like(Ps)
+        F = np.empty_like(Ps)
         Hp = ptr(_f64(H)) if H is not None else None
         self._check(self._L.zq_fock_jk_multi(self._h, Hp, ptr(Ps), nd, float(x_exch), ptr(F)))
         return F
@@ -232,9 +232,9 @@ class Context:
         C = _f64(C)
         n = C.shape[0]
         if block == "full":
-            out = np.zeros((n, n, n, n))
+            out = np.empty((n, n, n, n))
         else:
-            out = np.zeros((nocc, nocc, n - nocc, n - nocc))
+            out = np.empty((nocc, nocc, n - nocc, n - nocc))
         self._check(self._L.zq_ao2mo(self._h, ptr(C), nocc, BLOCK[block], PRECISION[precision], ptr(out)))
         return out
 
@@ -256,7 +256,7 @@ class Context:
         C, dC = _f64(C), _f64(dC)
         n = C.shape[0]
         shape = (n, n, n, n) if block == "full" else (nocc, nocc, n - nocc, n - nocc)
-        out, dout = np.zeros(shape), np.zeros(shape)
+        out, dout = np.empty(shape), np.empty(shape)
         self._check(self._L.zq_ao2mo_dual(self._h, dset._h, ptr(C), ptr(dC), nocc, BLOCK[block], ptr(out), ptr(dout)))
         return out, dout
 
@@ -309,7 +309,7 @@ class Context:
         zq_scf_run_device (everything n x n on the GPU; fock_precision="fp32" selects the mixed path)."""
         H, S = _f64(H), _f64(S)
         n = H.shape[0]
-        C, e, P, F = np.zeros((n, n)), np.zeros(n), np.zeros((n, n)), np.zeros((n, n))
+        C, e, P, F = np.empty((n, n)), np.empty(n), np.empty((n, n)), np.empty((n, n))
         opt = ScfOptions(int(diis or 0), int(iterations), float(threshold), int(bool(generalized)),
                          PRECISION[fock_precision])
         res = ScfResult()
@@ -323,7 +323,7 @@ class Context:
         """W, U with A = U diag(W) U^T, W ascending (zq_eigh; eigh of src/linear_algebra.zig:45-71)."""
         A = _f64(A)
         n = A.shape[0]
-        W, U = np.zeros(n), np.zeros((n, n))
+        W, U = np.empty(n), np.empty((n, n))
         self._check(self._L.zq_eigh(self._h, n, ptr(A), ptr(W), ptr(U)))
         return W, U
 
