@@ -10,13 +10,10 @@
 //   k_batch_count: molecules done, read by the host one iteration late.
 // The step is scf_step of zq_step.h, the one the device SCF of a small molecule runs, certified folds included.
 // Every per-molecule matrix lives in one workspace with leading dimension mp = n rounded up to 16 and
-// zero padding, so the small GEMMs of the eigenpair stage (zq_tile.h, A B^T on FP64 MFMA, one wave per
-// 16 x 16 tile) never need bounds checks.  After convergence: F' of the last extrapolated F for each molecule, rocSOLVER
-// dsyevd_strided_batched per distinct n, C = X V, and the MP2 energy from the OVOV transform of
+// zero padding, so the small GEMMs of the orbitals (zq_tile.h, A B^T on FP64 MFMA, one wave per
+// 16 x 16 tile) never need bounds checks.  After convergence: F' of the last extrapolated F, its eigenpairs and
+// C = X V in one launch, a workgroup per molecule (zq_jacobi.h), and the MP2 energy from the OVOV transform of
 // zq_transform.hip through a context that views the molecule's resident quartets.
-
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <atomic>
@@ -31,6 +28,7 @@
 
 #include "../../include/zinq_batch.h"
 #include "zq_internal.h"
+#include "zq_jacobi.h"
 #include "zq_linalg.h"
 #include "zq_step.h"
 #include "zq_tile.h"
@@ -129,46 +127,65 @@ __global__ void k_batch_count(const int *__restrict__ done, int m, int *__restri
   if (threadIdx.x == 0) *out = red[0];
 }
 
-// F' = X^T W X of every molecule into eig (n x n, leading dimension n, at eoff[m]).
-template <int NT>
-__global__ __launch_bounds__(NT) void k_batch_fprime(double *__restrict__ ws, const BMol *__restrict__ mols,
-                                                     double *__restrict__ eig, const long long *__restrict__ eoff) {
-  const BMol M = mols[blockIdx.x];
-  const int n = M.n, mp = M.mp;
-  const size_t mm = size_t(mp) * mp;
-  double *base = ws + M.ws;
-  double *XT = base + M_XT * mm, *W = base + M_W * mm, *T = base + M_T * mm, *Fpr = base + M_FPR * mm;
-  wg_gemm_nt<NT>(XT, W, T, mp, 1.0);
-  wg_gemm_nt<NT>(T, XT, Fpr, mp, 1.0);
-  double *out = eig + eoff[blockIdx.x];
-  for (int x = threadIdx.x; x < n * n; x += NT) {
-    const int i = x / n, j = x - i * n;
-    out[x] = 0.5 * (Fpr[size_t(i) * mp + j] + Fpr[size_t(j) * mp + i]);
-  }
-}
-
-// C = X V with the eigenvectors of eig (column-major: eigenvector k at eig[eoff + k*n ...]) into
-// cout (n x n, leading dimension n, at coff[m]).
-template <int NT>
-__global__ __launch_bounds__(NT) void k_batch_coef(double *__restrict__ ws, const BMol *__restrict__ mols,
-                                                   const double *__restrict__ eig, const long long *__restrict__ eoff,
-                                                   double *__restrict__ cout, const long long *__restrict__ coff) {
-  const BMol M = mols[blockIdx.x];
-  const int n = M.n, mp = M.mp;
-  const size_t mm = size_t(mp) * mp;
-  double *base = ws + M.ws;
-  double *X = base + M_X * mm, *T = base + M_T * mm, *FP = base + M_FP * mm;
-  const double *V = eig + eoff[blockIdx.x];
-  for (size_t x = threadIdx.x; x < mm; x += NT) {
-    const int k = int(x / mp), p = int(x - size_t(k) * mp);
-    T[x] = (k < n && p < n) ? V[size_t(k) * n + p] : 0.0;
+// Orbitals of molecule order[blockIdx.x]: F' = X^T W X (W the last extrapolated F), its eigenpairs by Jacobi
+// (zq_jacobi.h) on V started as X, so the rotated V is C = X V' at once; e ascending into w + woff, C into
+// cout + coff, columns in the same order, info 1 where the sweeps did not end.
+template <int W>
+__device__ void orbitals(double *lds, const double *X, const double *Fp, int n, int mp, double *__restrict__ e,
+                         double *__restrict__ C, int *__restrict__ info) {
+  zqj::Jacobi<W> J(
+      lds, n, [&](int i, int j) { return 0.5 * (Fp[size_t(i) * mp + j] + Fp[size_t(j) * mp + i]); },
+      [&](int r, int k) { return X[size_t(r) * mp + k]; });
+  bool ok;
+  const bool odd = J.run(&ok) & 1;
+  int *rank = reinterpret_cast<int *>(J.A);  // by position, -1: padding
+  __syncthreads();                           // A is read no more
+  for (int x = threadIdx.x; x < 2 * J.h; x += zqj::kThreads) {
+    const int k = odd ? 2 * J.h - 1 - x : x;  // the index that ended at position x
+    int r = -1;
+    if (k < n) {
+      r = 0;
+      const double d = J.diag[x];
+      for (int y = 0; y < 2 * J.h; ++y) {
+        const int l = odd ? 2 * J.h - 1 - y : y;
+        if (l < n) r += J.diag[y] < d || (J.diag[y] == d && l < k);
+      }
+      if (!ok) r = k;  // NaN has no rank
+      e[r] = d;
+    }
+    rank[x] = r;
   }
   __syncthreads();
-  wg_gemm_nt<NT>(X, T, FP, mp, 1.0);
-  double *out = cout + coff[blockIdx.x];
-  for (int x = threadIdx.x; x < n * n; x += NT) {
-    const int i = x / n, j = x - i * n;
-    out[x] = FP[size_t(i) * mp + j];
+#pragma unroll
+  for (int k = 0; k < J.kRows; ++k) {
+    const int r = J.g + J.kGroups * k;
+    if (r < n && J.i < J.h)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int c = rank[2 * J.i + b];
+        if (c >= 0) C[r * n + c] = J.v[k][b];
+      }
+  }
+  if (threadIdx.x == 0) *info = ok ? 0 : 1;
+}
+
+__global__ __launch_bounds__(zqj::kThreads) void k_batch_orbitals(double *__restrict__ ws, const BMol *__restrict__ mols,
+                                                                  const int *__restrict__ order,
+                                                                  const long long *__restrict__ off, double *__restrict__ e,
+                                                                  double *__restrict__ C, int *__restrict__ info) {
+  extern __shared__ __attribute__((aligned(16))) double step_lds[];
+  const int mi = order[blockIdx.x];
+  const BMol M = mols[mi];
+  const size_t mm = size_t(M.mp) * M.mp;
+  double *base = ws + M.ws;
+  double *X = base + M_X * mm, *XT = base + M_XT * mm, *W = base + M_W * mm, *T = base + M_T * mm, *Fp = base + M_FPR * mm;
+  wg_gemm_nt<zqj::kThreads>(XT, W, T, M.mp, 1.0);
+  wg_gemm_nt<zqj::kThreads>(T, XT, Fp, M.mp, 1.0);
+  const long long *o = off + 2 * mi;
+  switch (zqj::lanes_of(M.n)) {
+    case 16: orbitals<16>(step_lds, X, Fp, M.n, M.mp, e + o[1], C + o[0], info + mi); break;
+    case 32: orbitals<32>(step_lds, X, Fp, M.n, M.mp, e + o[1], C + o[0], info + mi); break;
+    default: orbitals<64>(step_lds, X, Fp, M.n, M.mp, e + o[1], C + o[0], info + mi); break;
   }
 }
 
@@ -202,31 +219,25 @@ struct zq_batch {
   std::vector<long long> eri_off, ws_off;
   size_t eri_count = 0;  // doubles in eri
   int mp_max = 16;       // largest padded size of the batch (the step's LDS)
+  int n_max = 1;         // largest n (the orbitals' LDS)
   int *h_count = nullptr;
   hipGraphExec_t graph = nullptr;
   std::string graph_key;
-  rocblas_handle solver = nullptr;
   // the grouped MP2's FP32 copy of the quartets (FP32 forms; made once per upload) and workspace
   float *eri32 = nullptr;
   void *mp2_ws = nullptr;
   size_t mp2_ws_bytes = 0;
   // the eigenpair stage's device buffers (grow-only, kept across runs) and pinned host copies of C, e and
-  // the solver's info codes, which a second stream brings back while the MP2 runs
-  double *d_eig = nullptr, *d_c = nullptr, *d_w = nullptr, *d_e = nullptr;
+  // the info codes, which a second stream brings back while the MP2 runs
+  double *d_c = nullptr, *d_w = nullptr;
   long long *d_eoff = nullptr;
   int *d_info = nullptr;
-  size_t eig_cap = 0, w_cap = 0, m_cap = 0;  // doubles of d_eig / d_c, of d_w / d_e; molecules
+  size_t c_cap = 0, w_cap = 0, m_cap = 0;  // doubles of d_c, of d_w; molecules
   double *h_c = nullptr, *h_w = nullptr;
   int *h_info = nullptr;
   size_t hc_cap = 0, hw_cap = 0, hi_cap = 0;
   hipStream_t copy_stream = nullptr;
   hipEvent_t coef_done = nullptr;
-  // the eigenpair stage's extra lanes: size groups of the batched eigensolver run side by side, each
-  // lane a stream with its own rocSOLVER handle (its own workspace); fork/join events
-  static constexpr int kEigLanes = 2;
-  hipStream_t eig_lane[kEigLanes] = {};
-  rocblas_handle eig_solver[kEigLanes] = {};
-  hipEvent_t eig_ev[kEigLanes + 1] = {};
   // results of the last run (C and e of molecule m at c_off[m], w_off[m] of h_c, h_w), and its stage
   // times (host wall clock, ms): SCF, eigenpairs, MP2, total
   std::vector<long long> c_off, w_off;
@@ -257,11 +268,11 @@ void free_plan(zq_batch *b) {
 
 void free_eig(zq_batch *b) {
   if (b->copy_stream) (void)hipStreamSynchronize(b->copy_stream);  // copies into the pinned buffers
-  for (void *p : {(void *)b->d_eig, (void *)b->d_c, (void *)b->d_w, (void *)b->d_e, (void *)b->d_eoff, (void *)b->d_info})
+  for (void *p : {(void *)b->d_c, (void *)b->d_w, (void *)b->d_eoff, (void *)b->d_info})
     if (p) (void)hipFree(p);
-  b->d_eig = b->d_c = b->d_w = b->d_e = nullptr;
+  b->d_c = b->d_w = nullptr;
   b->d_eoff = nullptr, b->d_info = nullptr;
-  b->eig_cap = b->w_cap = b->m_cap = 0;
+  b->c_cap = b->w_cap = b->m_cap = 0;
   for (void *p : {(void *)b->h_c, (void *)b->h_w, (void *)b->h_info})
     if (p) (void)hipHostFree(p);
   b->h_c = b->h_w = nullptr, b->h_info = nullptr;
@@ -269,28 +280,20 @@ void free_eig(zq_batch *b) {
 }
 
 // Grow-only device and pinned host buffers of the eigenpair stage.
-int eig_buffers(zq_batch *b, size_t etot, size_t wtot, size_t M) {
-  if (etot > b->eig_cap) {
-    for (double **p : {&b->d_eig, &b->d_c}) {
-      if (*p) (void)hipFree(*p);
-      *p = nullptr;
-    }
+int eig_buffers(zq_batch *b, size_t ctot, size_t wtot, size_t M) {
+  if (ctot > b->c_cap) {
+    if (b->d_c) (void)hipFree(b->d_c);
     if (b->h_c) (void)hipHostFree(b->h_c);
-    b->h_c = nullptr, b->eig_cap = b->hc_cap = 0;
-    BTRY(b, hipMalloc(&b->d_eig, etot * sizeof(double)));
-    BTRY(b, hipMalloc(&b->d_c, etot * sizeof(double)));
-    BTRY(b, hipHostMalloc((void **)&b->h_c, etot * sizeof(double), hipHostMallocDefault));
-    b->eig_cap = b->hc_cap = etot;
+    b->d_c = b->h_c = nullptr, b->c_cap = b->hc_cap = 0;
+    BTRY(b, hipMalloc(&b->d_c, ctot * sizeof(double)));
+    BTRY(b, hipHostMalloc((void **)&b->h_c, ctot * sizeof(double), hipHostMallocDefault));
+    b->c_cap = b->hc_cap = ctot;
   }
   if (wtot > b->w_cap) {
-    for (double **p : {&b->d_w, &b->d_e}) {
-      if (*p) (void)hipFree(*p);
-      *p = nullptr;
-    }
+    if (b->d_w) (void)hipFree(b->d_w);
     if (b->h_w) (void)hipHostFree(b->h_w);
-    b->h_w = nullptr, b->w_cap = b->hw_cap = 0;
+    b->d_w = b->h_w = nullptr, b->w_cap = b->hw_cap = 0;
     BTRY(b, hipMalloc(&b->d_w, wtot * sizeof(double)));
-    BTRY(b, hipMalloc(&b->d_e, wtot * sizeof(double)));
     BTRY(b, hipHostMalloc((void **)&b->h_w, wtot * sizeof(double), hipHostMallocDefault));
     b->w_cap = b->hw_cap = wtot;
   }
@@ -299,7 +302,7 @@ int eig_buffers(zq_batch *b, size_t etot, size_t wtot, size_t M) {
     if (b->d_info) (void)hipFree(b->d_info);
     if (b->h_info) (void)hipHostFree(b->h_info);
     b->d_eoff = nullptr, b->d_info = nullptr, b->h_info = nullptr, b->m_cap = b->hi_cap = 0;
-    BTRY(b, hipMalloc(&b->d_eoff, M * sizeof(long long)));
+    BTRY(b, hipMalloc(&b->d_eoff, 2 * M * sizeof(long long)));
     BTRY(b, hipMalloc(&b->d_info, M * sizeof(int)));
     BTRY(b, hipHostMalloc((void **)&b->h_info, M * sizeof(int), hipHostMallocDefault));
     b->m_cap = b->hi_cap = M;
@@ -393,6 +396,7 @@ int upload(zq_batch *b) {
     canon_max = std::max(canon_max, h.eri.size());
     bm[m] = BMol{(long long)b->ws_off[m], h.n, mp, h.nocc, 0, h.VN};
     b->mp_max = std::max(b->mp_max, mp);
+    b->n_max = std::max(b->n_max, h.n);
     jm[m] = JKMol{b->eri_off[m], b->ws_off[m] + M_P * (long long)mm, b->ws_off[m] + M_H * (long long)mm,
                   b->ws_off[m] + M_F * (long long)mm, mp, h.n};
   }
@@ -523,14 +527,6 @@ void zq_batch_destroy(zq_batch *b) {
   if (b->copy_stream) (void)hipStreamSynchronize(b->copy_stream);
   free_all(b);
   if (b->h_count) (void)hipHostFree(b->h_count);
-  if (b->solver) rocblas_destroy_handle(b->solver);
-  for (int l = 0; l < zq_batch::kEigLanes; ++l) {
-    if (b->eig_lane[l]) (void)hipStreamSynchronize(b->eig_lane[l]);
-    if (b->eig_solver[l]) rocblas_destroy_handle(b->eig_solver[l]);
-    if (b->eig_lane[l]) (void)hipStreamDestroy(b->eig_lane[l]);
-  }
-  for (hipEvent_t e : b->eig_ev)
-    if (e) (void)hipEventDestroy(e);
   if (b->coef_done) (void)hipEventDestroy(b->coef_done);
   if (b->copy_stream) (void)hipStreamDestroy(b->copy_stream);
   (void)hipStreamDestroy(b->stream);
@@ -667,88 +663,27 @@ int zq_batch_run(zq_batch *b, const zq_scf_options *opt, int mp2_precision, doub
   b->stage_ms[0] = since(t0);
   const auto t1 = std::chrono::steady_clock::now();
 
-  // eigenpairs of X^T F_ext X: molecules ordered by n so that each size is one strided batch
-  std::vector<int> order(M);
-  for (int m = 0; m < M; ++m) order[m] = m;
-  std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return b->mols[a].n < b->mols[c].n; });
-  std::vector<long long> eoff(M), coff(M), woff(M);
-  long long etot = 0, wtot = 0;
-  for (int m : order) {
-    eoff[m] = etot, woff[m] = wtot;
-    etot += (long long)b->mols[m].n * b->mols[m].n;
+  // orbitals of the last extrapolated F, one workgroup per molecule
+  std::vector<long long> off(2 * size_t(M)), coff(M), woff(M);
+  long long ctot = 0, wtot = 0;
+  for (int m = 0; m < M; ++m) {
+    off[2 * m] = coff[m] = ctot, off[2 * m + 1] = woff[m] = wtot;
+    ctot += (long long)b->mols[m].n * b->mols[m].n;
     wtot += b->mols[m].n;
   }
-  for (int m = 0; m < M; ++m) coff[m] = eoff[m];
   // the previous run's copies of C and e must have landed before their buffers are reused
   if (b->copy_stream) BTRY(b, hipStreamSynchronize(b->copy_stream));
-  if (int rc = eig_buffers(b, size_t(etot), size_t(wtot), size_t(M))) return rc;
-  double *d_eig = b->d_eig, *d_w = b->d_w, *d_e = b->d_e, *d_c = b->d_c;
-  long long *d_eoff = b->d_eoff;
+  if (int rc = eig_buffers(b, size_t(ctot), size_t(wtot), size_t(M))) return rc;
+  double *d_w = b->d_w, *d_c = b->d_c;
   int *d_info = b->d_info;
-  BTRY(b, hipMemcpyAsync(d_eoff, eoff.data(), M * sizeof(long long), hipMemcpyHostToDevice, b->stream));
-  if (b->nt == 512)
-    hipLaunchKernelGGL(k_batch_fprime<512>, dim3(M), dim3(512), 0, b->stream, b->ws, b->d_mols, d_eig, d_eoff);
-  else
-    hipLaunchKernelGGL(k_batch_fprime<256>, dim3(M), dim3(256), 0, b->stream, b->ws, b->d_mols, d_eig, d_eoff);
-  BTRY(b, hipGetLastError());
-  if (!b->solver) {
-    if (rocblas_create_handle(&b->solver) != rocblas_status_success) return bfail(b, ZQ_ERR_LAPACK, "rocblas handle");
-  }
-  rocblas_set_stream(b->solver, b->stream);
-  for (int l = 0; l < zq_batch::kEigLanes; ++l) {
-    if (!b->eig_lane[l]) BTRY(b, hipStreamCreateWithFlags(&b->eig_lane[l], hipStreamNonBlocking));
-    if (!b->eig_solver[l]) {
-      if (rocblas_create_handle(&b->eig_solver[l]) != rocblas_status_success)
-        return bfail(b, ZQ_ERR_LAPACK, "rocblas handle");
-      rocblas_set_stream(b->eig_solver[l], b->eig_lane[l]);
-    }
-  }
-  for (hipEvent_t &e : b->eig_ev)
-    if (!e) BTRY(b, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  // one strided batch per distinct n; the groups go to the least loaded lane (the batch's stream is
-  // lane 0), largest first by n^3 x count
-  struct Group {
-    int s, cnt, n;
-    double cost;
-  };
-  std::vector<Group> groups;
-  for (int s = 0; s < M;) {
-    const int n = b->mols[order[s]].n;
-    int t = s;
-    while (t < M && b->mols[order[t]].n == n) ++t;
-    groups.push_back(Group{s, t - s, n, double(n) * n * n * (t - s)});
-    s = t;
-  }
-  std::stable_sort(groups.begin(), groups.end(), [](const Group &x, const Group &y) { return x.cost > y.cost; });
-  BTRY(b, hipEventRecord(b->eig_ev[0], b->stream));  // F' is ready
-  for (int l = 0; l < zq_batch::kEigLanes; ++l) BTRY(b, hipStreamWaitEvent(b->eig_lane[l], b->eig_ev[0], 0));
-  double load[zq_batch::kEigLanes + 1] = {};
-  for (const Group &g : groups) {
-    int lane = 0;
-    for (int l = 1; l <= zq_batch::kEigLanes; ++l)
-      if (load[l] < load[lane]) lane = l;
-    load[lane] += g.cost;
-    const int m0 = order[g.s];
-    const rocblas_status rs = rocsolver_dsyevd_strided_batched(
-        lane == 0 ? b->solver : b->eig_solver[lane - 1], rocblas_evect_original, rocblas_fill_upper, g.n,
-        d_eig + eoff[m0], g.n, rocblas_stride(g.n) * g.n, d_w + woff[m0], rocblas_stride(g.n), d_e + woff[m0],
-        rocblas_stride(g.n), d_info + g.s, g.cnt);
-    if (rs != rocblas_status_success) return bfail(b, ZQ_ERR_LAPACK, "rocsolver_dsyevd_strided_batched");
-  }
-  // the batch's stream waits for every lane before the eigenvectors are used
-  for (int l = 0; l < zq_batch::kEigLanes; ++l) {
-    BTRY(b, hipEventRecord(b->eig_ev[1 + l], b->eig_lane[l]));
-    BTRY(b, hipStreamWaitEvent(b->stream, b->eig_ev[1 + l], 0));
-  }
-  if (b->nt == 512)
-    hipLaunchKernelGGL(k_batch_coef<512>, dim3(M), dim3(512), 0, b->stream, b->ws, b->d_mols, d_eig, d_eoff, d_c, d_eoff);
-  else
-    hipLaunchKernelGGL(k_batch_coef<256>, dim3(M), dim3(256), 0, b->stream, b->ws, b->d_mols, d_eig, d_eoff, d_c, d_eoff);
+  BTRY(b, hipMemcpyAsync(b->d_eoff, off.data(), off.size() * sizeof(long long), hipMemcpyHostToDevice, b->stream));
+  hipLaunchKernelGGL(k_batch_orbitals, dim3(M), dim3(zqj::kThreads), zqj::lds_doubles(b->n_max) * sizeof(double), b->stream,
+                     b->ws, b->d_mols, b->d_order, b->d_eoff, d_w, d_c, d_info);
   BTRY(b, hipGetLastError());
   // C, e and the info codes go to pinned host memory on the copy stream, overlapped with the MP2
   BTRY(b, hipEventRecord(b->coef_done, b->stream));
   BTRY(b, hipStreamWaitEvent(b->copy_stream, b->coef_done, 0));
-  BTRY(b, hipMemcpyAsync(b->h_c, d_c, etot * sizeof(double), hipMemcpyDeviceToHost, b->copy_stream));
+  BTRY(b, hipMemcpyAsync(b->h_c, d_c, ctot * sizeof(double), hipMemcpyDeviceToHost, b->copy_stream));
   BTRY(b, hipMemcpyAsync(b->h_w, d_w, wtot * sizeof(double), hipMemcpyDeviceToHost, b->copy_stream));
   BTRY(b, hipMemcpyAsync(b->h_info, d_info, M * sizeof(int), hipMemcpyDeviceToHost, b->copy_stream));
   b->c_off = coff, b->w_off = woff;
@@ -817,14 +752,12 @@ int zq_batch_run(zq_batch *b, const zq_scf_options *opt, int mp2_precision, doub
   }
   b->stage_ms[2] = since(t2);
   BTRY(b, hipStreamSynchronize(b->copy_stream));  // C, e and the info codes are on the host
-  std::vector<int> info(M);  // rocSOLVER wrote info by batch position; by molecule here
-  for (int s = 0; s < M; ++s) info[order[s]] = b->h_info[s] ? 1 : 0;
   b->stage_ms[3] = since(t0);
   for (int m = 0; m < M; ++m) {
     E_rhf[m] = hs[m].energy;
     iterations[m] = hs[m].it;
     status[m] = hs[m].done == 1 ? ZQ_OK : hs[m].done == 2 ? ZQ_ERR_NOT_CONVERGED : ZQ_ERR_LAPACK;
-    if (info[m] && status[m] == ZQ_OK) status[m] = ZQ_ERR_LAPACK;
+    if (b->h_info[m] && status[m] == ZQ_OK) status[m] = ZQ_ERR_LAPACK;
     if (rc_m[m] != ZQ_OK && status[m] == ZQ_OK) status[m] = rc_m[m];
   }
   return ZQ_OK;
