@@ -2,17 +2,18 @@
 // geigh in src/linear_algebra.zig:45-71, :184-199 (LAPACKE_dsyevd / dsygvd) on the GPU.
 //
 // rocSOLVER's dsyevd spends most of its time at these sizes launching the many small kernels of its
-// tridiagonal reduction (about 2.4 ms of 3.9 ms at n = 192).  Here the reduction is one workgroup:
-//
-// k_tridiag: 512 threads hold the n x n matrix in registers (thread (tr, tc) = (tid / 8, tid % 8) owns
-//   rows tr + 64 a and columns tc + 8 b), two waves per SIMD, so the per-step scalar work is issued
-//   twice per SIMD rather than for every one of many waves.  Householder reduction of the lower
-//   triangle as LAPACK dsytd2 (A = Q T Q^T, Q = H_0 ... H_(n-3)), step k:
+// tridiagonal reduction (about 2.4 ms of 3.9 ms at n = 192).  Here the reduction is one workgroup of 512 threads
+// that hold the matrix in registers: Householder reduction of the lower triangle as LAPACK dsytd2 (A = Q T Q^T,
+// Q = H_0 ... H_(n-3)), step k:
 //     row k -> LDS; alpha = A[k+1][k], beta = -sign(alpha) |A[k+1:][k]|, tau = (beta - alpha) / beta,
-//     v = (1, A[k+2:][k] / (alpha - beta));  p = tau A v;  w = p - tau/2 (p.v) v;  A -= v w^T + w v^T,
-//   two barriers a step; every wave computes the step's scalars itself, in the same order, so all agree
-//   bitwise; column blocks wholly left of k are skipped.  The reflectors stay in LDS until the end,
-//   when they go to global memory.
+//     v = (1, A[k+2:][k] / (alpha - beta));  p = tau A v;  w = p - tau/2 (p.v) v;  A -= v w^T + w v^T.
+// A step is bound by its serial chain, which every wave computes for itself, in the same order, so all
+// agree bitwise.  Two forms:
+// k_tridiag (n <= 32): two barriers a step, each quantity formed directly.
+// k_tridiag_wide (33 <= n <= 192): one barrier a step, the rank-2 update and the next product in one pass.  Its
+//   rounding differs; n <= 32 keeps the first form since the eigenvectors of a symmetric molecule (one water)
+//   take their signs from rounding there.  It is also the faster there: n = 24 29 us.
+// The reflectors stay in LDS until the end, when they go to global memory.
 // k_tridiag_q: Q^T = H_(n-3) ... H_0 accumulated in registers (same layout) by right multiplications
 //   M <- M H_k, whose row sums (quad sums) need no barrier.  It runs on a second stream while the
 //   tridiagonal problem is solved, which needs only d and e.
@@ -57,31 +58,23 @@ __device__ inline int vofs(int k, int n) { return k * (n - 1) - k * (k - 1) / 2;
 
 // A (n x n symmetric, ld lda) -> d (n), e (n - 1) and the reflectors R (refl_words(n): tau, scal, the
 // packed row tails) of A = Q T Q^T, n <= 16 RB.
-// One workgroup of 16 TR threads per matrix of a strided batch.  Thread (tr, tc) = (tid / 16, tid % 16)
-// owns rows tr + TR a (a < RA) and columns tc + 16 b (b < RB), at most 72 doubles (TR = 32 keeps two
-// waves per SIMD, so they fit the 256 registers a lane then has); a DPP row of 16 lanes holds one
-// thread row, so a row sum is four DPP steps.  Row k (= column k, A symmetric) reaches
-// LDS from the 16 lanes that own it, together with |A[k+2:][k]|^2, which they sum on the way.  p.v is
-// summed per wave into LDS before the step's second barrier and then added up in a fixed order, so no
-// step waits on a 64-lane shuffle reduction.  Row vectors in LDS are stored column-permuted,
+// One workgroup of 16 TR threads.  Thread (tr, tc) = (tid / 16, tid % 16) owns rows tr + TR a (a < RA) and
+// columns tc + 16 b (b < RB); a DPP row of 16 lanes holds one thread row, so a row sum is four DPP steps.  Row k
+// (= column k, A symmetric) reaches LDS from the 16 lanes that own it, together with |A[k+2:][k]|^2, which they
+// sum on the way.  p.v is summed per wave into LDS before the step's second barrier and then added up in a
+// fixed order, so no step waits on a 64-lane shuffle reduction.  Row vectors in LDS are stored column-permuted,
 // [c % 16][c / 16] with a padded stride, so a lane reads its own columns contiguously and the 16
-// column groups fall in different banks.  The reflectors (raw row tails and 1 / (alpha - beta)), d, e
-// and tau stay in LDS (at most 156 KB for n = 192) until the loop has ended, so no barrier waits for a
-// global store.
+// column groups fall in different banks.  Sized for 32 (8 waves, two columns a lane) rather than the 64 it
+// used to serve (16 waves, four): n = 7 13 -> 8 us, n = 24 46 -> 29, n = 32 62 -> 39, the same bits.
 template <int RB, int TR>
-__global__ __launch_bounds__(16 * TR) void k_tridiag(const double *__restrict__ A, int lda, long long sA, int n,
-                                                  double *__restrict__ d, double *__restrict__ e, long long sDE,
-                                                  double *__restrict__ R, long long sR) {
+__global__ __launch_bounds__(16 * TR) void k_tridiag(const double *__restrict__ A, int lda, int n, double *__restrict__ d,
+                                                  double *__restrict__ e, double *__restrict__ R) {
   constexpr int NT = 16 * TR, NM = 16 * RB, RA = (NM + TR - 1) / TR, CS = RB + 1;
   __shared__ double cbp[2][16 * CS];  // row k, permuted
   __shared__ double pvp[16 * CS];     // p = tau A v, permuted
   __shared__ double xn[2], pdot[2][TR / 4];
   __shared__ double taus[NM], scals[NM], dl[NM], el[NM];
   __shared__ double vl[(NM - 2) * (NM + 1) / 2];
-  A += blockIdx.x * sA;
-  d += blockIdx.x * sDE;
-  e += blockIdx.x * sDE;
-  R += blockIdx.x * sR;
   const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15, wv = tid >> 6;
   auto P = [](int j) { return (j & 15) * CS + (j >> 4); };
   double a[RA][RB];
@@ -211,18 +204,176 @@ __global__ __launch_bounds__(16 * TR) void k_tridiag(const double *__restrict__ 
   for (int t = tid; t < nv; t += NT) R[2 * n + t] = vl[t];
 }
 
-// Q from the reflectors k_tridiag left in R (one workgroup per matrix of the batch, the same thread
+// The same reduction for 32 < n <= 192 with one barrier a step and one pass over the registers.  512 threads,
+// thread (tr, tc) = (tid / 16, tid % 16) owns rows tr + 32 a and columns tc + 16 b.  With u the reflector's
+// direction scaled by a power of two near 1 / |beta| (u_(k+1) = (alpha - beta) s, u_j = A[k][j] s) and
+// g = 2 / u.u, step k is p = A u, w = g p - g^2 / 2 (p.u) u, A -= u w^T + w u^T.  Between two barriers:
+//   from p of the last step and the not yet updated row k, both in LDS, every 16-lane row works out p.u, w, the
+//   updated row k, its norm and the next u for its own columns and rows by itself;
+//   one pass then applies the last step's update and multiplies by the next u, three FMAs an element;
+//   the row sums p and the next row, k + 1, go to LDS.
+// The quotient g is needed only after the barrier, so it passes in the shadow of the pass; tau and
+// 1 / (alpha - beta) of the stored reflectors are computed at the end.  The steps run in stages of 32, one per row
+// block AK, which makes the finished rows and columns (blocks below AK, 2 AK) drop out at compile time;
+// smaller matrices start at a later stage (index shift 32 AK0), so one kernel serves every n.
+// Against the two-barrier form, which went over all of A twice a step: n = 150 709 -> 235 us, n = 64 130 -> 68,
+// n = 33 64 -> 37.
+constexpr int kWideRB = 12, kWideRA = kWideRB / 2, kWideN = 16 * kWideRB;
+
+// Sum over the 16 lanes of a DPP row, on every lane.
+__device__ inline double row_sum_all(double v) {
+  v += dpp_move<0xB1>(v);   // quad_perm 1 0 3 2
+  v += dpp_move<0x4E>(v);   // quad_perm 2 3 0 1
+  v += dpp_move<0x141>(v);  // half-row mirror
+  v += dpp_move<0x128>(v);  // rotate by 8
+  return v;
+}
+
+struct WideShared {
+  static constexpr int CS = kWideRB + 1;
+  double row[2][16 * CS], p[2][16 * CS];  // columns permuted, [c % 16][c / 16]
+  double alpha[kWideN], beta[kWideN], d[kWideN];
+  double tail[(kWideN - 2) * (kWideN + 1) / 2];
+};
+
+// What a step hands on to the next.
+struct WideState {
+  double a[kWideRA][kWideRB];        // this thread's elements
+  double uc[kWideRB], ur[kWideRA];   // the last u on its columns and rows
+  double g, u1, s;                   // the last g, u_(k+1) and scale
+};
+
+// The steps whose next row, k + 1, lies in row block AK: kk + 1 in [32 AK, 32 AK + 32), kk = k + shift.
+template <int AK>
+__device__ inline void wide_stage(WideState &t, WideShared &sh, int n, int shift) {
+  constexpr int CS = WideShared::CS, B0 = 2 * AK;
+  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15, end = n + shift;
+  auto P = [](int j) { return (j & 15) * CS + (j >> 4); };
+  const int k0 = max(32 * AK - 1, shift), k1 = min(32 * AK + 31, end - 1);
+  for (int kk = k0; kk < k1; ++kk) {
+    const int k = kk - shift, cur = kk & 1;
+    const double *row = sh.row[cur], *pl = sh.p[cur];
+    // w of the last step
+    // a stage's first u starts at column 32 AK - 1, which its blocks leave out
+    double dot = AK && kk == 32 * AK - 1 && tc == 15 ? pl[P(kk)] * t.u1 : 0.0;
+#pragma unroll
+    for (int b = B0; b < kWideRB; ++b) dot = fma(pl[tc * CS + b], t.uc[b], dot);
+    const double K = -0.5 * t.g * t.g * row_sum_all(dot);
+    double wc[kWideRB], wr[kWideRA];
+#pragma unroll
+    for (int b = B0; b < kWideRB; ++b) wc[b] = fma(K, t.uc[b], t.g * pl[tc * CS + b]);
+#pragma unroll
+    for (int a = AK; a < kWideRA; ++a) wr[a] = fma(K, t.ur[a], t.g * pl[P(tr + 32 * a)]);
+    // row k, updated, on this thread's columns; its norm beyond k + 1
+    const double wk = fma(K, t.u1, t.g * pl[P(kk)]);
+    double x[kWideRB], norm2 = 0.0;
+#pragma unroll
+    for (int b = B0; b < kWideRB; ++b) {
+      x[b] = fma(-wk, t.uc[b], fma(-t.u1, wc[b], row[tc * CS + b]));
+      const double y = tc + 16 * b >= kk + 2 ? x[b] : 0.0;
+      norm2 = fma(y, y, norm2);
+    }
+    norm2 = row_sum_all(norm2);
+    const double u2 = k > 0 ? sh.tail[vofs(k - 1, n) + 1] * t.s : 0.0;  // the last u at k + 1
+    const double alpha = fma(-wk, u2, fma(-t.u1, fma(K, u2, t.g * pl[P(kk + 1)]), row[P(kk + 1)]));
+    double beta = alpha;
+    if (norm2 != 0.0) beta = -copysign(sqrt(fma(alpha, alpha, norm2)), alpha);
+    const double s = __builtin_ldexp(1.0, min(1000, 1 - __builtin_amdgcn_frexp_exp(beta)));
+    const double as = alpha * s, bs = beta * s, u1 = as - bs;
+    // the row's raw tail for the back-accumulation: v_k[j] = tail[j] / (alpha - beta)
+    if (tr == 0 && k < n - 2) {
+#pragma unroll
+      for (int b = B0; b < kWideRB; ++b) {
+        const int j = tc + 16 * b;
+        if (j > kk && j < end) sh.tail[vofs(k, n) + j - kk - 1] = j == kk + 1 ? alpha : x[b];
+      }
+    }
+    if (tid == 0) sh.d[k] = fma(-2.0 * t.u1, wk, row[P(kk)]), sh.alpha[k] = alpha, sh.beta[k] = beta;
+    double xr[kWideRA], pt[kWideRA];
+#pragma unroll
+    for (int a = AK; a < kWideRA; ++a) {
+      const int r = tr + 32 * a;
+      const double y = fma(-wk, t.ur[a], fma(-t.u1, wr[a], row[P(r)])) * s;
+      xr[a] = r > kk + 1 ? y : (r == kk + 1 ? u1 : 0.0);
+      pt[a] = 0.0;
+    }
+#pragma unroll
+    for (int b = B0; b < kWideRB; ++b) {
+      const int j = tc + 16 * b;
+      x[b] = j > kk + 1 ? x[b] * s : (j == kk + 1 ? u1 : 0.0);
+#pragma unroll
+      for (int a = AK; a < kWideRA; ++a) {
+        t.a[a][b] = fma(-wr[a], t.uc[b], fma(-t.ur[a], wc[b], t.a[a][b]));
+        pt[a] = fma(t.a[a][b], x[b], pt[a]);
+      }
+      t.uc[b] = x[b];
+    }
+    if (tr == ((kk + 1) & 31))
+#pragma unroll
+      for (int b = B0; b < kWideRB; ++b) sh.row[cur ^ 1][tc * CS + b] = t.a[AK][b];
+#pragma unroll
+    for (int a = AK; a < kWideRA; ++a) {
+      const double q = row_sum_last(pt[a]);
+      if (tc == 15) sh.p[cur ^ 1][P(tr + 32 * a)] = q;
+      t.ur[a] = xr[a];
+    }
+    t.g = norm2 != 0.0 ? 1.0 / (bs * bs - as * bs) : 0.0;
+    t.u1 = u1, t.s = s;
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(512) void k_tridiag_wide(const double *__restrict__ A, int lda, int n, double *__restrict__ d,
+                                                      double *__restrict__ e, double *__restrict__ R) {
+  constexpr int CS = WideShared::CS;
+  __shared__ WideShared sh;
+  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
+  const int start = kWideRA - (n + 31) / 32, shift = 32 * start;
+  auto P = [](int j) { return (j & 15) * CS + (j >> 4); };
+  WideState t;
+#pragma unroll
+  for (int a = 0; a < kWideRA; ++a)
+#pragma unroll
+    for (int b = 0; b < kWideRB; ++b) {
+      const int r = tr + 32 * a - shift, c = tc + 16 * b - shift;
+      t.a[a][b] = (r >= 0 && c >= 0 && r < n && c < n) ? A[size_t(r) * lda + c] : 0.0;
+    }
+#pragma unroll
+  for (int b = 0; b < kWideRB; ++b) t.uc[b] = 0.0;
+#pragma unroll
+  for (int a = 0; a < kWideRA; ++a) t.ur[a] = 0.0;
+  t.g = t.u1 = 0.0, t.s = 1.0;
+  for (int x = tid; x < 2 * 16 * CS; x += 512) (&sh.p[0][0])[x] = (&sh.row[0][0])[x] = 0.0;
+  __syncthreads();
+  for (int c = tid; c < n; c += 512) sh.row[shift & 1][P(c + shift)] = A[c];  // row 0
+  __syncthreads();
+  if (start <= 0) wide_stage<0>(t, sh, n, shift);
+  if (start <= 1) wide_stage<1>(t, sh, n, shift);
+  if (start <= 2) wide_stage<2>(t, sh, n, shift);
+  if (start <= 3) wide_stage<3>(t, sh, n, shift);
+  wide_stage<4>(t, sh, n, shift);
+  wide_stage<5>(t, sh, n, shift);
+  // the last step (n - 2, no reflector) left row n - 1; d and e, then the reflectors
+  const int nk = n - 2, nv = vofs(n - 2, n), last = n - 1 + shift;
+  for (int k = tid; k < n; k += 512) d[k] = k < n - 1 ? sh.d[k] : sh.row[last & 1][P(last)];
+  for (int k = tid; k < n - 1; k += 512) e[k] = sh.beta[k];
+  for (int k = tid; k < nk; k += 512) {
+    const double al = sh.alpha[k], be = sh.beta[k];
+    R[k] = be != al ? (be - al) / be : 0.0;
+    R[n + k] = be != al ? 1.0 / (al - be) : 0.0;
+  }
+  for (int x = tid; x < nv; x += 512) R[2 * n + x] = sh.tail[x];
+}
+
+// Q from the reflectors k_tridiag left in R (one workgroup, the same thread
 // layout): M = Q^T = H_(n-3) ... H_0, from M = I by M <- M H_k = M - tau (M v) v^T for k = n-3 .. 0,
 // whose row sums (quad sums) need no barrier; then Q[c][r] = M[r][c].  It runs beside the tridiagonal
 // eigensolver, which needs only d and e.
 template <int RB, int TR>
-__global__ __launch_bounds__(16 * TR) void k_tridiag_q(const double *__restrict__ R, long long sR, int n,
-                                                    double *__restrict__ Q, long long sQ) {
+__global__ __launch_bounds__(16 * TR) void k_tridiag_q(const double *__restrict__ R, int n, double *__restrict__ Q) {
   constexpr int NT = 16 * TR, NM = 16 * RB, RA = (NM + TR - 1) / TR;
   __shared__ double taus[NM], scals[NM];
   __shared__ double vl[(NM - 2) * (NM + 1) / 2];
-  R += blockIdx.x * sR;
-  Q += blockIdx.x * sQ;
   const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
   const int nk = n > 2 ? n - 2 : 0, nv = n > 2 ? vofs(n - 2, n) : 0;
   for (int t = tid; t < nk; t += NT) taus[t] = R[t], scals[t] = R[n + t];
@@ -279,15 +430,20 @@ __global__ __launch_bounds__(16 * TR) void k_tridiag_q(const double *__restrict_
 inline size_t refl_words(int n) { return 2 * size_t(n) + (n > 2 ? size_t(n - 2) * (n + 1) / 2 : 0); }
 
 // The reduction on s; Q on s2, which waits for it, while s goes on (the caller joins s2 back).
-template <int RB, int TR>
-hipError_t launch_tridiag(hipStream_t s, hipStream_t s2, hipEvent_t fork, int count, const double *A, int lda,
-                          long long sA, int n, double *d, double *e, long long sDE, double *R, double *Q,
-                          long long sQ) {
-  const long long sR = (long long)refl_words(n);
-  hipLaunchKernelGGL((k_tridiag<RB, TR>), dim3(count), dim3(16 * TR), 0, s, A, lda, sA, n, d, e, sDE, R, sR);
+hipError_t launch_tridiag(hipStream_t s, hipStream_t s2, hipEvent_t fork, const double *A, int lda, int n, double *d,
+                          double *e, double *R, double *Q) {
+  if (n <= 32)
+    hipLaunchKernelGGL((k_tridiag<2, 32>), dim3(1), dim3(512), 0, s, A, lda, n, d, e, R);
+  else
+    hipLaunchKernelGGL(k_tridiag_wide, dim3(1), dim3(512), 0, s, A, lda, n, d, e, R);
   if (hipError_t err = hipEventRecord(fork, s)) return err;
   if (hipError_t err = hipStreamWaitEvent(s2, fork, 0)) return err;
-  hipLaunchKernelGGL((k_tridiag_q<RB, TR>), dim3(count), dim3(16 * TR), 0, s2, R, sR, n, Q, sQ);
+  if (n <= 64)
+    hipLaunchKernelGGL((k_tridiag_q<4, 64>), dim3(1), dim3(1024), 0, s2, R, n, Q);
+  else if (n <= 128)
+    hipLaunchKernelGGL((k_tridiag_q<8, 64>), dim3(1), dim3(1024), 0, s2, R, n, Q);
+  else
+    hipLaunchKernelGGL((k_tridiag_q<12, 32>), dim3(1), dim3(512), 0, s2, R, n, Q);
   return hipGetLastError();
 }
 
@@ -355,13 +511,7 @@ int zq_syev_rows(zq_ctx *ctx, double *A, int n, double *w, double *offd, int *in
     if (!ev) ZQ_TRY(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   hipStream_t s = ctx->stream;
   hipEvent_t fork = ctx->eig_events[0], join = ctx->eig_events[1];
-  hipError_t le;
-  if (n <= 64)
-    le = launch_tridiag<4, 64>(s, s2, fork, 1, A, n, 0, n, w, offd, 0, R, Qm, 0);
-  else if (n <= 128)
-    le = launch_tridiag<8, 64>(s, s2, fork, 1, A, n, 0, n, w, offd, 0, R, Qm, 0);
-  else
-    le = launch_tridiag<12, 32>(s, s2, fork, 1, A, n, 0, n, w, offd, 0, R, Qm, 0);
+  const hipError_t le = launch_tridiag(s, s2, fork, A, n, n, w, offd, R, Qm);
   if (le != hipSuccess) {
     zq_prof_end(ctx);
     return zq_check(ctx, le, "k_tridiag");
