@@ -1,0 +1,43 @@
+"""The first quarter transform at the edges of its layouts: one block and odd numbers of blocks, occupied counts on
+both sides of its 16-column tiles, against the transform in float64.  Bound of an element: four chained sums of n
+products each, 4 n eps times the same transform of the absolute values (eps of the element type, once more for
+rounding the integrals and coefficients to it)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from zinq_amd import hip
+    c = hip.Context(0)
+    yield c
+    c.close()
+
+
+def _ovov(g, C, o):
+    X = np.einsum("mnls,mi->inls", g, C[:, :o], optimize=True)
+    X = np.einsum("inls,lj->ijns", X, C[:, :o], optimize=True)
+    X = np.einsum("ijns,na->ijas", X, C[:, o:], optimize=True)
+    return np.einsum("ijas,sb->ijab", X, C[:, o:], optimize=True)
+
+
+@pytest.mark.parametrize("n,o", [(3, 1), (8, 7), (9, 1), (17, 15), (17, 16), (41, 16), (41, 17), (41, 31), (41, 33), (40, 39),
+                                 (57, 48), (58, 49)])
+def test_first_quarter_edges(ctx, n, o):
+    rng = np.random.default_rng(100 * n + o)
+    np_ = n * (n + 1) // 2
+    pk = rng.standard_normal(np_ * (np_ + 1) // 2)
+    tri = np.zeros((n, n), dtype=int)
+    tri[np.tril_indices(n)] = np.arange(np_)
+    tri = np.maximum(tri, tri.T)
+    I, J = tri[:, :, None, None], tri[None, None]
+    hi, lo = np.maximum(I, J), np.minimum(I, J)
+    g = pk[hi * (hi + 1) // 2 + lo]
+    C = rng.standard_normal((n, n)) / np.sqrt(n)
+    ctx.eri_load_packed(pk, n)
+    ref, scale = _ovov(g, C, o), _ovov(np.abs(g), np.abs(C), o)
+    for precision, eps in (("fp64", np.finfo(np.float64).eps), ("fp32", np.finfo(np.float32).eps), ("fp32c", np.finfo(np.float32).eps)):
+        out = ctx.ao2mo(C, o, "ovov", precision=precision)
+        assert np.all(np.abs(out - ref) <= (4 * n + 8) * eps * scale), (n, o, precision)

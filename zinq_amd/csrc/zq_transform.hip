@@ -144,17 +144,6 @@ __device__ inline E q1_val(const E *__restrict__ eri, const Q1Src &s, int K, int
   return eri[s.base + idx];
 }
 
-// Element index (within its quartet) of (mu = bmu*8+u, nu = bnu*8+w | K), branch-free.  Unlike q1_val the
-// non-canonical ket slots of a diagonal ket block are not zeroed: Q1 zeroes their outputs when it stores X.
-__device__ inline int q1_idx(const Q1Src &s, int K, int u, int w) {
-  int pl = s.swp ? w : u, ql = s.swp ? u : w;
-  const int hi = max(pl, ql), lo = min(pl, ql);
-  if (s.diagB) pl = hi, ql = lo;
-  const int bl = pl * 8 + ql;
-  const int kbl = s.Ib > s.Jb ? K * 64 + bl : bl * 64 + K;
-  return s.Ib == s.Jb ? min(K, bl) * 64 + max(K, bl) : kbl;
-}
-
 // ---------------------------------------------------------------- Q1, FP64 / FP32
 // Workgroup (256 threads) owns half kh of ket block pair Jb's 64 slots (K = 32 kh .. 32 kh + 31) x AO
 // block bnu (8 nu) x a group of 16 MT occupied orbitals.  Loop over mu blocks: stage
@@ -162,22 +151,24 @@ __device__ inline int q1_idx(const Q1Src &s, int K, int u, int w) {
 // owns the 16-column tiles 4w .. 4w+3 (K = 32 kh + 8w .. 8w+7, all 8 nu) for all MT row tiles, so each
 // LDS operand feeds MT MFMAs.
 //
-// On gfx950 the FP64 MFMAs do not co-issue with other vector ALU instructions, so the loop is written to
-// issue few of them:
+// On gfx950 the FP64 MFMAs do not co-issue with other vector ALU instructions, and every load or LDS store beside
+// them costs about as much again (each of the step's loads and stores taken out gives 20 of 1500 us at n = 192,
+// o = 40, whether or not it reaches memory), so a step issues few of them:
 // - a thread's eight staging elements of a quartet block lie at one per-thread offset plus a uniform
 //   stride, for each storage order (bra-fastest [K][bra] or ket-fastest [bra][K]) and bra orientation;
-//   the offsets are computed once, and only the diagonal forms (Ib == Jb, or a diagonal bra block stored
-//   ket-fastest) compute indices element by element;
-// - LDS stores and operand reads use immediate offsets from fixed per-thread bases;
+//   the offsets are computed once and the strides are scalar arithmetic; only the odd forms (Ib == Jb, or a
+//   diagonal bra block stored ket-fastest; at most two blocks of a workgroup) are read again, element by element;
+// - the forms of 64 blocks are worked out at once, a block a lane, and read back lane by lane;
+// - C1 is laid out so that both steps' A operands of a lane are one load (q1_c_index);
+// - LDS operand reads use immediate offsets from fixed per-thread bases;
 // - the non-canonical ket slots of a diagonal ket block are zeroed in the epilogue (X there is exactly
 //   +0, as the zeroed inputs gave).
-// Quartet blocks are fetched two mu blocks ahead and staged one ahead (double-buffered LDS, one barrier
-// per block); the C1 operands of a block are loaded one block ahead, before the quartet fetch.  Loads,
-// fetches and stages are unconditional (indices past the last block are clamped: their copies land in
-// the buffer no later step reads, and the A-operand rows past m1 load row m1 - 1, which only reaches output
-// rows that are never stored), so every path through the loop leaves the same loads in flight and the
-// compiler's memory-counter waits are exact: the MFMAs wait only for their C1 operands, a stage only for
-// its own quartet block.
+// A block is fetched and its operands are loaded while the one before is multiplied, the loads dealt out between
+// the MFMAs (1.57 ms behind one another, 1.47 so), and staged into the other LDS buffer, one barrier per
+// block.  Loads are unconditional (indices past the last block are clamped: their copies land in the buffer no
+// later step reads, and the A operands past m1 take column m1 - 1, which only reaches output rows that are never
+// stored).  n = 192, o = 40, FP64: 1607 -> 1470 us (MFMA peak of the executed tiles 940); n = 101, o = 20, FP32C:
+// 106 -> 94; a group of 96 molecules n <= 72: 636 -> 546.
 // The body takes the workgroup's coordinates (bx, by, bz) as arguments, so that a grouped launch over
 // many molecules can run it for each molecule's share of the grid.
 struct Q1Slots {
@@ -185,61 +176,68 @@ struct Q1Slots {
   int offA0, offA1, offAd, offB0, offB1;
 };
 
-// Loads this thread's eight elements of block (bm, bnu | Jb); returns true for ket-fastest slots.  Only the
-// element indices depend on the block's form, the loads are one sequence (separate load paths would make
-// the compiler merge their memory-counter states conservatively).  The slots are taken by value: a select
-// between the addresses of their fields would keep them in scratch memory.
+// Form of block (bmu, bnu | Jb): quartet index and, in .y, kQ1* bits.
+enum { kQ1Bra = 1, kQ1Ket = 2, kQ1Swap = 4, kQ1Diag = 8 };  // bra-fastest, ket-fastest (neither: Ib == Jb)
+__device__ inline uint2 q1_form(int bmu, int bnu, int br, int bs, int Jb) {
+  const Q1Src s = q1_src(bmu, bnu, br, bs, Jb);
+  return make_uint2(unsigned(s.base / ZQ_QUARTET), (s.Ib > Jb ? kQ1Bra : s.Ib < Jb ? kQ1Ket : 0) | (s.swp ? kQ1Swap : 0) |
+                                                       (s.diagB ? kQ1Diag : 0));
+}
+
+// This thread's eight elements of the block at q, element j at off + j stride (bytes; the stride is uniform).
+// Blocks whose elements do not lie like that (q1_odd) read eight elements of theirs that mean nothing.
 template <class T, class E>
-__device__ __forceinline__ bool q1_fetch(const E *__restrict__ eri, const Q1Src src, const Q1Slots sl, int K0,
-                                         T (&v)[8]) {
-  const E *q = eri + src.base;
-  const bool bra = src.Ib > src.Jb, ket = src.Ib < src.Jb;
-  int idx[8];
-  if (bra || (ket && !src.diagB)) {
-    const int offA = sl.offA0 + (src.swp ? sl.offA1 - sl.offA0 : 0) + (src.diagB ? sl.offAd - sl.offA0 : 0);
-    const int offK = src.swp ? sl.offB1 + 0 : sl.offB0 + 0;
-    const int off = bra ? offA : offK;
-    const int stride = bra ? 256 : (src.swp ? 64 : 512);
+__device__ __forceinline__ void q1_fetch(const E *__restrict__ q, unsigned form, const Q1Slots sl, T (&v)[8]) {
+  const bool bra = form & kQ1Bra, swp = form & kQ1Swap;
+  const int offA = form & kQ1Diag ? sl.offAd + 0 : (swp ? sl.offA1 + 0 : sl.offA0 + 0);
+  const int offK = swp ? sl.offB1 + 0 : sl.offB0 + 0;
+  const unsigned off = unsigned(bra ? offA : offK) * unsigned(sizeof(E));
+  const int stride = (bra ? 256 : (swp ? 64 : 512)) * int(sizeof(E));
 #pragma unroll
-    for (int j = 0; j < 8; ++j) idx[j] = off + stride * j;
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int kl = ket ? sl.kB + 0 : sl.kA + 4 * j, u = ket ? j : sl.uA + 0, w = ket ? sl.wB + 0 : sl.wA + 0;
-      idx[j] = q1_idx(src, K0 + kl, u, w);
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = T(q[idx[j]]);
-  return ket;
+  for (int j = 0; j < 8; ++j) v[j] = T(*reinterpret_cast<const E *>(reinterpret_cast<const char *>(q) + j * stride + off));
 }
 
-// T[kl][u*8+w] of the staged block: bra-fastest slots at lA + 4 rows per j, ket-fastest at lB + 8 per j.
-template <class T>
-__device__ __forceinline__ void q1_stage(T *lA, T *lB, const T (&v)[8], bool ket) {
-  if (ket) {
+// A diagonal bra block stored ket-fastest, and Ib == Jb, where the smaller of the two pairs is the row.
+__device__ inline bool q1_odd(unsigned form) {
+  return (form & (kQ1Ket | kQ1Diag)) == (kQ1Ket | kQ1Diag) || !(form & (kQ1Bra | kQ1Ket));
+}
+template <class T, class E>
+__device__ __forceinline__ void q1_fetch_odd(const E *__restrict__ q, unsigned form, const Q1Slots sl, int K0, T (&v)[8]) {
+  const bool ket = form & kQ1Ket, swp = form & kQ1Swap, diag = form & kQ1Diag;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) lB[8 * j] = v[j];
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) lA[4 * 65 * j] = v[j];
+  for (int j = 0; j < 8; ++j) {
+    const int K = K0 + (ket ? sl.kB + 0 : sl.kA + 4 * j), u = ket ? j : sl.uA + 0, w = ket ? sl.wB + 0 : sl.wA + 0;
+    const int pl = swp ? w : u, ql = swp ? u : w, hi = diag ? max(pl, ql) : pl, lo = diag ? min(pl, ql) : ql;
+    const int bl = hi * 8 + lo, row = ket ? bl : min(K, bl), col = ket ? K : max(K, bl);
+    v[j] = T(q[row * 64 + col]);
   }
 }
 
-// A operands of one mu block: C1[8 bm + 4 ks + (lane >> 4)][i0 + 16 h + (lane & 15)], cb at the block's row
-// and coff[h] the (clamped) column of row tile h.
+// Where C1[mu][i] lies: each mu block's 8 m1 values by tile of 16 i, there the two values of MFMA lane
+// (mu & 3, i & 15) side by side, so that a lane fetches both steps' operands in one load.  The last tile holds
+// its m1 mod 16 columns only, so C1 takes np m1 elements as a plain matrix would.
+__host__ __device__ inline size_t q1_c_index(int mu, int i, int m1) {
+  const int tile = i >> 4, w = m1 - 16 * tile < 16 ? m1 - 16 * tile : 16;
+  return size_t(mu >> 3) * 8 * m1 + 128 * tile + ((mu & 3) * w + (i & 15)) * 2 + ((mu >> 2) & 1);
+}
+
+// A operands of one mu block: C1[8 bm + 4 ks + (lane >> 4)][i0 + 16 h + (lane & 15)], cb at the block
+// (uniform) and coff[h] the lane's byte offset in row tile h (columns past m1 take the last one).
 template <class T, int MT>
-__device__ __forceinline__ void q1_load_c(const T *__restrict__ cb, size_t ldc1, const int (&coff)[MT], T (&cv)[2][MT]) {
+__device__ __forceinline__ void q1_load_c(const T *cb, const unsigned (&coff)[MT], T (&cv)[MT][2]) {
+  typedef T T2 __attribute__((ext_vector_type(2)));
+  const char *q = reinterpret_cast<const char *>(cb);
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-    for (int h = 0; h < MT; ++h) cv[ks][h] = cb[ks * 4 * ldc1 + coff[h]];
+  for (int h = 0; h < MT; ++h) {
+    const T2 v = *reinterpret_cast<const T2 *>(q + coff[h]);
+    cv[h][0] = v.x, cv[h][1] = v.y;
+  }
 }
 
 // The block's MFMAs: B operand of column tile c is T[8w + 2c + ((lane >> 3) & 1)][(4 ks + (lane >> 4)) * 8
 // + (lane & 7)], read from lR + 130 c + 32 ks.
 template <class MF, int MT>
-__device__ __forceinline__ void q1_mfmas(const typename MF::T *lR, const typename MF::T (&cv)[2][MT],
+__device__ __forceinline__ void q1_mfmas(const typename MF::T *lR, const typename MF::T (&cv)[MT][2],
                                          typename MF::acc (&acc)[MT][4]) {
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks)
@@ -247,7 +245,7 @@ __device__ __forceinline__ void q1_mfmas(const typename MF::T *lR, const typenam
     for (int c = 0; c < 4; ++c) {
       const typename MF::T b = lR[2 * c * 65 + 32 * ks];
 #pragma unroll
-      for (int h = 0; h < MT; ++h) acc[h][c] = MF::mma(cv[ks][h], b, acc[h][c]);
+      for (int h = 0; h < MT; ++h) acc[h][c] = MF::mma(cv[h][ks], b, acc[h][c]);
     }
 #pragma unroll
   for (int h = 0; h < MT; ++h)
@@ -256,7 +254,7 @@ __device__ __forceinline__ void q1_mfmas(const typename MF::T *lR, const typenam
 }
 
 template <class MF, int MT, class E>
-__device__ __forceinline__ void q1_body(const E *__restrict__ eri, const typename MF::T *__restrict__ C1, int ldc1,
+__device__ __forceinline__ void q1_body(const E *__restrict__ eri, const typename MF::T *__restrict__ C1,
                                         int m1, int nb, int npad, typename MF::T *__restrict__ X, int bx, int by,
                                         int bz) {
   typedef typename MF::T T;
@@ -284,36 +282,65 @@ __device__ __forceinline__ void q1_body(const E *__restrict__ eri, const typenam
   sl.offAd = (K0 + sl.kA) * 64 + max(sl.uA, sl.wA) * 8 + min(sl.uA, sl.wA);
   sl.offB0 = sl.wB * 64 + K0 + sl.kB;
   sl.offB1 = sl.wB * 512 + K0 + sl.kB;
-  T *const lA0 = &Ts[0][sl.kA][tid & 63], *const lA1 = &Ts[1][sl.kA][tid & 63];
-  T *const lB0 = &Ts[0][sl.kB][sl.wB], *const lB1 = &Ts[1][sl.kB][sl.wB];
-  const T *const lR0 = &Ts[0][8 * wave + ((lane >> 3) & 1)][(lane >> 4) * 8 + (lane & 7)];
-  const T *const lR1 = &Ts[1][8 * wave + ((lane >> 3) & 1)][(lane >> 4) * 8 + (lane & 7)];
-  const T *const cbase = C1 + size_t(lane >> 4) * ldc1;
-  const size_t ldc = size_t(ldc1);
-  int coff[MT];
+  // T[kl][u*8+w] of a staged block: bra-fastest elements at lA + 4 rows per j, ket-fastest at lB + 8 per j
+  T *const lA = &Ts[0][sl.kA][tid & 63], *const lB = &Ts[0][sl.kB][sl.wB];
+  const T *const lR = &Ts[0][8 * wave + ((lane >> 3) & 1)][(lane >> 4) * 8 + (lane & 7)];
+  constexpr int kBuf = 32 * 65;
+  unsigned coff[MT];
 #pragma unroll
-  for (int h = 0; h < MT; ++h) coff[h] = min(i0 + 16 * h + (lane & 15), m1 - 1);
+  for (int h = 0; h < MT; ++h)
+    coff[h] = unsigned(q1_c_index(lane >> 4, min(i0 + 16 * h + (lane & 15), m1 - 1), m1)) * unsigned(sizeof(T));
 
-  T ca[2][MT], cb[2][MT], ra[8], rb[8];
+  T ca[MT][2], cb[MT][2], r[8];
   const int last = nb - 1;
-  q1_load_c<T, MT>(cbase, ldc, coff, ca);
-  q1_stage(lA0, lB0, ra, q1_fetch<T, E>(eri, q1_src(0, bnu, br, bs, Jb), sl, K0, ra));
-  bool kb = q1_fetch<T, E>(eri, q1_src(min(1, last), bnu, br, bs, Jb), sl, K0, rb);
+  // lane l holds the form of block (64 g + l, bnu | Jb), g the group of 64 blocks the fetches have reached
+  uint2 forms = make_uint2(0u, 0u);
+  auto form_of = [&](int bm) {
+    if ((bm & 63) == 0) forms = q1_form(min(bm + lane, last), bnu, br, bs, Jb);
+    return make_uint2(unsigned(__builtin_amdgcn_readlane(int(forms.x), bm & 63)),
+                      unsigned(__builtin_amdgcn_readlane(int(forms.y), bm & 63)));
+  };
+  auto stage = [&](int buf, unsigned form) {
+    const bool ket = (form & kQ1Ket) != 0;
+    T *const l = (ket ? lB : lA) + buf * kBuf;
+    const int st = ket ? 8 : 4 * 65;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) l[j * st] = r[j];
+  };
+  // one step: block bm from buffer buf with cv, while block bm + 1 is on its way (operands into cn, elements through
+  // r into the other buffer).  One basic block up to the rare odd forms, in which the loads are dealt out
+  // between the MFMAs.
+  auto step = [&](int bm, int buf, const T(&cv)[MT][2], T(&cn)[MT][2]) {
+    const int next = min(bm + 1, last);
+    const uint2 f = form_of(next);
+    const E *q = eri + size_t(f.x) * ZQ_QUARTET;
+    q1_load_c<T, MT>(C1 + size_t(next) * 8 * m1, coff, cn);
+    q1_fetch<T, E>(q, f.y, sl, r);
+    q1_mfmas<MF, MT>(lR + buf * kBuf, cv, acc);
+    // operand reads first, then a load behind each of the first MFMAs
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int j = 0; j < 8 + MT; ++j) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    }
+    if (q1_odd(f.y)) q1_fetch_odd<T, E>(q, f.y, sl, K0, r);
+    stage(buf ^ 1, f.y);
+    __syncthreads();
+  };
+  const uint2 f0 = form_of(0);
+  const E *q0 = eri + size_t(f0.x) * ZQ_QUARTET;
+  q1_load_c<T, MT>(C1, coff, ca);
+  q1_fetch<T, E>(q0, f0.y, sl, r);
+  if (q1_odd(f0.y)) q1_fetch_odd<T, E>(q0, f0.y, sl, K0, r);
+  stage(0, f0.y);
   __syncthreads();
-  for (int bm = 0; bm < nb; bm += 2) {
-    // block bm from buffer 0 with ca; fetch bm + 2 into ra; stage bm + 1 (rb) into buffer 1
-    q1_load_c<T, MT>(cbase + size_t(min(bm + 1, last)) * 8 * ldc, ldc, coff, cb);
-    const bool ka = q1_fetch<T, E>(eri, q1_src(min(bm + 2, last), bnu, br, bs, Jb), sl, K0, ra);
-    q1_mfmas<MF, MT>(lR0, ca, acc);
-    q1_stage(lA1, lB1, rb, kb);
-    __syncthreads();
-    // block bm + 1 from buffer 1 with cb; fetch bm + 3 into rb; stage bm + 2 (ra) into buffer 0
-    q1_load_c<T, MT>(cbase + size_t(min(bm + 2, last)) * 8 * ldc, ldc, coff, ca);
-    kb = q1_fetch<T, E>(eri, q1_src(min(bm + 3, last), bnu, br, bs, Jb), sl, K0, rb);
-    if (bm + 1 < nb) q1_mfmas<MF, MT>(lR1, cb, acc);
-    q1_stage(lA0, lB0, ra, ka);
-    __syncthreads();
+  int bm = 0;
+  for (; bm + 1 < nb; bm += 2) {
+    step(bm, 0, ca, cb);
+    step(bm + 1, 1, cb, ca);
   }
+  if (bm < nb) q1_mfmas<MF, MT>(lR, ca, acc);
   const bool diagK = br == bs;
 #pragma unroll
   for (int h = 0; h < MT; ++h)
@@ -330,17 +357,20 @@ __device__ __forceinline__ void q1_body(const E *__restrict__ eri, const typenam
     }
 }
 
-// Two workgroups per CU (the accumulators then sit in the architectural VGPRs), unless the accumulators
+// Waves per SIMD asked for: two (the accumulators then sit in the architectural VGPRs), unless the accumulators
 // alone take more than 144 of a wave's registers (FP32 products with FP64 sums at MT = 4), which would spill.
+// Three for FP64 at MT = 3: 1.47 ms against 1.50 at n = 192, o = 40, although a few registers spill; FP32C at
+// MT = 2 loses by it (103 us against 94 at n = 101, o = 20).
 template <class MF, int MT>
 constexpr int q1_min_waves() {
-  return MT * 4 * MF::kAccRegs <= 144 ? 2 : 1;
+  constexpr int regs = MT * 4 * MF::kAccRegs;
+  return sizeof(typename MF::T) == 8 && regs <= 96 ? 3 : regs <= 144 ? 2 : 1;
 }
 
 template <class MF, int MT, class E>
 __global__ __launch_bounds__(256, (q1_min_waves<MF, MT>())) void zq_q1(const E *__restrict__ eri, const typename MF::T *__restrict__ C1,
-                                                int ldc1, int m1, int nb, int npad, typename MF::T *__restrict__ X) {
-  q1_body<MF, MT, E>(eri, C1, ldc1, m1, nb, npad, X, blockIdx.x, blockIdx.y, blockIdx.z);
+                                                int m1, int nb, int npad, typename MF::T *__restrict__ X) {
+  q1_body<MF, MT, E>(eri, C1, m1, nb, npad, X, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // ---------------------------------------------------------------- Q1, BF16X3
@@ -936,7 +966,7 @@ __device__ __forceinline__ void c_slices_body(const double *__restrict__ C, int 
                                               int mu) {
   for (int t = threadIdx.x; t < m1 + m2 + m3; t += blockDim.x) {
     if (t < m1) {
-      c1[size_t(mu) * m1 + t] = mu < n ? T(C[size_t(mu) * n + t]) : T(0);
+      c1[q1_c_index(mu, t, m1)] = mu < n ? T(C[size_t(mu) * n + t]) : T(0);
     } else if (t < m1 + m2) {
       const int j = t - m1;
       c2t[size_t(j) * np + mu] = mu < n ? T(C[size_t(mu) * n + j]) : T(0);
@@ -1066,7 +1096,7 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     std::vector<T> h1(size_t(np) * m1, T(0)), h2t(size_t(m2) * np, T(0)), h3(size_t(np) * m3, T(0)),
         h4(own4 ? size_t(np) * m4 : 0, T(0));
     for (int mu = 0; mu < n; ++mu) {
-      for (int i = 0; i < m1; ++i) h1[size_t(mu) * m1 + i] = T(cf.q[0][size_t(mu) * n + i]);
+      for (int i = 0; i < m1; ++i) h1[q1_c_index(mu, i, m1)] = T(cf.q[0][size_t(mu) * n + i]);
       for (int j = 0; j < m2; ++j) h2t[size_t(j) * np + mu] = T(cf.q[1][size_t(mu) * n + j]);
       for (int a = 0; a < m3; ++a) h3[size_t(mu) * m3 + a] = T(cf.q[2][size_t(mu) * n + d.off3 + a]);
       if (own4)
@@ -1127,18 +1157,18 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
         // FP32 forms: read the FP32 copy of the quartets (the same rounding as converting on the fly)
         const float *e32 = ctx->eri32;
         switch (mt) {
-          case 1: hipLaunchKernelGGL((zq_q1<MF, 1, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, m1, nb, np, X); break;
-          case 2: hipLaunchKernelGGL((zq_q1<MF, 2, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, m1, nb, np, X); break;
-          case 3: hipLaunchKernelGGL((zq_q1<MF, 3, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, m1, nb, np, X); break;
-          default: hipLaunchKernelGGL((zq_q1<MF, 4, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, m1, nb, np, X); break;
+          case 1: hipLaunchKernelGGL((zq_q1<MF, 1, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, nb, np, X); break;
+          case 2: hipLaunchKernelGGL((zq_q1<MF, 2, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, nb, np, X); break;
+          case 3: hipLaunchKernelGGL((zq_q1<MF, 3, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, nb, np, X); break;
+          default: hipLaunchKernelGGL((zq_q1<MF, 4, float>), grid2, dim3(256), 0, ctx->stream, e32, d1, m1, nb, np, X); break;
         }
       } else {
         const double *e64 = ctx->eri;
         switch (mt) {
-          case 1: hipLaunchKernelGGL((zq_q1<MF, 1, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, m1, nb, np, X); break;
-          case 2: hipLaunchKernelGGL((zq_q1<MF, 2, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, m1, nb, np, X); break;
-          case 3: hipLaunchKernelGGL((zq_q1<MF, 3, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, m1, nb, np, X); break;
-          default: hipLaunchKernelGGL((zq_q1<MF, 4, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, m1, nb, np, X); break;
+          case 1: hipLaunchKernelGGL((zq_q1<MF, 1, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, nb, np, X); break;
+          case 2: hipLaunchKernelGGL((zq_q1<MF, 2, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, nb, np, X); break;
+          case 3: hipLaunchKernelGGL((zq_q1<MF, 3, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, nb, np, X); break;
+          default: hipLaunchKernelGGL((zq_q1<MF, 4, double>), grid2, dim3(256), 0, ctx->stream, e64, d1, m1, nb, np, X); break;
         }
       }
     }
@@ -1400,7 +1430,7 @@ __global__ __launch_bounds__(256, (q1_min_waves<MF, 1>())) void zq_group_q1(cons
   const int m = group_find(start, nmol, blockIdx.x);
   const GJob<typename MF::T, E> J = jobs[m];
   const int l = int(blockIdx.x) - start[m], gx = J.Nb * J.nb, t = l / gx;
-  q1_body<MF, 1, E>(J.eri, J.c1, J.o, J.o, J.nb, J.np, J.X, l - t * gx, t % J.groups, t / J.groups);
+  q1_body<MF, 1, E>(J.eri, J.c1, J.o, J.nb, J.np, J.X, l - t * gx, t % J.groups, t / J.groups);
 }
 
 template <class MF, class E>
