@@ -366,8 +366,10 @@ zq_ctx *zq_create(int device) {
   if (hipGetDeviceCount(&count) != hipSuccess || device < 0 || device >= count) return nullptr;
   if (hipSetDevice(device) != hipSuccess) return nullptr;
   zq_noalloc_setup(device);
+  static std::atomic<unsigned> turns{0};
   auto *ctx = new zq_ctx;
   ctx->device = device;
+  ctx->turn = turns.fetch_add(1);
   if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
     delete ctx;
     return nullptr;

@@ -20,11 +20,10 @@
 //   eigenvalue's distance at least once, and the iteration stops.
 //   X symmetric, so only tiles ti <= tj are computed and mirrored; the epilogue applies the branch and
 //   writes per-tile partial traces (tr X, ||X||_F^2 = tr X^2), which every workgroup of the next step
-//   sums in the same fixed order, so all of them take the same branch.  X is ping-ponged between two
-//   buffers (input [p], output [p^1]).
-//   Two forms, bitwise equal on plain runs: k_sp2_run takes every step in one launch (tiles handed out
-//   by ticket, a step's tiles counted before the next reads X), which the device SCF uses; k_sp2_step
-//   is one launch per step, used by the host-checked driver.
+//   sums in the same fixed order, so all of them take the same branch.
+//   Three forms, bitwise equal on plain runs: k_sp2_home and k_sp2_run take every step in one launch (tiles
+//   handed out by ticket), on one XCD and on all of them, which the device SCF uses; k_sp2_step is one launch per
+//   step, used by the host-checked driver.  k_sp2_run and k_sp2_step ping-pong X between two buffers.
 //
 // Certified scale-and-fold steps (one-launch form in the device SCF).  With bounds a_k >= every
 // virtual eigenvalue of X_k and b_k <= every occupied one (a_k < b_k), the down step may fold at
@@ -51,6 +50,12 @@ namespace {
 
 using namespace zqt;
 using namespace zqs;
+
+// The one-launch form's counters: a ticket and a finished count per step; on one XCD the first is the only
+// ticket and the word past them all is the XCD's number + 1.
+constexpr int kSp2Home = 2 * kSp2MaxSteps, kSp2Sync = kSp2Home + 1;
+constexpr int kXccId = 20 | (31 << 11);                    // s_getreg of HW_REG_XCC_ID, all bits
+constexpr unsigned long long kSp2Unset = ~0ull;            // a partial trace not yet written (no sum gives these bits)
 
 template <bool VEC>
 __global__ __launch_bounds__(64) void k_gemm_nt(const double *__restrict__ A, int lda, const double *__restrict__ B,
@@ -171,7 +176,9 @@ __global__ __launch_bounds__(256) void k_gershgorin(const double *__restrict__ F
   }
 }
 
-// Writes the partial traces of the tile this wave holds (vals[j] at rows i0+4j+q, column j0+r).
+// Writes the partial traces of the tile this wave holds (vals[j] at rows i0+4j+q, column j0+r).  DRAIN: once the
+// wave's stores before are in the L2, as the partials tell readers on the XCD that the tile is there.
+template <bool DRAIN = false>
 __device__ inline void tile_partials(const double v[4], int ti, int tj, int i0, int j0, double2 *__restrict__ part, int t) {
   const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
   double s1 = 0.0, s2 = 0.0;
@@ -182,6 +189,7 @@ __device__ inline void tile_partials(const double v[4], int ti, int tj, int i0, 
   }
   s1 = wave_sum(s1);
   s2 = wave_sum(s2);
+  if (DRAIN) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (lane == 0) part[t] = make_double2(s1, ti == tj ? s2 : 2.0 * s2);
 }
 
@@ -208,8 +216,10 @@ __global__ __launch_bounds__(64) void k_sp2_init(const double *__restrict__ F, i
     if (ti != tj) X[size_t(col) * m + row] = x;
   }
   tile_partials(v, ti, tj, i0, j0, part, blockIdx.x);
+  const double unset = __longlong_as_double((long long)kSp2Unset);
+  for (int k = 1 + lane; k <= kSp2MaxSteps; k += 64) part[size_t(k) * gridDim.x + blockIdx.x] = make_double2(unset, unset);
   if (blockIdx.x == 0) {
-    for (int u = lane; u < 2 * kSp2MaxSteps; u += 64) sync[u] = 0u;
+    for (int u = lane; u < kSp2Sync; u += 64) sync[u] = 0u;
     if (lane == 0) state[0] = -1, state[1] = 0, state[4] = 0, state[5] = 0;
   }
 }
@@ -253,19 +263,22 @@ __device__ inline void sp2_load(Sp2Ops<PRE> &o, const double *__restrict__ Xin, 
 // X_out tile = alpha X_in^2 + beta X_in + gamma I, stored with its mirror, and its partial traces in
 // pout[t].  Every wave of the workgroup calls it; PRE sums the waves' partial products in LDS, in wave
 // order, and wave 0 finishes the tile.
-template <bool PRE>
+// ready(): called between the waves' products and the barrier that hands them to wave 0.
+template <bool PRE, bool HOME = false, class R>
 __device__ inline void sp2_finish(const Sp2Ops<PRE> &o, const double *__restrict__ Xin, double *__restrict__ Xout, int m,
-                                  int ti, int tj, const Sp2Map &p, double2 *__restrict__ pout, int t) {
+                                  int ti, int tj, const Sp2Map &p, double2 *__restrict__ pout, int t, int buf, R &&ready) {
   const int i0 = ti * 16, j0 = tj * 16, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4, w = threadIdx.x >> 6;
   d4 acc = {0.0, 0.0, 0.0, 0.0};
   if (PRE) {
-    __shared__ d4 red[3][64];
+    __shared__ d4 reds[HOME ? 2 : 1][3][64];
+    d4(*const red)[64] = reds[HOME ? buf : 0];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (16 * (w + 4 * i) < m)
 #pragma unroll
         for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(o.f.a[i][u], o.f.b[i][u], acc, 0, 0, 0);
     if (w > 0) red[w - 1][lane] = acc;
+    ready();
     __syncthreads();
     if (w == 0) {
       acc += red[0][lane];
@@ -284,12 +297,22 @@ __device__ inline void sp2_finish(const Sp2Ops<PRE> &o, const double *__restrict
     if (i0 + 4 * j + q == j0 + r) v[j] += p.gamma;
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = i0 + 4 * j + q, col = j0 + r;
-    Xout[size_t(row) * m + col] = v[j];
-    if (ti != tj) Xout[size_t(col) * m + row] = v[j];
+  for (int j = 0; j < 4; ++j) Xout[size_t(i0 + 4 * j + q) * m + j0 + r] = v[j];
+  if (ti != tj) {
+    if (PRE) {  // the mirror turned in LDS, so that it leaves in whole row segments too
+      __shared__ double turn[16][17];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) turn[r][4 * j + q] = v[j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 4; ++j) Xout[size_t(j0 + 4 * j + q) * m + i0 + r] = turn[4 * j + q][r];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) Xout[size_t(j0 + r) * m + i0 + 4 * j + q] = v[j];
+    }
   }
-  tile_partials(v, ti, tj, i0, j0, pout, t);
+  tile_partials<HOME>(v, ti, tj, i0, j0, pout, t);
 }
 
 __device__ inline void sum_partials(const double2 *__restrict__ pin, int ntiles, double &t1, double &t2) {
@@ -327,14 +350,143 @@ __global__ __launch_bounds__(sp2_threads(PRE)) void k_sp2_step(const double *__r
     sout[0] = count, sout[1] = steps + 1;
     if (count == 2) *final = pout_parity;  // X_out is the settled projector
   }
-  sp2_finish<PRE>(o, Xin, Xout, m, ti, tj, mp, pout, blockIdx.x);
+  sp2_finish<PRE>(o, Xin, Xout, m, ti, tj, mp, pout, blockIdx.x, 0, [] {});
+}
+
+__device__ inline double load_past_l1(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Bounded waits of the one-launch SP2: a wait that runs out raises *abort, and so makes the launch's
 // result count as unsettled; a wait that sees *abort raised gives up too.
 constexpr unsigned kSpinLimit = 1u << 22;
 
-// Tiles per workgroup and step of the one-launch SP2 (the grid is ceil(tiles / kSp2TilesPerGroup)).
+// Largest m of the one-XCD form.  Both forms, us per run of about 27 steps (one XCD / all): n = 72 51 / 84, 96 56 / 86,
+// 128 83 / 98, 144 96 / 113, 160 99 / 120, 176 133 / 137, 192 146 / 146, 224 227 / 170: past 64 tiles a compute
+// unit of the XCD has three.
+constexpr int kSp2HomeMax = 160;
+
+// Every step of SP2 in one launch, m <= kSp2HomeMax: on the compute units of one XCD, which share an L2, so a step is
+// handed over without the write-back and the invalidation of the L2s that fences between XCDs cost.  Eight times
+// the workgroups are launched, one in eight takes part (consecutive ones go to the XCDs in turn), and the first
+// of these to arrive makes its XCD the run's home and keeps its records; those that find themselves elsewhere
+// leave; contexts take their turn of eight, so that runs at the same time have homes of their own.  The number that
+// stays only bounds the speed: tiles of all steps are numbered through and handed out by
+// one ticket, drawn while the tile before is computed.
+// A tile's partial traces tell that it is there: wave 0, which alone writes tiles, stores them after its other
+// stores have drained to the L2, and a workgroup that needs X_k polls for all partials of X_k, which it has to sum
+// anyway, past its L1.  Every step writes an X of its own, which no compute unit has read before in the launch, so
+// the tiles are read through the L1s without a stale line.  A wait only ever depends on tiles that running
+// workgroups have taken, so the launch finishes whichever of its workgroups are resident.
+// Partials are kept per step, so a workgroup that takes no tile of a step replays the branch and stop decisions
+// from them; every workgroup sums them in the same order and so takes the same decisions.  Each tile is computed
+// as by k_sp2_step, so the result is bitwise that of the step-per-launch form.  state gets {count, steps} in
+// the pair 2 * (nsteps & 1), as k_sp2_step leaves them, and the settled X's index in [4]; [5] is the abort flag.
+// Bound by a step's serial chain: poll, operands from the L2, MFMAs, sums, drain (2.1 us at n = 96, 3.6 at 144).
+__global__ __launch_bounds__(256) void k_sp2_home(double *__restrict__ X, size_t mm, int m, int nocc,
+                                                double2 *__restrict__ part, unsigned *__restrict__ sync,
+                                                int *__restrict__ state, int nsteps, double tol,
+                                                const int *__restrict__ skip, double *__restrict__ est, unsigned turn) {
+  if (skip && *skip) return;
+  if ((blockIdx.x & 7) != turn) return;
+  __shared__ unsigned s_home, s_ticket[2];
+  __shared__ double s_sum[2][2];
+  __shared__ int s_ok[2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) {
+    const unsigned me = 1u + (__builtin_amdgcn_s_getreg(kXccId) & 15u);
+    unsigned at = 0;
+    s_home = __hip_atomic_compare_exchange_strong(&sync[kSp2Home], &at, me, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                 ? 2u
+                 : unsigned(at == me);
+    if (s_home) s_ticket[0] = __hip_atomic_fetch_add(&sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (s_home == 0) return;
+  const bool keeper = s_home == 2;
+  const int T = m / 16, ntiles = T * (T + 1) / 2;
+  // folding bounds, carried identically by every wave; the history is the keeper's
+  bool fold = false;
+  double fa = 0.0, fb = 1.0;
+  if (est && est[kEstFold] != 0.0) fold = true, fa = est[kEstA0], fb = est[kEstB0];
+  double *hist = (est && keeper && threadIdx.x == 0) ? est + kEstHist : nullptr;
+  int *abort = state + 5;
+  int count = -1, steps = 0, fin = 0, slot = 0;
+  unsigned t = s_ticket[0];
+  for (int k = 0; k < nsteps; ++k) {
+    const double *Xin = X + k * mm;
+    double *Xout = X + (k + 1) * mm;
+    if (wave == 0) {
+      const double2 *p = part + size_t(k) * ntiles;
+      bool ok = true;
+      double t1 = 0.0, t2 = 0.0;
+      for (unsigned spins = 0;;) {
+        bool all = true;
+        t1 = t2 = 0.0;
+        for (int u = lane; u < ntiles; u += 64) {
+          const double2 v = make_double2(load_past_l1(&p[u].x), load_past_l1(&p[u].y));
+          all = all && (unsigned long long)(__double_as_longlong(v.x)) != kSp2Unset &&
+                (unsigned long long)(__double_as_longlong(v.y)) != kSp2Unset;
+          t1 += v.x, t2 += v.y;
+        }
+        if (__all(all)) break;
+        if ((spins & 63) == 63 && __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+          ok = false;
+          break;
+        }
+        if (++spins > kSpinLimit / 8) {  // a poll here is a round trip past the L1
+          __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ok = false;
+          break;
+        }
+      }
+      t1 = wave_sum(t1);
+      t2 = wave_sum(t2);
+      if (lane == 0) s_sum[k & 1][0] = t1, s_sum[k & 1][1] = t2, s_ok[k & 1] = ok;
+    }
+    __syncthreads();
+    if (!s_ok[k & 1]) break;
+    // the operands of the tile already taken are loaded before the branch is worked out
+    Sp2Ops<true> o;
+    int ti = 0, tj = 0;
+    const unsigned end = unsigned(k + 1) * unsigned(ntiles);
+    if (t < end) {
+      tile_of(int(t - unsigned(k) * unsigned(ntiles)), T, ti, tj);
+      sp2_load<true>(o, Xin, m, ti * 16, tj * 16);
+    }
+    const double t1 = s_sum[k & 1][0], t2 = s_sum[k & 1][1];
+    const Sp2Map mp = sp2_map(t1, t2, tol, nocc, count, fold, fa, fb);
+    if (hist) hist[4 * k] = t1, hist[4 * k + 1] = t2, hist[4 * k + 2] = mp.down ? 1.0 : 0.0, hist[4 * k + 3] = mp.s;
+    steps = k + 1;
+    if (count == 2) fin = k + 1;
+    double2 *pout = part + size_t(k + 1) * ntiles;
+    while (t < end) {
+      unsigned next = 0;
+      if (threadIdx.x == 0) next = __hip_atomic_fetch_add(&sync[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      slot ^= 1;
+      sp2_finish<true, true>(o, Xin, Xout, m, ti, tj, mp, pout, int(t - unsigned(k) * unsigned(ntiles)), slot, [&] {
+        if (threadIdx.x == 0) s_ticket[slot] = next;
+      });
+      t = s_ticket[slot];
+      if (t < end) {
+        tile_of(int(t - unsigned(k) * unsigned(ntiles)), T, ti, tj);
+        sp2_load<true>(o, Xin, m, ti * 16, tj * 16);
+      }
+    }
+    if (count >= 2 || k + 1 == nsteps) break;  // the launch's end publishes the last step
+  }
+  if (keeper && threadIdx.x == 0) {
+    int *pair = state + 2 * (nsteps & 1);
+    pair[0] = count, pair[1] = steps;
+    state[4] = fin;
+    if (est) est[kEstSteps] = steps, est[kEstSettled] = count >= 2 ? 1.0 : 0.0, est[kEstStepSum] += steps;
+  }
+}
+
+// The same on all XCDs, for the larger m.
+
+// Tiles per workgroup and step (the grid is ceil(tiles / kSp2TilesPerGroup)).
 constexpr int kSp2TilesPerGroup = 1;
 
 // With several waves a workgroup (NW > 1) takes its tiles through wave 0: lane 0 of wave 0 draws the
@@ -396,7 +548,7 @@ __device__ inline bool wait_done(const unsigned *done, unsigned target, int *abo
   return ok;
 }
 
-// Every step of SP2 in one launch.  The tiles of step k are handed out by the ticket counter sync[k];
+// The tiles of step k are handed out by the ticket counter sync[k];
 // a workgroup takes tiles until none is left, counts each finished one in sync[kSp2MaxSteps + k], and
 // waits for all of step k before it reads X_(k+1).  A wait only ever depends on tiles that running
 // workgroups have taken, so the launch finishes whichever of its workgroups are resident.  Partials are
@@ -441,7 +593,7 @@ __global__ __launch_bounds__(sp2_threads(PRE)) void k_sp2_run(double *__restrict
     double2 *pout = part + size_t(k + 1) * ntiles;
     unsigned mine = 0;
     while (t < unsigned(ntiles)) {
-      sp2_finish<PRE>(o, Xin, Xout, m, ti, tj, mp, pout, int(t));
+      sp2_finish<PRE>(o, Xin, Xout, m, ti, tj, mp, pout, int(t), 0, [] {});
       ++mine;
       t = claim<NW>(&ticket[k], slot);
       if (t < unsigned(ntiles)) {
@@ -485,8 +637,9 @@ int zq_gemm_nt(zq_ctx *ctx, const double *A, int lda, const double *B, int ldb, 
 
 namespace {
 
-// X: two m x m buffers; part: the partials of X_0 .. X_kSp2MaxSteps (ntiles each; the step-per-launch
-// form ping-pongs between the first two); sync: the tickets and finished counts of the one-launch form.
+// X: two m x m buffers (nx for the one-XCD form: an X per step); part: the partials of X_0 .. X_kSp2MaxSteps
+// (ntiles each; the step-per-launch form ping-pongs between the first two); sync: the counters of the one-launch
+// forms.
 struct Sp2Bufs {
   int m, T, ntiles;
   size_t mm;
@@ -495,13 +648,13 @@ struct Sp2Bufs {
   unsigned *sync, *gcount;
 };
 
-int sp2_bufs(zq_ctx *ctx, int n, Sp2Bufs &b) {
+int sp2_bufs(zq_ctx *ctx, int n, int nx, Sp2Bufs &b) {
   b.m = (n + 15) / 16 * 16, b.T = b.m / 16, b.ntiles = b.T * (b.T + 1) / 2;
   b.mm = size_t(b.m) * b.m;
-  b.X = (double *)zq_scratch(ctx, "sp2_X", 2 * b.mm * sizeof(double));
+  b.X = (double *)zq_scratch(ctx, "sp2_X", size_t(nx) * b.mm * sizeof(double));
   b.part = (double2 *)zq_scratch(ctx, "sp2_part", size_t(kSp2MaxSteps + 1) * b.ntiles * sizeof(double2));
   b.scal = (double *)zq_scratch(ctx, "sp2_scal", 2 * sizeof(double));
-  b.sync = (unsigned *)zq_scratch(ctx, "sp2_sync", 2 * kSp2MaxSteps * sizeof(unsigned));
+  b.sync = (unsigned *)zq_scratch(ctx, "sp2_sync", kSp2Sync * sizeof(unsigned));
   b.est = zq_sp2_est(ctx);
   b.ref = (double *)zq_scratch(ctx, "sp2_ref", 2 * size_t(n) * n * sizeof(double));
   b.gpart = (double *)zq_scratch(ctx, "sp2_gpart", 4 * kGershBlocks * sizeof(double));
@@ -542,14 +695,17 @@ int zq_sp2_enqueue(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, i
   if (nsteps < 1 || nsteps > kSp2MaxSteps) return zq_fail(ctx, ZQ_ERR_INVALID, "SP2 step budget out of range");
   if (track < 0 || track > 2) return zq_fail(ctx, ZQ_ERR_INVALID, "SP2 fold tracking mode out of range");
   Sp2Bufs b;
-  if (int rc = sp2_bufs(ctx, n, b)) return rc;
+  if (int rc = sp2_bufs(ctx, n, n <= kSp2HomeMax ? nsteps + 1 : 2, b)) return rc;
   zq_prof_begin(ctx, "scf_sp2");
   sp2_start(ctx, b, dF, n, nocc, state6, skip, track);
   double *est = track ? b.est : nullptr;
   // about kSp2TilesPerGroup tiles per workgroup and step: fewer workgroups hand each step over with fewer
   // release fences, at the cost of more tiles per workgroup on the step's critical path
   const int groups = std::max(1, (b.ntiles + kSp2TilesPerGroup - 1) / kSp2TilesPerGroup);
-  if (b.m <= 256)
+  if (b.m <= kSp2HomeMax)
+    hipLaunchKernelGGL(k_sp2_home, dim3(8 * b.ntiles), dim3(256), 0, ctx->stream, b.X, b.mm, b.m, nocc, b.part, b.sync, state6,
+                       nsteps, tol, skip, est, ctx->turn & 7);
+  else if (b.m <= 256)
     hipLaunchKernelGGL(k_sp2_run<true>, dim3(groups), dim3(sp2_threads(true)), 0, ctx->stream, b.X, b.mm, b.m, nocc, b.part, b.sync,
                        state6, nsteps, tol, skip, est);
   else
@@ -568,7 +724,7 @@ double *zq_sp2_est(zq_ctx *ctx) { return (double *)zq_scratch(ctx, "sp2_est", kE
 int zq_sp2_density(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, int max_steps, int *steps_hint,
                    const double **dD, int *ld, int *steps) {
   Sp2Bufs b;
-  if (int rc = sp2_bufs(ctx, n, b)) return rc;
+  if (int rc = sp2_bufs(ctx, n, 2, b)) return rc;
   auto *state = (int *)zq_scratch(ctx, "sp2_state", 6 * sizeof(int));
   if (!state) return zq_fail(ctx, ZQ_ERR_OOM, "SP2 buffers");
   zq_prof_begin(ctx, "scf_sp2");

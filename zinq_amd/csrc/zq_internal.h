@@ -86,6 +86,7 @@ struct DevBuf {
 
 struct zq_ctx {
   int device = 0;
+  unsigned turn = 0;  // contexts counted through: which XCD a one-XCD kernel of this one prefers
   hipStream_t stream = nullptr;
   std::string err;
 
@@ -279,7 +280,7 @@ int zq_gemm_nt(zq_ctx *ctx, const double *A, int lda, const double *B, int ldb, 
 int zq_sp2_density(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, int max_steps, int *steps_hint,
                    const double **dD, int *ld, int *steps);  // zq_dense.hip
 // Enqueues SP2 with a budget of nsteps <= kSp2MaxSteps steps (one launch that stops once settled) and no
-// host synchronisation.  state6 = two {count, steps} pairs, the parity of the buffer that holds the
+// host synchronisation.  state6 = two {count, steps} pairs, the index of the buffer that holds the
 // settled projector, and an abort flag: the projector is *dX + state6[4] * *stride (m x m, ld m), which
 // a kernel selects at run time.  The final pair is state6 + 2 * (nsteps & 1); the result is settled when
 // count >= 2 there and state6[5] == 0.  All kernels return at once while *skip != 0.  track = 1 (the
