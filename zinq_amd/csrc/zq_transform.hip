@@ -513,47 +513,26 @@ __device__ inline T gemm_b(const GemmArgs<T> &g, const T *B, int k, int n) {
 // - each thread loads 4 elements of A and 4 of B per K step at per-thread offsets fixed for the whole
 //   loop, from uniform K-step bases; rows past M and columns past N are clamped to the last one (they
 //   only reach outputs that are not stored), so no load is masked;
-// - the gathered B of Q2 (mode 1, element (lambda, (sigma, nu)) at X[slot(lambda, sigma)][i][nu]) picks,
-//   per element, one of three per-thread offsets by whether lambda's AO block lies above, below or at
-//   sigma's, plus a uniform part per lambda block;
 // - K steps are loaded two ahead and staged one ahead, unconditionally (step indices past the last are
 //   clamped and their copies land in the LDS buffer no later step reads), so every path leaves the same
 //   loads in flight and the compiler's memory-counter waits are exact;
 // - a K that is not a multiple of 16 ends with one masked step (k >= K loads k = K - 1 and stages 0).
 struct GemmSlots {
-  unsigned offA[4], offB[4];           // mode 0: element offsets from the K-step bases (within one matrix)
-  unsigned long long p1[4], p2[4], pe[4];  // mode 1: slot offsets, lambda's block above / below / at sigma's
+  unsigned offA[4], offB[4];           // element offsets from the K-step bases (within one matrix)
   int kA[4], kB[4];                    // k of element j within its step
   int mA[4], nB[4];                    // row of A element j, column of B element j (clamped)
 };
 
 template <class MF>
 __device__ __forceinline__ void gemm_load(const GemmArgs<typename MF::T> &g, const typename MF::T *A,
-                                          const typename MF::T *B, const GemmSlots sl, int k0, int sb,
+                                          const typename MF::T *B, const GemmSlots sl, int k0,
                                           typename MF::T (&ra)[4], typename MF::T (&rb)[4]) {
   const typename MF::T *Ak = A + (long long)k0 * g.sAk;
 #pragma unroll
   for (int j = 0; j < 4; ++j) ra[j] = Ak[sl.offA[j]];
-  if (g.mode == 1) {
-    const unsigned long long sX = (unsigned long long)g.sXs;
+  const typename MF::T *Bk = B + (long long)k0 * g.sBk;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int lb = (k0 >> 3) + h;  // lambda block of elements 2h, 2h + 1 (uniform)
-      const unsigned long long u1 = (unsigned long long)(lb * (lb + 1) / 2) * 64 * sX;  // block pair (lb, sb)
-      const unsigned long long u2 = (unsigned long long)lb * 64 * sX;                    // block pair (sb, lb)
-      const int rel = lb - sb;
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int j = 2 * h + q;
-        const unsigned long long off = rel > 0 ? u1 + sl.p1[j] : (rel < 0 ? u2 + sl.p2[j] : sl.pe[j]);
-        rb[j] = B[off];
-      }
-    }
-  } else {
-    const typename MF::T *Bk = B + (long long)k0 * g.sBk;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) rb[j] = Bk[sl.offB[j]];
-  }
+  for (int j = 0; j < 4; ++j) rb[j] = Bk[sl.offB[j]];
 }
 
 // The last, partial K step: elements with k >= K are zero (their loads read k = K - 1).
@@ -571,7 +550,7 @@ __device__ __forceinline__ void gemm_load_tail(const GemmArgs<typename MF::T> &g
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int k = k0 + sl.kB[j], kc = min(k, g.K - 1);
-    const T x = gemm_b(g, B, kc, sl.nB[j]);
+    const T x = B[(long long)kc * g.sBk + (long long)sl.nB[j] * g.sBn];
     rb[j] = k < g.K ? x : T(0);
   }
 }
@@ -643,7 +622,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs<typename MF::T> &g, int
 #pragma unroll
     for (int y = 0; y < 2; ++y) acc[x][y] = MF::zero();
   const bool a_kfast = (g.sAk == 1);
-  const bool b_nfast = (g.mode == 1) || (g.sBn == 1);
+  const bool b_nfast = g.sBn == 1;
   bool live[2][2];
 #pragma unroll
   for (int x = 0; x < 2; ++x)
@@ -654,7 +633,6 @@ __device__ __forceinline__ void gemm_body(const GemmArgs<typename MF::T> &g, int
   // (tid >> 6) + 4 j); B (k, n) = ((tid >> 6) + 4 j, n0 + (tid & 63)) if b_nfast, else (tid & 15,
   // n0 + (tid >> 4) + 16 j)
   GemmSlots sl;
-  int sb = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int mm = a_kfast ? (tid >> 4) + 16 * j : tid & 63, kk = a_kfast ? tid & 15 : (tid >> 6) + 4 * j;
@@ -666,19 +644,6 @@ __device__ __forceinline__ void gemm_body(const GemmArgs<typename MF::T> &g, int
     sl.nB[j] = n, sl.kB[j] = kb;
     sl.offB[j] = unsigned((long long)kb * g.sBk + (long long)n * g.sBn);
   }
-  if (g.mode == 1) {
-    // slot(lambda, sigma) = bpair(max block, min block) * 64 + (max & 7) * 8 + (min & 7), as slot_of
-    const int n = sl.nB[0], sig = n / g.npad, nu = n - sig * g.npad, sr = sig & 7;
-    sb = sig >> 3;
-    const unsigned long long sX = (unsigned long long)g.sXs;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int lr = ((tid >> 6) + 4 * j) & 7;
-      sl.p1[j] = (unsigned long long)(sb * 64 + lr * 8 + sr) * sX + nu;
-      sl.p2[j] = (unsigned long long)((sb * (sb + 1) / 2) * 64 + sr * 8 + lr) * sX + nu;
-      sl.pe[j] = (unsigned long long)((sb * (sb + 1) / 2 + sb) * 64 + max(lr, sr) * 8 + min(lr, sr)) * sX + nu;
-    }
-  }
   T *const lA0 = a_kfast ? &As[0][tid & 15][tid >> 4] : &As[0][tid >> 6][tid & 63], *const lA1 = lA0 + 16 * 65;
   T *const lB0 = b_nfast ? &Bs[0][tid >> 6][tid & 63] : &Bs[0][tid & 15][tid >> 4], *const lB1 = lB0 + 16 * 65;
   const T *const lRA0 = &As[0][lane >> 4][wm + (lane & 15)], *const lRA1 = lRA0 + 16 * 65;
@@ -687,18 +652,18 @@ __device__ __forceinline__ void gemm_body(const GemmArgs<typename MF::T> &g, int
   const int nfull = g.K >> 4, last = nfull - 1;
   T ra[4], qa[4], rb[4], qb[4];  // (A, B) of the step in flight by parity: (ra, qa) even, (rb, qb) odd
   if (nfull > 0) {
-    gemm_load<MF>(g, A, B, sl, 0, sb, ra, qa);
+    gemm_load<MF>(g, A, B, sl, 0, ra, qa);
     gemm_stage(lA0, lB0, a_kfast, b_nfast, ra, qa);
-    gemm_load<MF>(g, A, B, sl, 16 * min(1, last), sb, rb, qb);
+    gemm_load<MF>(g, A, B, sl, 16 * min(1, last), rb, qb);
     __syncthreads();
     for (int s = 0; s < nfull; s += 2) {
       // step s from buffer 0; load s + 2 into (ra, qa); stage s + 1 (rb, qb) into buffer 1
-      gemm_load<MF>(g, A, B, sl, 16 * min(s + 2, last), sb, ra, qa);
+      gemm_load<MF>(g, A, B, sl, 16 * min(s + 2, last), ra, qa);
       gemm_mfmas<MF>(lRA0, lRB0, live, acc);
       gemm_stage(lA1, lB1, a_kfast, b_nfast, rb, qb);
       __syncthreads();
       // step s + 1 from buffer 1; load s + 3 into (rb, qb); stage s + 2 (ra, qa) into buffer 0
-      gemm_load<MF>(g, A, B, sl, 16 * min(s + 3, last), sb, rb, qb);
+      gemm_load<MF>(g, A, B, sl, 16 * min(s + 3, last), rb, qb);
       if (s + 1 < nfull) gemm_mfmas<MF>(lRA1, lRB1, live, acc);
       gemm_stage(lA0, lB0, a_kfast, b_nfast, ra, qa);
       __syncthreads();
@@ -935,6 +900,130 @@ int launch_gemm_bf16x3(zq_ctx *ctx, const GemmArgs<float> &g, int batch, const c
   return ZQ_OK;
 }
 
+// ---------------------------------------------------------------- Q2, FP64 / FP32
+// Y[i][j][sig][nu] = sum_lam C2[lam,j] X[slot(lam, sig)][i][nu]: few rows j (j <= i in a symmetric transform), very
+// many columns (sig, nu).  A wave owns 32 columns and up to 16 MT rows and walks lam by blocks of 8, operands from
+// memory straight into registers: no column is shared between waves and C2 stays in the L1, so there is no
+// staging and no barrier.  Lane l holds the columns 2 (l & 15) + {0, 1} of its wave's 32 (one load of two elements
+// per lam, one column in each of two MFMA tiles), rows of A as q1_c_index lays them out (one load per
+// row tile and block).  32 columns lie within one AO block of sig (8 npad columns, a multiple of 64), so which of
+// lam and sig is the larger block is uniform: an element's address is a scalar base for the lam block plus
+// one of three per-lane offsets (lam's block above, below or at sig's).  Operands are kept kQ2Ahead blocks ahead.
+// Against 64 x 64 tiles through LDS, half of whose rows are empty for small i: n = 192, o = 40, FP64 607 -> 412 us (the
+// X that it reads and the Y that it writes, 1.3 GB, at the copy rate 300; MFMA peak of its tiles 226); n = 101,
+// o = 20, FP32C 62 -> 24; 96 molecules n <= 72 550 -> 208.  Two to four blocks ahead do alike.
+constexpr int kQ2Ahead = 4;
+
+// The wave's columns n0 .. n0 + 31 of rows m0 .. m0 + 16 H - 1.
+template <class MF, int H>
+__device__ __forceinline__ void q2_tiles(const GemmArgs<typename MF::T> &g, const typename MF::T *A, const typename MF::T *B,
+                                         typename MF::T *C, int M, int m0, int n0) {
+  typedef typename MF::T T;
+  typedef T T2 __attribute__((ext_vector_type(2)));
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int np = g.npad, n = n0 + 2 * r, nc = min(n, g.N - 2), sig = nc / np, nu = nc - sig * np, sr = sig & 7;
+  const int sb = (n0 / np) >> 3;  // the wave's block of sig
+  const unsigned sX = unsigned(g.sXs);
+  unsigned up[2], down[2], at[2], coff[H];  // byte offsets: lam's block above, below, at sig's; rows of A
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const int lr = 4 * ks + q;
+    up[ks] = (unsigned(lr * 8 + sr) * sX + nu) * unsigned(sizeof(T));
+    down[ks] = (unsigned(sr * 8 + lr) * sX + nu) * unsigned(sizeof(T));
+    at[ks] = (unsigned(max(lr, sr) * 8 + min(lr, sr)) * sX + nu) * unsigned(sizeof(T));
+  }
+#pragma unroll
+  for (int h = 0; h < H; ++h)
+    coff[h] = unsigned(q1_c_index(q, min(m0 + 16 * h + r, g.M - 1), g.M)) * unsigned(sizeof(T));
+  typename MF::acc acc[H][2];
+#pragma unroll
+  for (int h = 0; h < H; ++h) acc[h][0] = acc[h][1] = MF::zero();
+  const int nblk = g.K / 8, last = nblk - 1;
+  T2 a[kQ2Ahead][H], b[kQ2Ahead][2];
+  auto load = [&](int lb, T2(&av)[H], T2(&bv)[2]) {
+    const size_t slot = 64 * size_t(lb > sb ? zq_bpair(lb, sb) : zq_bpair(sb, lb));
+    const char *pb = reinterpret_cast<const char *>(B + slot * g.sXs), *pa = reinterpret_cast<const char *>(A + size_t(lb) * 8 * g.M);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const unsigned off = lb > sb ? up[ks] : (lb < sb ? down[ks] : at[ks]);
+      bv[ks] = *reinterpret_cast<const T2 *>(pb + off);
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) av[h] = *reinterpret_cast<const T2 *>(pa + coff[h]);
+  };
+  auto multiply = [&](int lb, const T2(&av)[H], const T2(&bv)[2]) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[h][c] = MF::mma(av[h][ks], bv[ks][c], acc[h][c]);
+    if (std::is_same<MF, MF32C>::value && ((lb & 1) || lb == last))
+#pragma unroll
+      for (int h = 0; h < H; ++h) MF::flush(acc[h][0]), MF::flush(acc[h][1]);
+  };
+#pragma unroll
+  for (int u = 0; u < kQ2Ahead; ++u) load(min(u, last), a[u], b[u]);
+  int lb = 0;
+  for (; lb + kQ2Ahead <= nblk; lb += kQ2Ahead)
+#pragma unroll
+    for (int u = 0; u < kQ2Ahead; ++u) {
+      multiply(lb + u, a[u], b[u]);
+      load(min(lb + u + kQ2Ahead, last), a[u], b[u]);
+    }
+#pragma unroll
+  for (int u = 0; u + 1 < kQ2Ahead; ++u)
+    if (lb + u < nblk) multiply(lb + u, a[u], b[u]);
+  if (n >= g.N) return;
+#pragma unroll
+  for (int h = 0; h < H; ++h)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int m = m0 + 16 * h + MF::row(lane, j);
+      if (m < M) *reinterpret_cast<T2 *>(C + m * g.sCm + n) = T2{T(MF::val(acc[h][0], j)), T(MF::val(acc[h][1], j))};
+    }
+}
+
+template <class MF, int MT>
+__device__ __forceinline__ void q2_body(const GemmArgs<typename MF::T> &g, int bx, int by, int bz) {
+  const typename MF::T *A, *B;
+  typename MF::T *C;
+  int M;
+  gemm_batch(g, g.b0 + bz, A, B, C, M);
+  const int m0 = by * 16 * MT, n0 = __builtin_amdgcn_readfirstlane(bx * 128 + int(threadIdx.x >> 6) * 32);
+  if (m0 >= M || n0 >= g.N) return;  // no barrier follows
+  // only the row tiles below M
+  const int live = (M - m0 + 15) / 16;
+  if (MT == 1 || live <= 1) q2_tiles<MF, 1>(g, A, B, C, M, m0, n0);
+  else if (MT == 2 || live == 2) q2_tiles<MF, MT >= 2 ? 2 : 1>(g, A, B, C, M, m0, n0);
+  else if (MT == 3 || live == 3) q2_tiles<MF, MT >= 3 ? 3 : 1>(g, A, B, C, M, m0, n0);
+  else q2_tiles<MF, MT>(g, A, B, C, M, m0, n0);
+}
+
+template <class MF, int MT>
+__global__ __launch_bounds__(256) void zq_q2(const GemmArgs<typename MF::T> g) {
+  q2_body<MF, MT>(g, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+template <class MF>
+int launch_q2(zq_ctx *ctx, const GemmArgs<typename MF::T> &g, int batch) {
+  const int mt = std::min(4, (g.M + 15) / 16);
+  zq_prof_begin(ctx, "ao2mo_q2");
+  for (int b0 = 0; b0 < batch; b0 += kMaxGridZ) {
+    const dim3 grid(unsigned((g.N + 127) / 128), unsigned((g.M + 16 * mt - 1) / (16 * mt)), unsigned(std::min(kMaxGridZ, batch - b0)));
+    const auto s = batch_slice(g, b0);
+    switch (mt) {
+      case 1: hipLaunchKernelGGL((zq_q2<MF, 1>), grid, dim3(256), 0, ctx->stream, s); break;
+      case 2: hipLaunchKernelGGL((zq_q2<MF, 2>), grid, dim3(256), 0, ctx->stream, s); break;
+      case 3: hipLaunchKernelGGL((zq_q2<MF, 3>), grid, dim3(256), 0, ctx->stream, s); break;
+      default: hipLaunchKernelGGL((zq_q2<MF, 4>), grid, dim3(256), 0, ctx->stream, s); break;
+    }
+  }
+  zq_prof_end(ctx);
+  ZQ_LAUNCH_CHECK(ctx, "ao2mo_q2");
+  return ZQ_OK;
+}
+
 // Device buffers of one transform: the context's grow-only scratch, or (base != null) consecutive
 // 256-byte aligned pieces of the static no-allocation scratch, cap bytes long.
 struct Arena {
@@ -962,14 +1051,14 @@ int upload(zq_ctx *ctx, const char *name, const std::vector<T> &h, T **d) {
 // same element conversions as the host staging, so the values are identical.
 template <class T>
 __device__ __forceinline__ void c_slices_body(const double *__restrict__ C, int n, int np, int m1, int m2, int m3,
-                                              int off3, T *__restrict__ c1, T *__restrict__ c2t, T *__restrict__ c3,
-                                              int mu) {
+                                              int off3, T *__restrict__ c1, T *__restrict__ c2, bool c2t,
+                                              T *__restrict__ c3, int mu) {
   for (int t = threadIdx.x; t < m1 + m2 + m3; t += blockDim.x) {
     if (t < m1) {
       c1[q1_c_index(mu, t, m1)] = mu < n ? T(C[size_t(mu) * n + t]) : T(0);
     } else if (t < m1 + m2) {
       const int j = t - m1;
-      c2t[size_t(j) * np + mu] = mu < n ? T(C[size_t(mu) * n + j]) : T(0);
+      c2[c2t ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = mu < n ? T(C[size_t(mu) * n + j]) : T(0);
     } else {
       const int a = t - m1 - m2;
       c3[size_t(mu) * m3 + a] = mu < n ? T(C[size_t(mu) * n + off3 + a]) : T(0);
@@ -979,8 +1068,8 @@ __device__ __forceinline__ void c_slices_body(const double *__restrict__ C, int 
 
 template <class T>
 __global__ void zq_c_slices(const double *__restrict__ C, int n, int np, int m1, int m2, int m3, int off3,
-                            T *__restrict__ c1, T *__restrict__ c2t, T *__restrict__ c3) {
-  c_slices_body<T>(C, n, np, m1, m2, m3, off3, c1, c2t, c3, blockIdx.x);  // one workgroup per row mu < np
+                            T *__restrict__ c1, T *__restrict__ c2, bool c2t, T *__restrict__ c3) {
+  c_slices_body<T>(C, n, np, m1, m2, m3, off3, c1, c2, c2t, c3, blockIdx.x);  // one workgroup per row mu < np
 }
 
 // y = x (n doubles; x may be pinned host memory)
@@ -1046,7 +1135,8 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     return zq_fail(ctx, ZQ_ERR_INVALID, "one coefficient matrix only");
   // BF16X3 Q1 takes C1 split and transposed: C1h/C1l[i][mu], mu padded to a multiple of 32
   const int ldt = ((nb + 3) / 4) * 32;
-  T *d1, *d2t, *d3, *d4 = nullptr;
+  T *d1, *d2, *d3, *d4 = nullptr;
+  const bool c2t = precision == ZQ_PREC_BF16X3;  // its Q2 takes C2 transposed, the others' as q1_c_index lays it out
   bf16 *d1h = nullptr, *d1l = nullptr;
   if constexpr (sizeof(T) == 4) {
     if (precision != ZQ_PREC_BF16X3) {
@@ -1059,17 +1149,17 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
   if (fixed) {
     auto *dC = (double *)ar.get("C", size_t(n) * n * 8);
     d1 = (T *)ar.get("C1", size_t(np) * m1 * sizeof(T));
-    d2t = (T *)ar.get("C2T", size_t(m2) * np * sizeof(T));
+    d2 = (T *)ar.get("C2", size_t(m2) * np * sizeof(T));
     d3 = (T *)ar.get("C3", size_t(np) * m3 * sizeof(T));
     if (precision == ZQ_PREC_BF16X3) {
       d1h = (bf16 *)ar.get("C1h", size_t(m1) * ldt * sizeof(bf16));
       d1l = (bf16 *)ar.get("C1l", size_t(m1) * ldt * sizeof(bf16));
     }
-    if (!dC || !d1 || !d2t || !d3 || (precision == ZQ_PREC_BF16X3 && (!d1h || !d1l)))
+    if (!dC || !d1 || !d2 || !d3 || (precision == ZQ_PREC_BF16X3 && (!d1h || !d1l)))
       return zq_fail(ctx, ZQ_ERR_INVALID, "zq_mp2_noalloc: static scratch too small");
     ZQ_TRY(ctx, hipMemcpyAsync(dC, C, size_t(n) * n * 8, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(zq_c_slices<T>, dim3(unsigned(np)), dim3(256), 0, ctx->stream, dC, n, np, m1, m2, m3, d.off3, d1,
-                       d2t, d3);
+                       d2, c2t, d3);
     if (precision == ZQ_PREC_BF16X3)
       hipLaunchKernelGGL(zq_c1_split, dim3(unsigned(m1)), dim3(256), 0, ctx->stream, dC, n, m1, ldt, d1h, d1l);
     ZQ_LAUNCH_CHECK(ctx, "zq_c_slices");
@@ -1077,33 +1167,33 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     // C readable by kernels: the slices are cut on the device, as above, into the buffers the host staging
     // of the dual transform's matrices below fills
     d1 = (T *)zq_scratch(ctx, "C1", size_t(np) * m1 * sizeof(T), nullptr, false);
-    d2t = (T *)zq_scratch(ctx, "C2T", size_t(m2) * np * sizeof(T), nullptr, false);
+    d2 = (T *)zq_scratch(ctx, "C2", size_t(m2) * np * sizeof(T), nullptr, false);
     d3 = (T *)zq_scratch(ctx, "C3", size_t(np) * m3 * sizeof(T), nullptr, false);
     if (precision == ZQ_PREC_BF16X3) {
       d1h = (bf16 *)zq_scratch(ctx, "C1h", size_t(m1) * ldt * sizeof(bf16), nullptr, false);
       d1l = (bf16 *)zq_scratch(ctx, "C1l", size_t(m1) * ldt * sizeof(bf16), nullptr, false);
     }
-    if (!d1 || !d2t || !d3 || (precision == ZQ_PREC_BF16X3 && (!d1h || !d1l)))
+    if (!d1 || !d2 || !d3 || (precision == ZQ_PREC_BF16X3 && (!d1h || !d1l)))
       return zq_fail(ctx, ZQ_ERR_OOM, "transform scratch C slices");
     hipLaunchKernelGGL(zq_c_slices<T>, dim3(unsigned(np)), dim3(256), 0, ctx->stream, C, n, np, m1, m2, m3, d.off3, d1,
-                       d2t, d3);
+                       d2, c2t, d3);
     if (precision == ZQ_PREC_BF16X3)
       hipLaunchKernelGGL(zq_c1_split, dim3(unsigned(m1)), dim3(256), 0, ctx->stream, C, n, m1, ldt, d1h, d1l);
     ZQ_LAUNCH_CHECK(ctx, "zq_c_slices");
   } else {
-    // coefficient slices, zero rows for padded AOs: C1 (np x m1), C2T (m2 x np), C3 = C4 (np x m3)
+    // coefficient slices, zero rows for padded AOs: C1 (np x m1), C2 (np x m2), C3 = C4 (np x m3)
     // (each quarter from its own matrix cf.q[0..3]; the same C unless this is a term of the dual transform)
-    std::vector<T> h1(size_t(np) * m1, T(0)), h2t(size_t(m2) * np, T(0)), h3(size_t(np) * m3, T(0)),
+    std::vector<T> h1(size_t(np) * m1, T(0)), h2(size_t(m2) * np, T(0)), h3(size_t(np) * m3, T(0)),
         h4(own4 ? size_t(np) * m4 : 0, T(0));
     for (int mu = 0; mu < n; ++mu) {
       for (int i = 0; i < m1; ++i) h1[q1_c_index(mu, i, m1)] = T(cf.q[0][size_t(mu) * n + i]);
-      for (int j = 0; j < m2; ++j) h2t[size_t(j) * np + mu] = T(cf.q[1][size_t(mu) * n + j]);
+      for (int j = 0; j < m2; ++j) h2[c2t ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = T(cf.q[1][size_t(mu) * n + j]);
       for (int a = 0; a < m3; ++a) h3[size_t(mu) * m3 + a] = T(cf.q[2][size_t(mu) * n + d.off3 + a]);
       if (own4)
         for (int b = 0; b < m4; ++b) h4[size_t(mu) * m4 + b] = T(cf.q[3][size_t(mu) * n + d.off3 + b]);
     }
     if (int rc = upload(ctx, "C1", h1, &d1)) return rc;
-    if (int rc = upload(ctx, "C2T", h2t, &d2t)) return rc;
+    if (int rc = upload(ctx, "C2", h2, &d2)) return rc;
     if (int rc = upload(ctx, "C3", h3, &d3)) return rc;
     if (own4)
       if (int rc = upload(ctx, "C4", h4, &d4)) return rc;
@@ -1176,8 +1266,9 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     ZQ_LAUNCH_CHECK(ctx, "ao2mo_q1");
   }
   GemmArgs<T> g2{}, g3{}, g4{};
-  // Q2: batch over i; A = C2T (m2 x np), B gathered from X, out Y[i][j][sig][nu] (j <= i if symmetric)
-  g2.A = d2t, g2.sAb = 0, g2.sAm = np, g2.sAk = 1;
+  // Q2: batch over i; A = C2 (BF16X3: its transpose, m2 x np), B gathered from X, out Y[i][j][sig][nu] (j <= i if
+  // symmetric)
+  g2.A = d2, g2.sAb = 0, g2.sAm = np, g2.sAk = 1;
   g2.B = X, g2.sBb = np, g2.mode = 1, g2.npad = np, g2.sXs = (long long)m1 * np;
   g2.C = Y, g2.sCb = (long long)m2 * np * np, g2.sCm = (long long)np * np, g2.sCn = 1;
   g2.M = m2, g2.N = np * np, g2.K = np;
@@ -1203,7 +1294,7 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
       return ZQ_OK;
     }
   }
-  if (int rc = launch_gemm<MF>(ctx, g2, m1, "ao2mo_q2")) return rc;
+  if (int rc = launch_q2<MF>(ctx, g2, m1)) return rc;
   if (int rc = launch_gemm<MF>(ctx, g3, nij, "ao2mo_q3")) return rc;
   // Q4 on the tile kernel in every precision (no library GEMM in the transform)
   if (int rc = launch_gemm<MF>(ctx, g4, nij, "ao2mo_q4")) return rc;
@@ -1394,7 +1485,7 @@ template <class T, class E>
 struct GJob {
   const E *eri;
   const double *C, *e;
-  T *c1, *c2t, *c3, *X, *O;
+  T *c1, *c2, *c3, *X, *O;
   double *partial, *out;
   int n, np, nb, Nb, o, v, groups, pairs;
   GemmArgs<T> g[3];  // Q2, Q3, Q4
@@ -1421,7 +1512,7 @@ __global__ __launch_bounds__(256) void zq_group_slices(const GJob<T, E> *__restr
                                                        int nmol) {
   const int m = group_find(start, nmol, blockIdx.x);
   const GJob<T, E> J = jobs[m];
-  c_slices_body<T>(J.C, J.n, J.np, J.o, J.o, J.v, J.o, J.c1, J.c2t, J.c3, int(blockIdx.x) - start[m]);
+  c_slices_body<T>(J.C, J.n, J.np, J.o, J.o, J.v, J.o, J.c1, J.c2, false, J.c3, int(blockIdx.x) - start[m]);
 }
 
 template <class MF, class E>
@@ -1440,6 +1531,15 @@ __global__ __launch_bounds__(256, 2) void zq_group_gemm(const GJob<typename MF::
   const GemmArgs<typename MF::T> g = jobs[m].g[q];
   const int l = int(blockIdx.x) - start[m], gx = (g.N + 63) / 64, gy = (g.M + 63) / 64, t = l / gx;
   gemm_body<MF>(g, l - t * gx, t % gy, t / gy);
+}
+
+template <class MF, class E>
+__global__ __launch_bounds__(256) void zq_group_q2(const GJob<typename MF::T, E> *__restrict__ jobs,
+                                                   const int *__restrict__ start, int nmol) {
+  const int m = group_find(start, nmol, blockIdx.x);
+  const GemmArgs<typename MF::T> g = jobs[m].g[0];
+  const int l = int(blockIdx.x) - start[m], gx = (g.N + 127) / 128, gy = (g.M + 15) / 16, t = l / gx;
+  q2_body<MF, 1>(g, l - t * gx, t % gy, t / gy);
 }
 
 template <class T, class E>
@@ -1520,7 +1620,7 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
         J.eri = mo.eri;
       J.C = mo.C, J.e = mo.e;
       J.c1 = (T *)take(np * o * sizeof(T));
-      J.c2t = (T *)take(o * np * sizeof(T));
+      J.c2 = (T *)take(o * np * sizeof(T));
       J.c3 = (T *)take(np * v * sizeof(T));
       J.X = (T *)take(size_t(J.Nb) * 64 * o * np * sizeof(T));
       T *Y = (T *)take(o * o * np * np * sizeof(T));
@@ -1528,10 +1628,10 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
       J.O = (T *)take(pr * v * v * sizeof(T));
       J.partial = (double *)take(pr * 8 + 8);
       J.out = d_out + k;
-      // Q2: batch over i; A = C2T (o x np), B gathered from X, out Y[i][j][sig][nu], j <= i
+      // Q2: batch over i; A = C2, B gathered from X, out Y[i][j][sig][nu], j <= i
       GemmArgs<T> &g2 = J.g[0];
       g2 = GemmArgs<T>{};
-      g2.A = J.c2t, g2.sAb = 0, g2.sAm = J.np, g2.sAk = 1;
+      g2.A = J.c2, g2.sAb = 0, g2.sAm = J.np, g2.sAk = 1;
       g2.B = J.X, g2.sBb = J.np, g2.mode = 1, g2.npad = J.np, g2.sXs = (long long)o * np;
       g2.C = Y, g2.sCb = (long long)o * np * np, g2.sCm = (long long)np * np, g2.sCn = 1;
       g2.M = J.o, g2.N = J.np * J.np, g2.K = J.np, g2.tri = 1;
@@ -1553,7 +1653,7 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
       const long long cnt[GS_COUNT] = {
           J.np,
           (long long)J.Nb * J.nb * J.groups * 2,
-          (long long)((g2.N + 63) / 64) * ((g2.M + 63) / 64) * J.o,
+          (long long)((g2.N + 127) / 128) * ((g2.M + 15) / 16) * J.o,
           (long long)((g3.N + 63) / 64) * ((g3.M + 63) / 64) * J.pairs,
           (long long)((g4.N + 63) / 64) * ((g4.M + 63) / 64) * J.pairs,
           (long long)J.pairs};
@@ -1575,7 +1675,8 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
     auto total = [&](int s) { return unsigned(start[size_t(s) * (nm + 1) + nm]); };
     hipLaunchKernelGGL((zq_group_slices<T, E>), dim3(total(GS_SLICES)), dim3(256), 0, stream, d_jobs, st(GS_SLICES), nm);
     hipLaunchKernelGGL((zq_group_q1<MF, E>), dim3(total(GS_Q1)), dim3(256), 0, stream, d_jobs, st(GS_Q1), nm);
-    for (int q = 0; q < 3; ++q)
+    hipLaunchKernelGGL((zq_group_q2<MF, E>), dim3(total(GS_Q2)), dim3(256), 0, stream, d_jobs, st(GS_Q2), nm);
+    for (int q = 1; q < 3; ++q)
       hipLaunchKernelGGL((zq_group_gemm<MF, E>), dim3(total(GS_Q2 + q)), dim3(256), 0, stream, d_jobs, st(GS_Q2 + q), nm, q);
     hipLaunchKernelGGL((zq_group_pairs<T, E>), dim3(total(GS_PAIRS)), dim3(256), 0, stream, d_jobs, st(GS_PAIRS), nm);
     hipLaunchKernelGGL((zq_group_sum<T, E>), dim3(unsigned(nm)), dim3(64), 0, stream, d_jobs);
