@@ -41,3 +41,26 @@ def test_first_quarter_edges(ctx, n, o):
     for precision, eps in (("fp64", np.finfo(np.float64).eps), ("fp32", np.finfo(np.float32).eps), ("fp32c", np.finfo(np.float32).eps)):
         out = ctx.ao2mo(C, o, "ovov", precision=precision)
         assert np.all(np.abs(out - ref) <= (4 * n + 8) * eps * scale), (n, o, precision)
+
+
+@pytest.mark.parametrize("n,o", [(2, 1), (9, 8), (33, 16), (34, 17), (41, 20), (58, 25), (75, 11)])
+def test_group_takes_the_same_path(n, o):
+    """A batch's MP2 is zq_mp2 of its orbitals to the last bit in every precision: odd and even numbers of virtuals
+    (the register-direct Q3 and Q4 take pairs of them, or one at a time), one to four tiles of them."""
+    from zinq_amd import hip
+    from zinq_amd.batch import Batch
+    rng = np.random.default_rng(n + o)
+    np_ = n * (n + 1) // 2
+    pk = 1e-3 * rng.standard_normal(np_ * (np_ + 1) // 2)  # small: the SCF is that of H
+    H = np.diag(np.concatenate([np.linspace(-9.0, -3.0, o), np.linspace(1.0, 5.0, n - o)]))
+    for precision in ("fp64", "fp32", "fp32c"):
+        b = Batch(0)
+        b.add(H, np.eye(n), 0.0, o, pk)
+        r = b.run(mp2_precision=precision)
+        e, C = b.orbitals(0)
+        b.close()
+        c = hip.Context(0)
+        c.eri_load_packed(pk, n)
+        assert r["status"][0] == 0
+        assert r["E_corr"][0] == c.mp2(C, e, o, precision=precision), precision
+        c.close()

@@ -507,7 +507,7 @@ __device__ inline T gemm_b(const GemmArgs<T> &g, const T *B, int k, int n) {
   return B[k * g.sBk + n * g.sBn];
 }
 
-// FP64 / FP32 / FP32C: 64 x 64 tiles, BK = 16, four waves of 32 x 32 (2 x 2 MFMA tiles, so each LDS
+// FP64 Q3 and Q4: 64 x 64 tiles, BK = 16, four waves of 32 x 32 (2 x 2 MFMA tiles, so each LDS
 // operand read feeds two MFMAs).  Written, like Q1, to issue few vector ALU instructions (the FP64 MFMAs
 // do not co-issue with them):
 // - each thread loads 4 elements of A and 4 of B per K step at per-thread offsets fixed for the whole
@@ -900,37 +900,52 @@ int launch_gemm_bf16x3(zq_ctx *ctx, const GemmArgs<float> &g, int batch, const c
   return ZQ_OK;
 }
 
-// ---------------------------------------------------------------- Q2, FP64 / FP32
-// Y[i][j][sig][nu] = sum_lam C2[lam,j] X[slot(lam, sig)][i][nu]: few rows j (j <= i in a symmetric transform), very
-// many columns (sig, nu).  A wave owns 32 columns and up to 16 MT rows and walks lam by blocks of 8, operands from
-// memory straight into registers: no column is shared between waves and C2 stays in the L1, so there is no
-// staging and no barrier.  Lane l holds the columns 2 (l & 15) + {0, 1} of its wave's 32 (one load of two elements
-// per lam, one column in each of two MFMA tiles), rows of A as q1_c_index lays them out (one load per
-// row tile and block).  32 columns lie within one AO block of sig (8 npad columns, a multiple of 64), so which of
-// lam and sig is the larger block is uniform: an element's address is a scalar base for the lam block plus
-// one of three per-lane offsets (lam's block above, below or at sig's).  Operands are kept kQ2Ahead blocks ahead.
-// Against 64 x 64 tiles through LDS, half of whose rows are empty for small i: n = 192, o = 40, FP64 607 -> 412 us (the
-// X that it reads and the Y that it writes, 1.3 GB, at the copy rate 300; MFMA peak of its tiles 226); n = 101,
-// o = 20, FP32C 62 -> 24; 96 molecules n <= 72 550 -> 208.  Two to four blocks ahead do alike.
-constexpr int kQ2Ahead = 4;
+// ---------------------------------------------------------------- Q2, Q3, Q4, FP64 / FP32
+// Q2, and in the 4-byte forms Q3 and Q4, contract one index of a wide array, Wd[k][w] (w contiguous), with a narrow one of few columns f:
+//   Q2  Y[i][j][sig][nu] = sum_lam C2[lam,j] X[slot(lam, sig)][i][nu]   w = (sig, nu), f = j (j <= i if symmetric)
+//   Q3  W[ij][nu][b]     = sum_sig Y[ij][sig][nu] C4[sig,b]             w = nu, f = b
+//   Q4  out[ij][a][b]    = sum_nu  C3[nu,a] W[ij][nu][b]                w = b, f = a
+// A wave owns 32 w and up to 16 MT f and walks k by blocks of 8, operands from memory straight into registers: no w
+// is shared between waves and the coefficients stay in the L1, so there is no staging and no barrier.  Lane l
+// holds w = 2 (l & 15) + {0, 1} of its wave's 32 (one load of two elements per k, one w in each of two MFMA tiles);
+// the coefficients lie as q1_c_index has them (one load per tile of f and block).  Operands are kept kWideAhead
+// blocks ahead.  ROWS: f are the rows of the output (w contiguous in it), else its columns (f contiguous).
+// SLOTS (Q2): 32 w lie within one AO block of sig (8 npad of them, a multiple of 64), so which of lam and sig is the
+// larger block is uniform: an element's address is a scalar base for the lam block plus one of three per-lane
+// offsets (lam's block above, below or at sig's).  Otherwise k has the stride sBk; odd strides (PAIRS false) take
+// the two elements one by one.
+// Against 64 x 64 tiles through LDS: Q2 at n = 192, o = 40, FP64 607 -> 408 us (the X that it reads and the Y that it
+// writes, 1.3 GB, at the copy rate 300; MFMA peak of its tiles 226; half the rows of a 64 x 64 tile are empty for
+// small i); n = 101, o = 20, FP32C Q2 62 -> 24, Q3 18 -> 13, Q4 18 -> 11; 96 molecules n <= 72 Q2 550 -> 208.  Q3 and
+// Q4 stay with the tiles in FP64, whose operands are as wide as two of these waves' registers: 231 and 219 us at
+// n = 192 against 291 and 278.  Two to four blocks ahead do alike.
+constexpr int kWideAhead = 2;
 
-// The wave's columns n0 .. n0 + 31 of rows m0 .. m0 + 16 H - 1.
-template <class MF, int H>
-__device__ __forceinline__ void q2_tiles(const GemmArgs<typename MF::T> &g, const typename MF::T *A, const typename MF::T *B,
-                                         typename MF::T *C, int M, int m0, int n0) {
+// w = n0 .. n0 + 31, f = m0 .. m0 + 16 H - 1 below M.
+template <class MF, int H, bool SLOTS, bool ROWS, bool PAIRS>
+__device__ __forceinline__ void wide_tiles(const GemmArgs<typename MF::T> &g, const typename MF::T *A, const typename MF::T *B,
+                                           typename MF::T *C, int M, int m0, int n0) {
   typedef typename MF::T T;
   typedef T T2 __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-  const int np = g.npad, n = n0 + 2 * r, nc = min(n, g.N - 2), sig = nc / np, nu = nc - sig * np, sr = sig & 7;
-  const int sb = (n0 / np) >> 3;  // the wave's block of sig
-  const unsigned sX = unsigned(g.sXs);
-  unsigned up[2], down[2], at[2], coff[H];  // byte offsets: lam's block above, below, at sig's; rows of A
+  const int n = n0 + 2 * r, nc = PAIRS ? min(n, g.N - 2) : min(n, g.N - 1), nd = PAIRS ? nc + 1 : min(n + 1, g.N - 1);
+  // byte offsets: of the two w at the block's rows (SLOTS: with lam's block above, below, at sig's) and of f
+  unsigned up[2], down[2], at[2], more = unsigned(nd - nc) * unsigned(sizeof(T)), coff[H];
+  int sb = 0;  // the wave's block of sig
+  if (SLOTS) {
+    const int np = g.npad, sig = nc / np, nu = nc - sig * np, sr = sig & 7;
+    const unsigned sX = unsigned(g.sXs);
+    sb = (n0 / np) >> 3;
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int lr = 4 * ks + q;
-    up[ks] = (unsigned(lr * 8 + sr) * sX + nu) * unsigned(sizeof(T));
-    down[ks] = (unsigned(sr * 8 + lr) * sX + nu) * unsigned(sizeof(T));
-    at[ks] = (unsigned(max(lr, sr) * 8 + min(lr, sr)) * sX + nu) * unsigned(sizeof(T));
+    for (int ks = 0; ks < 2; ++ks) {
+      const int lr = 4 * ks + q;
+      up[ks] = (unsigned(lr * 8 + sr) * sX + nu) * unsigned(sizeof(T));
+      down[ks] = (unsigned(sr * 8 + lr) * sX + nu) * unsigned(sizeof(T));
+      at[ks] = (unsigned(max(lr, sr) * 8 + min(lr, sr)) * sX + nu) * unsigned(sizeof(T));
+    }
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) up[ks] = down[ks] = at[ks] = (unsigned(4 * ks + q) * unsigned(g.sBk) + nc) * unsigned(sizeof(T));
   }
 #pragma unroll
   for (int h = 0; h < H; ++h)
@@ -939,14 +954,17 @@ __device__ __forceinline__ void q2_tiles(const GemmArgs<typename MF::T> &g, cons
 #pragma unroll
   for (int h = 0; h < H; ++h) acc[h][0] = acc[h][1] = MF::zero();
   const int nblk = g.K / 8, last = nblk - 1;
-  T2 a[kQ2Ahead][H], b[kQ2Ahead][2];
+  T2 a[kWideAhead][H], b[kWideAhead][2];
   auto load = [&](int lb, T2(&av)[H], T2(&bv)[2]) {
-    const size_t slot = 64 * size_t(lb > sb ? zq_bpair(lb, sb) : zq_bpair(sb, lb));
-    const char *pb = reinterpret_cast<const char *>(B + slot * g.sXs), *pa = reinterpret_cast<const char *>(A + size_t(lb) * 8 * g.M);
+    const size_t row = SLOTS ? 64 * size_t(lb > sb ? zq_bpair(lb, sb) : zq_bpair(sb, lb)) * g.sXs : size_t(lb) * 8 * g.sBk;
+    const char *pb = reinterpret_cast<const char *>(B + row), *pa = reinterpret_cast<const char *>(A + size_t(lb) * 8 * g.M);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const unsigned off = lb > sb ? up[ks] : (lb < sb ? down[ks] : at[ks]);
-      bv[ks] = *reinterpret_cast<const T2 *>(pb + off);
+      const unsigned off = !SLOTS || lb > sb ? up[ks] : (lb < sb ? down[ks] : at[ks]);
+      if (PAIRS)
+        bv[ks] = *reinterpret_cast<const T2 *>(pb + off);
+      else
+        bv[ks] = T2{*reinterpret_cast<const T *>(pb + off), *reinterpret_cast<const T *>(pb + (off + more))};
     }
 #pragma unroll
     for (int h = 0; h < H; ++h) av[h] = *reinterpret_cast<const T2 *>(pa + coff[h]);
@@ -957,70 +975,163 @@ __device__ __forceinline__ void q2_tiles(const GemmArgs<typename MF::T> &g, cons
 #pragma unroll
       for (int h = 0; h < H; ++h)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) acc[h][c] = MF::mma(av[h][ks], bv[ks][c], acc[h][c]);
+        for (int c = 0; c < 2; ++c)
+          acc[h][c] = ROWS ? MF::mma(av[h][ks], bv[ks][c], acc[h][c]) : MF::mma(bv[ks][c], av[h][ks], acc[h][c]);
     if (std::is_same<MF, MF32C>::value && ((lb & 1) || lb == last))
 #pragma unroll
       for (int h = 0; h < H; ++h) MF::flush(acc[h][0]), MF::flush(acc[h][1]);
   };
 #pragma unroll
-  for (int u = 0; u < kQ2Ahead; ++u) load(min(u, last), a[u], b[u]);
+  for (int u = 0; u < kWideAhead; ++u) load(min(u, last), a[u], b[u]);
   int lb = 0;
-  for (; lb + kQ2Ahead <= nblk; lb += kQ2Ahead)
+  for (; lb + kWideAhead <= nblk; lb += kWideAhead)
 #pragma unroll
-    for (int u = 0; u < kQ2Ahead; ++u) {
+    for (int u = 0; u < kWideAhead; ++u) {
       multiply(lb + u, a[u], b[u]);
-      load(min(lb + u + kQ2Ahead, last), a[u], b[u]);
+      load(min(lb + u + kWideAhead, last), a[u], b[u]);
     }
 #pragma unroll
-  for (int u = 0; u + 1 < kQ2Ahead; ++u)
+  for (int u = 0; u + 1 < kWideAhead; ++u)
     if (lb + u < nblk) multiply(lb + u, a[u], b[u]);
-  if (n >= g.N) return;
 #pragma unroll
   for (int h = 0; h < H; ++h)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int m = m0 + 16 * h + MF::row(lane, j);
-      if (m < M) *reinterpret_cast<T2 *>(C + m * g.sCm + n) = T2{T(MF::val(acc[h][0], j)), T(MF::val(acc[h][1], j))};
+      const T v0 = T(MF::val(acc[h][0], j)), v1 = T(MF::val(acc[h][1], j));
+      if (ROWS) {
+        const int m = m0 + 16 * h + MF::row(lane, j);
+        if (m >= M) continue;
+        T *o = C + m * g.sCm + n;
+        if (PAIRS && n < g.N) {
+          *reinterpret_cast<T2 *>(o) = T2{v0, v1};
+        } else if (!PAIRS) {
+          if (n < g.N) o[0] = v0;
+          if (n + 1 < g.N) o[1] = v1;
+        }
+      } else {
+        const int w = n0 + 2 * MF::row(lane, j), m = m0 + 16 * h + r;
+        if (m >= M) continue;
+        if (w < g.N) C[w * g.sCn + m] = v0;
+        if (w + 1 < g.N) C[(w + 1) * g.sCn + m] = v1;
+      }
     }
 }
 
-template <class MF, int MT>
-__device__ __forceinline__ void q2_body(const GemmArgs<typename MF::T> &g, int bx, int by, int bz) {
+// Operand bases and the count of f of batch entry b (tri 2: the wide operand is that of pair b).
+template <class T>
+__device__ inline void wide_batch(const GemmArgs<T> &g, int b, const T *&A, const T *&B, T *&C, int &M) {
+  M = g.tri == 1 ? min(g.M, b + 1) : g.M;
+  A = g.A;
+  if (g.tri == 2) {
+    int i, j;
+    pair_of(b, i, j);
+    B = g.B + i * g.sAi + j * g.sAj;
+  } else {
+    B = g.B + b * g.sBb;
+  }
+  C = g.C + b * g.sCb;
+}
+
+template <class MF, int MT, bool SLOTS, bool ROWS>
+__device__ __forceinline__ void wide_body(const GemmArgs<typename MF::T> &g, int bx, int by, int bz) {
   const typename MF::T *A, *B;
   typename MF::T *C;
   int M;
-  gemm_batch(g, g.b0 + bz, A, B, C, M);
+  wide_batch(g, g.b0 + bz, A, B, C, M);
   const int m0 = by * 16 * MT, n0 = __builtin_amdgcn_readfirstlane(bx * 128 + int(threadIdx.x >> 6) * 32);
   if (m0 >= M || n0 >= g.N) return;  // no barrier follows
-  // only the row tiles below M
+  const bool pairs = SLOTS || g.sBk % 2 == 0;
+  // only the tiles below M
   const int live = (M - m0 + 15) / 16;
-  if (MT == 1 || live <= 1) q2_tiles<MF, 1>(g, A, B, C, M, m0, n0);
-  else if (MT == 2 || live == 2) q2_tiles<MF, MT >= 2 ? 2 : 1>(g, A, B, C, M, m0, n0);
-  else if (MT == 3 || live == 3) q2_tiles<MF, MT >= 3 ? 3 : 1>(g, A, B, C, M, m0, n0);
-  else q2_tiles<MF, MT>(g, A, B, C, M, m0, n0);
+  auto run = [&](auto h) {
+    constexpr int H = decltype(h)::value;
+    if (SLOTS || pairs) wide_tiles<MF, H, SLOTS, ROWS, true>(g, A, B, C, M, m0, n0);
+    else wide_tiles<MF, H, SLOTS, ROWS, false>(g, A, B, C, M, m0, n0);
+  };
+  if (MT == 1 || live <= 1) run(std::integral_constant<int, 1>());
+  else if (MT == 2 || live == 2) run(std::integral_constant<int, MT >= 2 ? 2 : 1>());
+  else if (MT == 3 || live == 3) run(std::integral_constant<int, MT >= 3 ? 3 : 1>());
+  else run(std::integral_constant<int, MT>());
 }
 
-template <class MF, int MT>
-__global__ __launch_bounds__(256) void zq_q2(const GemmArgs<typename MF::T> g) {
-  q2_body<MF, MT>(g, blockIdx.x, blockIdx.y, blockIdx.z);
+template <class MF, int MT, bool SLOTS, bool ROWS>
+__global__ __launch_bounds__(256) void zq_wide(const GemmArgs<typename MF::T> g) {
+  wide_body<MF, MT, SLOTS, ROWS>(g, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-template <class MF>
-int launch_q2(zq_ctx *ctx, const GemmArgs<typename MF::T> &g, int batch) {
-  const int mt = std::min(4, (g.M + 15) / 16);
-  zq_prof_begin(ctx, "ao2mo_q2");
+// Tiles of f a wave takes: all up to four, else the most even split.
+inline int wide_mt(int M) {
+  const int tiles = (M + 15) / 16, groups = (tiles + 3) / 4;
+  return (tiles + groups - 1) / groups;
+}
+
+// Q2 (f = j), batch over i.
+template <class T>
+GemmArgs<T> q2_args(const T *X, const T *c2, T *Y, int np, int m1, int m2, bool sym) {
+  GemmArgs<T> g{};
+  g.A = c2, g.B = X, g.sBb = np, g.mode = 1, g.npad = np, g.sXs = (long long)m1 * np;
+  g.C = Y, g.sCb = (long long)m2 * np * np, g.sCm = (long long)np * np, g.sCn = 1;
+  g.M = m2, g.N = np * np, g.K = np;
+  g.tri = sym ? 1 : 0;
+  return g;
+}
+// Q3 (f = b) and Q4 (f = a) of the pairs: Y of pair (i, j) at Y + (i m2 + j) np np, or of the p-th of the pairs i >= j.
+template <class T>
+GemmArgs<T> q3_args(const T *Y, const T *c4, T *W, int np, int m2, int m4, bool sym) {
+  GemmArgs<T> g{};
+  g.A = c4, g.B = Y, g.sBb = (long long)np * np, g.sBk = np;
+  g.C = W, g.sCb = (long long)np * m4, g.sCn = m4;
+  g.M = m4, g.N = np, g.K = np;
+  if (sym) g.tri = 2, g.sAi = (long long)m2 * np * np, g.sAj = (long long)np * np;
+  return g;
+}
+template <class T>
+GemmArgs<T> q4_args(const T *W, const T *c3, T *out, int np, int m3, int m4) {
+  GemmArgs<T> g{};
+  g.A = c3, g.B = W, g.sBb = (long long)np * m4, g.sBk = m4;
+  g.C = out, g.sCb = (long long)m3 * m4, g.sCm = m4;
+  g.M = m3, g.N = m4, g.K = np;
+  return g;
+}
+
+// The same two on 64 x 64 tiles, nu first: Q3 A = Y_ij [sig][nu], B = C3 [nu][a], out W[ij][sig][a]; Q4 A[a][sig] =
+// W[sig][a], B = C4 [sig][b], out[ij][a][b].
+template <class T>
+GemmArgs<T> q3_tile_args(const T *Y, const T *c3, T *W, int np, int m2, int m3, bool sym) {
+  GemmArgs<T> g{};
+  g.A = Y, g.sAb = (long long)np * np, g.sAm = np, g.sAk = 1;
+  g.B = c3, g.sBb = 0, g.sBk = m3, g.sBn = 1;
+  g.C = W, g.sCb = (long long)np * m3, g.sCm = m3, g.sCn = 1;
+  g.M = np, g.N = m3, g.K = np;
+  if (sym) g.tri = 2, g.sAi = (long long)m2 * np * np, g.sAj = (long long)np * np;
+  return g;
+}
+template <class T>
+GemmArgs<T> q4_tile_args(const T *W, const T *c4, T *out, int np, int m3, int m4) {
+  GemmArgs<T> g{};
+  g.A = W, g.sAb = (long long)np * m3, g.sAm = 1, g.sAk = m3;
+  g.B = c4, g.sBb = 0, g.sBk = m4, g.sBn = 1;
+  g.C = out, g.sCb = (long long)m3 * m4, g.sCm = m4, g.sCn = 1;
+  g.M = m3, g.N = m4, g.K = np;
+  return g;
+}
+
+template <class MF, bool SLOTS, bool ROWS>
+int launch_wide(zq_ctx *ctx, const GemmArgs<typename MF::T> &g, int batch, const char *name) {
+  const int mt = wide_mt(g.M);
+  zq_prof_begin(ctx, name);
   for (int b0 = 0; b0 < batch; b0 += kMaxGridZ) {
     const dim3 grid(unsigned((g.N + 127) / 128), unsigned((g.M + 16 * mt - 1) / (16 * mt)), unsigned(std::min(kMaxGridZ, batch - b0)));
     const auto s = batch_slice(g, b0);
     switch (mt) {
-      case 1: hipLaunchKernelGGL((zq_q2<MF, 1>), grid, dim3(256), 0, ctx->stream, s); break;
-      case 2: hipLaunchKernelGGL((zq_q2<MF, 2>), grid, dim3(256), 0, ctx->stream, s); break;
-      case 3: hipLaunchKernelGGL((zq_q2<MF, 3>), grid, dim3(256), 0, ctx->stream, s); break;
-      default: hipLaunchKernelGGL((zq_q2<MF, 4>), grid, dim3(256), 0, ctx->stream, s); break;
+      case 1: hipLaunchKernelGGL((zq_wide<MF, 1, SLOTS, ROWS>), grid, dim3(256), 0, ctx->stream, s); break;
+      case 2: hipLaunchKernelGGL((zq_wide<MF, 2, SLOTS, ROWS>), grid, dim3(256), 0, ctx->stream, s); break;
+      case 3: hipLaunchKernelGGL((zq_wide<MF, 3, SLOTS, ROWS>), grid, dim3(256), 0, ctx->stream, s); break;
+      default: hipLaunchKernelGGL((zq_wide<MF, 4, SLOTS, ROWS>), grid, dim3(256), 0, ctx->stream, s); break;
     }
   }
   zq_prof_end(ctx);
-  ZQ_LAUNCH_CHECK(ctx, "ao2mo_q2");
+  ZQ_LAUNCH_CHECK(ctx, name);
   return ZQ_OK;
 }
 
@@ -1051,25 +1162,25 @@ int upload(zq_ctx *ctx, const char *name, const std::vector<T> &h, T **d) {
 // same element conversions as the host staging, so the values are identical.
 template <class T>
 __device__ __forceinline__ void c_slices_body(const double *__restrict__ C, int n, int np, int m1, int m2, int m3,
-                                              int off3, T *__restrict__ c1, T *__restrict__ c2, bool c2t,
+                                              int off3, T *__restrict__ c1, T *__restrict__ c2, bool plain,
                                               T *__restrict__ c3, int mu) {
   for (int t = threadIdx.x; t < m1 + m2 + m3; t += blockDim.x) {
     if (t < m1) {
       c1[q1_c_index(mu, t, m1)] = mu < n ? T(C[size_t(mu) * n + t]) : T(0);
     } else if (t < m1 + m2) {
       const int j = t - m1;
-      c2[c2t ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = mu < n ? T(C[size_t(mu) * n + j]) : T(0);
+      c2[plain ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = mu < n ? T(C[size_t(mu) * n + j]) : T(0);
     } else {
       const int a = t - m1 - m2;
-      c3[size_t(mu) * m3 + a] = mu < n ? T(C[size_t(mu) * n + off3 + a]) : T(0);
+      c3[plain || sizeof(T) == 8 ? size_t(mu) * m3 + a : q1_c_index(mu, a, m3)] = mu < n ? T(C[size_t(mu) * n + off3 + a]) : T(0);
     }
   }
 }
 
 template <class T>
 __global__ void zq_c_slices(const double *__restrict__ C, int n, int np, int m1, int m2, int m3, int off3,
-                            T *__restrict__ c1, T *__restrict__ c2, bool c2t, T *__restrict__ c3) {
-  c_slices_body<T>(C, n, np, m1, m2, m3, off3, c1, c2, c2t, c3, blockIdx.x);  // one workgroup per row mu < np
+                            T *__restrict__ c1, T *__restrict__ c2, bool plain, T *__restrict__ c3) {
+  c_slices_body<T>(C, n, np, m1, m2, m3, off3, c1, c2, plain, c3, blockIdx.x);  // one workgroup per row mu < np
 }
 
 // y = x (n doubles; x may be pinned host memory)
@@ -1136,7 +1247,8 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
   // BF16X3 Q1 takes C1 split and transposed: C1h/C1l[i][mu], mu padded to a multiple of 32
   const int ldt = ((nb + 3) / 4) * 32;
   T *d1, *d2, *d3, *d4 = nullptr;
-  const bool c2t = precision == ZQ_PREC_BF16X3;  // its Q2 takes C2 transposed, the others' as q1_c_index lays it out
+  // BF16X3 takes C2 transposed and C3, C4 as plain matrices, FP64 C3 and C4; the others as q1_c_index lays them out
+  const bool plain = precision == ZQ_PREC_BF16X3;
   bf16 *d1h = nullptr, *d1l = nullptr;
   if constexpr (sizeof(T) == 4) {
     if (precision != ZQ_PREC_BF16X3) {
@@ -1159,7 +1271,7 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
       return zq_fail(ctx, ZQ_ERR_INVALID, "zq_mp2_noalloc: static scratch too small");
     ZQ_TRY(ctx, hipMemcpyAsync(dC, C, size_t(n) * n * 8, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(zq_c_slices<T>, dim3(unsigned(np)), dim3(256), 0, ctx->stream, dC, n, np, m1, m2, m3, d.off3, d1,
-                       d2, c2t, d3);
+                       d2, plain, d3);
     if (precision == ZQ_PREC_BF16X3)
       hipLaunchKernelGGL(zq_c1_split, dim3(unsigned(m1)), dim3(256), 0, ctx->stream, dC, n, m1, ldt, d1h, d1l);
     ZQ_LAUNCH_CHECK(ctx, "zq_c_slices");
@@ -1176,7 +1288,7 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     if (!d1 || !d2 || !d3 || (precision == ZQ_PREC_BF16X3 && (!d1h || !d1l)))
       return zq_fail(ctx, ZQ_ERR_OOM, "transform scratch C slices");
     hipLaunchKernelGGL(zq_c_slices<T>, dim3(unsigned(np)), dim3(256), 0, ctx->stream, C, n, np, m1, m2, m3, d.off3, d1,
-                       d2, c2t, d3);
+                       d2, plain, d3);
     if (precision == ZQ_PREC_BF16X3)
       hipLaunchKernelGGL(zq_c1_split, dim3(unsigned(m1)), dim3(256), 0, ctx->stream, C, n, m1, ldt, d1h, d1l);
     ZQ_LAUNCH_CHECK(ctx, "zq_c_slices");
@@ -1187,10 +1299,10 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
         h4(own4 ? size_t(np) * m4 : 0, T(0));
     for (int mu = 0; mu < n; ++mu) {
       for (int i = 0; i < m1; ++i) h1[q1_c_index(mu, i, m1)] = T(cf.q[0][size_t(mu) * n + i]);
-      for (int j = 0; j < m2; ++j) h2[c2t ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = T(cf.q[1][size_t(mu) * n + j]);
-      for (int a = 0; a < m3; ++a) h3[size_t(mu) * m3 + a] = T(cf.q[2][size_t(mu) * n + d.off3 + a]);
+      for (int j = 0; j < m2; ++j) h2[plain ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = T(cf.q[1][size_t(mu) * n + j]);
+      for (int a = 0; a < m3; ++a) h3[plain || sizeof(T) == 8 ? size_t(mu) * m3 + a : q1_c_index(mu, a, m3)] = T(cf.q[2][size_t(mu) * n + d.off3 + a]);
       if (own4)
-        for (int b = 0; b < m4; ++b) h4[size_t(mu) * m4 + b] = T(cf.q[3][size_t(mu) * n + d.off3 + b]);
+        for (int b = 0; b < m4; ++b) h4[plain || sizeof(T) == 8 ? size_t(mu) * m4 + b : q1_c_index(mu, b, m4)] = T(cf.q[3][size_t(mu) * n + d.off3 + b]);
     }
     if (int rc = upload(ctx, "C1", h1, &d1)) return rc;
     if (int rc = upload(ctx, "C2", h2, &d2)) return rc;
@@ -1265,28 +1377,13 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     zq_prof_end(ctx);
     ZQ_LAUNCH_CHECK(ctx, "ao2mo_q1");
   }
-  GemmArgs<T> g2{}, g3{}, g4{};
-  // Q2: batch over i; A = C2 (BF16X3: its transpose, m2 x np), B gathered from X, out Y[i][j][sig][nu] (j <= i if
-  // symmetric)
-  g2.A = d2, g2.sAb = 0, g2.sAm = np, g2.sAk = 1;
-  g2.B = X, g2.sBb = np, g2.mode = 1, g2.npad = np, g2.sXs = (long long)m1 * np;
-  g2.C = Y, g2.sCb = (long long)m2 * np * np, g2.sCm = (long long)np * np, g2.sCn = 1;
-  g2.M = m2, g2.N = np * np, g2.K = np;
-  g2.tri = sym ? 1 : 0;
-  // Q3: batch over (i,j) (the pairs i >= j if symmetric); A = Y_ij [sig][nu], B = C3 [nu][a], out W[ij][sig][a]
-  g3.A = Y, g3.sAb = (long long)np * np, g3.sAm = np, g3.sAk = 1;
-  g3.B = d3, g3.sBb = 0, g3.sBk = m3, g3.sBn = 1;
-  g3.C = W, g3.sCb = (long long)np * m3, g3.sCm = m3, g3.sCn = 1;
-  g3.M = np, g3.N = m3, g3.K = np;
-  if (sym) g3.tri = 2, g3.sAi = (long long)m2 * np * np, g3.sAj = (long long)np * np;
-  // Q4: batch over the same (i,j); A[a][sig] = W[sig][a], B = C4 [sig][b], out[ij][a][b]
-  g4.A = W, g4.sAb = (long long)np * m3, g4.sAm = 1, g4.sAk = m3;
-  g4.B = d4, g4.sBb = 0, g4.sBk = m4, g4.sBn = 1;
-  g4.C = O, g4.sCb = (long long)m3 * m4, g4.sCm = m4, g4.sCn = 1;
-  g4.M = m3, g4.N = m4, g4.K = np;
+  // Q2: batch over i; C2 (BF16X3: its transpose, m2 x np) and the gathered X, out Y[i][j][sig][nu] (j <= i if symmetric)
+  GemmArgs<T> g2 = q2_args(X, d2, Y, np, m1, m2, sym);
   *packed = sym;
   if constexpr (sizeof(T) == 4) {
     if (precision == ZQ_PREC_BF16X3) {
+      const GemmArgs<T> g3 = q3_tile_args<T>(Y, d3, W, np, m2, m3, sym), g4 = q4_tile_args<T>(W, d4, O, np, m3, m4);
+      g2.sAm = np, g2.sAk = 1;
       if (int rc = launch_gemm_bf16x3(ctx, g2, m1, "ao2mo_q2")) return rc;
       if (int rc = launch_gemm_bf16x3(ctx, g3, nij, "ao2mo_q3")) return rc;
       if (int rc = launch_gemm_bf16x3(ctx, g4, nij, "ao2mo_q4")) return rc;
@@ -1294,10 +1391,14 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
       return ZQ_OK;
     }
   }
-  if (int rc = launch_q2<MF>(ctx, g2, m1)) return rc;
-  if (int rc = launch_gemm<MF>(ctx, g3, nij, "ao2mo_q3")) return rc;
-  // Q4 on the tile kernel in every precision (no library GEMM in the transform)
-  if (int rc = launch_gemm<MF>(ctx, g4, nij, "ao2mo_q4")) return rc;
+  if (int rc = launch_wide<MF, true, true>(ctx, g2, m1, "ao2mo_q2")) return rc;
+  if constexpr (sizeof(T) == 4) {
+    if (int rc = launch_wide<MF, false, false>(ctx, q3_args<T>(Y, d4, W, np, m2, m4, sym), nij, "ao2mo_q3")) return rc;
+    if (int rc = launch_wide<MF, false, true>(ctx, q4_args<T>(W, d3, O, np, m3, m4), nij, "ao2mo_q4")) return rc;
+  } else {
+    if (int rc = launch_gemm<MF>(ctx, q3_tile_args<T>(Y, d3, W, np, m2, m3, sym), nij, "ao2mo_q3")) return rc;
+    if (int rc = launch_gemm<MF>(ctx, q4_tile_args<T>(W, d4, O, np, m3, m4), nij, "ao2mo_q4")) return rc;
+  }
   *d_out = O;
   return ZQ_OK;
 }
@@ -1524,6 +1625,16 @@ __global__ __launch_bounds__(256, (q1_min_waves<MF, 1>())) void zq_group_q1(cons
   q1_body<MF, 1, E>(J.eri, J.c1, J.o, J.nb, J.np, J.X, l - t * gx, t % J.groups, t / J.groups);
 }
 
+// Stage q of Q2, Q3, Q4 (0 .. 2).
+template <class MF, class E, int MT, bool SLOTS, bool ROWS>
+__global__ __launch_bounds__(256) void zq_group_wide(const GJob<typename MF::T, E> *__restrict__ jobs,
+                                                     const int *__restrict__ start, int nmol, int q) {
+  const int m = group_find(start, nmol, blockIdx.x);
+  const GemmArgs<typename MF::T> g = jobs[m].g[q];
+  const int l = int(blockIdx.x) - start[m], gx = (g.N + 127) / 128, gy = (g.M + 16 * MT - 1) / (16 * MT), t = l / gx;
+  wide_body<MF, MT, SLOTS, ROWS>(g, l - t * gx, t % gy, t / gy);
+}
+
 template <class MF, class E>
 __global__ __launch_bounds__(256, 2) void zq_group_gemm(const GJob<typename MF::T, E> *__restrict__ jobs,
                                                      const int *__restrict__ start, int nmol, int q) {
@@ -1531,15 +1642,6 @@ __global__ __launch_bounds__(256, 2) void zq_group_gemm(const GJob<typename MF::
   const GemmArgs<typename MF::T> g = jobs[m].g[q];
   const int l = int(blockIdx.x) - start[m], gx = (g.N + 63) / 64, gy = (g.M + 63) / 64, t = l / gx;
   gemm_body<MF>(g, l - t * gx, t % gy, t / gy);
-}
-
-template <class MF, class E>
-__global__ __launch_bounds__(256) void zq_group_q2(const GJob<typename MF::T, E> *__restrict__ jobs,
-                                                   const int *__restrict__ start, int nmol) {
-  const int m = group_find(start, nmol, blockIdx.x);
-  const GemmArgs<typename MF::T> g = jobs[m].g[0];
-  const int l = int(blockIdx.x) - start[m], gx = (g.N + 127) / 128, gy = (g.M + 15) / 16, t = l / gx;
-  q2_body<MF, 1>(g, l - t * gx, t % gy, t / gy);
 }
 
 template <class T, class E>
@@ -1628,34 +1730,17 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
       J.O = (T *)take(pr * v * v * sizeof(T));
       J.partial = (double *)take(pr * 8 + 8);
       J.out = d_out + k;
-      // Q2: batch over i; A = C2, B gathered from X, out Y[i][j][sig][nu], j <= i
-      GemmArgs<T> &g2 = J.g[0];
-      g2 = GemmArgs<T>{};
-      g2.A = J.c2, g2.sAb = 0, g2.sAm = J.np, g2.sAk = 1;
-      g2.B = J.X, g2.sBb = J.np, g2.mode = 1, g2.npad = J.np, g2.sXs = (long long)o * np;
-      g2.C = Y, g2.sCb = (long long)o * np * np, g2.sCm = (long long)np * np, g2.sCn = 1;
-      g2.M = J.o, g2.N = J.np * J.np, g2.K = J.np, g2.tri = 1;
-      // Q3: batch over the pairs i >= j; A = Y_ij [sig][nu], B = C3 [nu][a], out W[p][sig][a]
-      GemmArgs<T> &g3 = J.g[1];
-      g3 = GemmArgs<T>{};
-      g3.A = Y, g3.sAb = (long long)np * np, g3.sAm = J.np, g3.sAk = 1;
-      g3.B = J.c3, g3.sBb = 0, g3.sBk = J.v, g3.sBn = 1;
-      g3.C = W, g3.sCb = (long long)np * v, g3.sCm = J.v, g3.sCn = 1;
-      g3.M = J.np, g3.N = J.v, g3.K = J.np;
-      g3.tri = 2, g3.sAi = (long long)o * np * np, g3.sAj = (long long)np * np;
-      // Q4: batch over the pairs; A[a][sig] = W[sig][a], B = C3 [sig][b], out[p][a][b]
-      GemmArgs<T> &g4 = J.g[2];
-      g4 = GemmArgs<T>{};
-      g4.A = W, g4.sAb = (long long)np * v, g4.sAm = 1, g4.sAk = J.v;
-      g4.B = J.c3, g4.sBb = 0, g4.sBk = J.v, g4.sBn = 1;
-      g4.C = J.O, g4.sCb = (long long)v * v, g4.sCm = J.v, g4.sCn = 1;
-      g4.M = J.v, g4.N = J.v, g4.K = J.np;
+      const GemmArgs<T> &g2 = J.g[0] = q2_args(J.X, J.c2, Y, J.np, J.o, J.o, true);
+      constexpr bool wide = sizeof(T) == 4;
+      const GemmArgs<T> &g3 = J.g[1] = wide ? q3_args<T>(Y, J.c3, W, J.np, J.o, J.v, true) : q3_tile_args<T>(Y, J.c3, W, J.np, J.o, J.v, true);
+      const GemmArgs<T> &g4 = J.g[2] = wide ? q4_args<T>(W, J.c3, J.O, J.np, J.v, J.v) : q4_tile_args<T>(W, J.c3, J.O, J.np, J.v, J.v);
+      constexpr int cols = wide ? 128 : 64;
       const long long cnt[GS_COUNT] = {
           J.np,
           (long long)J.Nb * J.nb * J.groups * 2,
           (long long)((g2.N + 127) / 128) * ((g2.M + 15) / 16) * J.o,
-          (long long)((g3.N + 63) / 64) * ((g3.M + 63) / 64) * J.pairs,
-          (long long)((g4.N + 63) / 64) * ((g4.M + 63) / 64) * J.pairs,
+          (long long)((g3.N + cols - 1) / cols) * ((g3.M + 63) / 64) * J.pairs,
+          (long long)((g4.N + cols - 1) / cols) * ((g4.M + 63) / 64) * J.pairs,
           (long long)J.pairs};
       for (int s = 0; s < GS_COUNT; ++s) {
         const long long next = start[size_t(s) * (nm + 1) + k] + cnt[s];
@@ -1675,9 +1760,14 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
     auto total = [&](int s) { return unsigned(start[size_t(s) * (nm + 1) + nm]); };
     hipLaunchKernelGGL((zq_group_slices<T, E>), dim3(total(GS_SLICES)), dim3(256), 0, stream, d_jobs, st(GS_SLICES), nm);
     hipLaunchKernelGGL((zq_group_q1<MF, E>), dim3(total(GS_Q1)), dim3(256), 0, stream, d_jobs, st(GS_Q1), nm);
-    hipLaunchKernelGGL((zq_group_q2<MF, E>), dim3(total(GS_Q2)), dim3(256), 0, stream, d_jobs, st(GS_Q2), nm);
-    for (int q = 1; q < 3; ++q)
-      hipLaunchKernelGGL((zq_group_gemm<MF, E>), dim3(total(GS_Q2 + q)), dim3(256), 0, stream, d_jobs, st(GS_Q2 + q), nm, q);
+    hipLaunchKernelGGL((zq_group_wide<MF, E, 1, true, true>), dim3(total(GS_Q2)), dim3(256), 0, stream, d_jobs, st(GS_Q2), nm, 0);
+    if constexpr (sizeof(T) == 4) {
+      hipLaunchKernelGGL((zq_group_wide<MF, E, 4, false, false>), dim3(total(GS_Q3)), dim3(256), 0, stream, d_jobs, st(GS_Q3), nm, 1);
+      hipLaunchKernelGGL((zq_group_wide<MF, E, 4, false, true>), dim3(total(GS_Q4)), dim3(256), 0, stream, d_jobs, st(GS_Q4), nm, 2);
+    } else {
+      for (int q = 1; q < 3; ++q)
+        hipLaunchKernelGGL((zq_group_gemm<MF, E>), dim3(total(GS_Q2 + q)), dim3(256), 0, stream, d_jobs, st(GS_Q2 + q), nm, q);
+    }
     hipLaunchKernelGGL((zq_group_pairs<T, E>), dim3(total(GS_PAIRS)), dim3(256), 0, stream, d_jobs, st(GS_PAIRS), nm);
     hipLaunchKernelGGL((zq_group_sum<T, E>), dim3(unsigned(nm)), dim3(64), 0, stream, d_jobs);
     if (hipGetLastError() != hipSuccess) {
