@@ -479,7 +479,7 @@ void launch_step(zq_batch *b, int mode, int diis, double thr, int maxit) {
 
 int enqueue_iteration(zq_batch *b, int diis, double thr, int maxit) {
   BTRY(b, zq_jk_group(b->stream, b->eri, b->d_items, b->nitems, b->ws, 0.5, b->rec, b->d_jkm, b->d_done, b->d_ptr,
-                      b->d_idx, b->d_blk, b->nblk, b->ws, b->ws));
+                      b->d_idx, b->d_blk, b->nblk, b->ws, b->ws, b->mp_max, b->chunk));
   launch_step(b, kStepIter, diis, thr, maxit);
   hipLaunchKernelGGL(k_batch_count, dim3(1), dim3(256), 0, b->stream, b->d_done, int(b->mols.size()), b->d_count);
   BTRY(b, hipGetLastError());
@@ -584,7 +584,7 @@ int zq_batch_autotune(zq_batch *b, int chosen[2]) {
     if (int rc = build_plan(b, ch)) return rc;
     const float ms = time_it([&] {
       (void)zq_jk_group(b->stream, b->eri, b->d_items, b->nitems, b->ws, 0.5, b->rec, b->d_jkm, b->d_done, b->d_ptr,
-                        b->d_idx, b->d_blk, b->nblk, b->ws, b->ws);
+                        b->d_idx, b->d_blk, b->nblk, b->ws, b->ws, b->mp_max, b->chunk);
     });
     if (ms < best) best = ms, best_chunk = ch;
   }

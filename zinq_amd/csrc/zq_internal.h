@@ -259,10 +259,11 @@ constexpr int kZqMaxDevices = 64;
 // with `device` current (zq_transform.hip).
 void zq_noalloc_setup(int device);
 // Grouped J/K on `stream`: F = H + G(P) (x_exch) for every molecule of a grouped plan whose done flag
-// is 0.  blk[g] = (molecule, output block) for the nblk CSR rows.  Returns the launch status.
+// is 0.  blk[g] = (molecule, output block) for the nblk CSR rows; ld_max: the largest leading dimension of a P;
+// chunk: the plan's item size (0: each molecule's own).  Returns the launch status.
 hipError_t zq_jk_group(hipStream_t stream, const double *eri, const JKItem *items, int nitems, const double *P,
                        double x_exch, double *rec, const JKMol *mols, const int *done, const int *csr_ptr,
-                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F);
+                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F, int ld_max, int chunk);
 // Packs canonical chemist ERIs (zq_eri_load_packed layout) into 8x8 AO-block quartets (zq_context.hip).
 __global__ __launch_bounds__(256) void zq_pack_quartets(const double *__restrict__ canon, double *__restrict__ out, int n,
                                                         size_t nquartets);

@@ -121,23 +121,31 @@ __device__ inline double sum8_scatter_high(const double (&v)[8], int lane) {
 }
 
 // One workgroup (4 waves) per work item; wave w handles ket rows r = 2w, 2w+1 of every quartet for all
-// 64 bra pairs (lane = bra pair (p,q)), loading its two 512-byte rows straight into registers.  While a
-// quartet is being contracted, the next quartet's rows and the per-lane density values it needs are
-// already in flight (they are issued before any load the current contraction waits on, so the in-order
-// vmcnt wait never stalls on them); density values common to the wave come in through scalar loads.
+// 64 bra pairs (lane = bra pair (p,q)), loading its two 512-byte rows straight into registers.  The rows of P
+// that the item's bra block needs are staged in LDS first (LONG; items of one quartet or two read them in place,
+// which is quicker for them); density values common to the wave come in through scalar loads.  So the quartets
+// are a long item's only vector loads, and the in-order wait for one of them waits for no later one.  They are
+// kept two quartets ahead (3 in the 4-byte form) in a ring of register sets that the unrolled loop walks: nothing is
+// copied from set to set (a copy of a set in flight waits for it), and the loads are unconditional, since a path
+// without them would make every wait count for the fewer in flight; past the item's end the buffer descriptor's
+// bound makes them return 0 without a fetch.
 // Cross-wave sums (K[p,s], K[q,s] at the end of a bs run, J[p,q] at the end of the item) go through
 // LDS in a fixed order.
+// Bound by memory for long items.  Against loads of P in the loop, a conditional prefetch and sets copied along, which
+// together waited for every load of a step within it (n = 192: 4.2 TB/s): n = 192 322 -> 309 us, n = 144 104 -> 97, six
+// densities at n = 93 180 -> 131, 96 molecules n <= 72 197 -> 184, n = 96 in FP32 28.6 -> 18.8, n = 72 14.5 -> 12.6.
 // GROUP: the item's molecule selects the quartets, P and its leading dimension from mols[], and the
 // item is skipped once done[molecule] is set.
 // MULTI: blockIdx.x is the density d (P + d * pstride, records + d * rstride) and blockIdx.y the item,
 // so the densities of one item run back to back and share its quartet reads through the caches.
-template <class E, bool GROUP, bool MULTI = false>
+template <class E, bool GROUP, bool MULTI, bool LONG>
 __global__ __launch_bounds__(256) void zq_jk_records(const E *__restrict__ eri, const JKItem *__restrict__ items,
                                                      int nitems, const double *__restrict__ P, int npad, double xexch,
                                                      double *__restrict__ rec, const int *__restrict__ skip,
                                                      const JKMol *__restrict__ mols, const int *__restrict__ done,
-                                                     long long pstride = 0, long long rstride = 0) {
+                                                     long long pstride, long long rstride) {
   __shared__ double red[2][4][2][64];  // two buffers, so each cross-wave sum needs one barrier
+  extern __shared__ __attribute__((aligned(16))) double Ps[];  // rows of P: block bp, block bq (jk_lds)
   const int item_id = MULTI ? blockIdx.y : blockIdx.x;
   if (MULTI) {
     P += blockIdx.x * pstride;
@@ -158,12 +166,10 @@ __global__ __launch_bounds__(256) void zq_jk_records(const E *__restrict__ eri, 
 
   const int p = lane >> 3, q = lane & 7;
   const int Pg = bp * 8 + p, Qg = bq * 8 + q;
-  // fI halves the bra pairs counted twice (p == q on a diagonal bra block).  It is a power of two and
-  // constant per lane, so it is folded into this lane's density values (exactly) rather than into every
-  // integral; Jbra, which takes no such value, is scaled once at the end.
+  // fI halves the bra pairs counted twice (p == q on a diagonal bra block).  It is a power of two and constant per
+  // lane, so it scales the sums instead of every integral, exactly.
   const double fI = (bp == bq && p == q) ? 0.5 : 1.0;
-  const double *Prow = P + size_t(Pg) * npad, *Qrow = P + size_t(Qg) * npad;
-  const double Ppq = Prow[Qg] * fI;
+  const double Ppq = P[size_t(Pg) * npad + Qg] * fI;
 
   int bs = 0, kk = k0;
   for (;; ++bs) {
@@ -175,55 +181,55 @@ __global__ __launch_bounds__(256) void zq_jk_records(const E *__restrict__ eri, 
 
   double *out = rec + size_t(rec0) * 64;
   int rb = 0;  // buffer of red for the next cross-wave sum
-  // this wave's two rows of the item's first quartet: element (r*8+s)*64 + lane, r = 2w + rr
-  const E *src = eri + (size_t(Ib) * (Ib + 1) / 2 + size_t(k0)) * ZQ_QUARTET + (2 * wave) * 512 + lane;
-  double Jbra = 0.0;
-  // quartets in flight ahead of the contraction, kept in their stored type (4-byte ones leave room for 4)
-  constexpr int D = sizeof(E) == 4 ? 4 : 2;
-  double Kps[8], Kqs[8], Pp_s[8], Pq_s[8], cur[16];
-  E pf[D][16];
-  double Pr_cur[4], Pr_nxt[4];  // Prow[br*8+r], Qrow[br*8+r] for the wave's two rows
+  // quartets in flight ahead of the contraction, kept in their stored type
+  constexpr int D = !LONG ? 0 : sizeof(E) == 4 ? 3 : 2, R = D + 1;
+  E ring[R][16];
+  // this wave's two rows of the item's quartets: element (r*8+s)*64 + lane, r = 2w + rr
+  const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<E *>(eri) + (size_t(Ib) * (Ib + 1) / 2 + size_t(k0)) * ZQ_QUARTET, 0, (k1 - k0) * int(ZQ_QUARTET * sizeof(E)),
+      0x00027000);
+  int at = (2 * wave * 512 + lane) * int(sizeof(E));  // byte offset of the next quartet to load
+  auto load = [&](E(&set)[16]) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {  // non-temporal: the stream is read once per build
+      if constexpr (sizeof(E) == 8) {
+        typedef unsigned u2 __attribute__((ext_vector_type(2)));
+        const u2 v = __builtin_amdgcn_raw_buffer_load_b64(src, at + j * 512, 0, 2);
+        set[j] = __hiloint2double(int(v.y), int(v.x));
+      } else {
+        set[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(src, at + j * 256, 0, 2));
+      }
+    }
+    at += int(ZQ_QUARTET * sizeof(E));
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(ring[d]);
+
+  // rows of P as far as the item's kets reach (r, s blocks up to bp)
+  const int ldp = npad + 2;
+  if (LONG) {
+    const int row = tid >> 4;
+    const double *from = P + size_t((row < 8 ? bp : bq - 1) * 8 + row) * npad;
+    for (int c = tid & 15; c < 8 * (bp + 1); c += 16) Ps[row * ldp + c] = from[c];
+    __syncthreads();
+  }
+  const double *const Pp = LONG ? Ps + p * ldp : P + size_t(Pg) * npad, *const Pq = LONG ? Ps + (8 + q) * ldp : P + size_t(Qg) * npad;
+
+  double Jbra = 0.0, Kps[8], Kqs[8], Pp_s[8], Pq_s[8];
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
     Kps[s] = Kqs[s] = 0.0;
-    Pp_s[s] = Prow[bs * 8 + s] * fI;
-    Pq_s[s] = Qrow[bs * 8 + s] * fI;
+    Pp_s[s] = Pp[bs * 8 + s];
+    Pq_s[s] = Pq[bs * 8 + s];
   }
-#pragma unroll
-  for (int rr = 0; rr < 2; ++rr) {
-    Pr_cur[2 * rr] = Prow[br * 8 + 2 * wave + rr] * fI;
-    Pr_cur[2 * rr + 1] = Qrow[br * 8 + 2 * wave + rr] * fI;
-  }
-  // the quartet stream is read once per build: non-temporal loads, D quartets ahead of the contraction
-#pragma unroll
-  for (int j = 0; j < 16; ++j) cur[j] = double(__builtin_nontemporal_load(src + j * 64));
-#pragma unroll
-  for (int d = 0; d + 1 < D; ++d)
-    if (k0 + 1 + d < k1) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) pf[d][j] = __builtin_nontemporal_load(src + size_t(1 + d) * ZQ_QUARTET + j * 64);
-    }
 
-  for (int k = k0; k < k1; ++k) {
-    if (k + D < k1) {
-      const E *nxd = src + size_t(k + D - k0) * ZQ_QUARTET;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) pf[D - 1][j] = __builtin_nontemporal_load(nxd + j * 64);
-    }
+  auto contract = [&](int k, double(&cur)[16]) {
     const bool run_end = (br + 1 > (bs <= bq ? bp : bp - 1));
     int nbs = bs, nbr = br + 1;
     if (run_end) {
       ++nbs;
       while (nbs <= bp && zq_run_len(bp, bq, nbs) <= 0) ++nbs;
       nbr = nbs;
-    }
-    if (k + 1 < k1) {
-#pragma unroll
-      for (int rr = 0; rr < 2; ++rr) {
-        Pr_nxt[2 * rr] = Prow[nbr * 8 + 2 * wave + rr] * fI;
-        Pr_nxt[2 * rr + 1] = Qrow[nbr * 8 + 2 * wave + rr] * fI;
-      }
-      // quartet k + 1 is already in flight (pf[0])
     }
     const int Jb = zq_bpair(br, bs);
     const bool diagJ = (br == bs), diagQ = (Jb == Ib);
@@ -243,7 +249,7 @@ __global__ __launch_bounds__(256) void zq_jk_records(const E *__restrict__ eri, 
 #pragma unroll
     for (int rr = 0; rr < 2; ++rr) {
       const int r = 2 * wave + rr;
-      const double Pp_r = Pr_cur[2 * rr], Pq_r = Pr_cur[2 * rr + 1];
+      const double Pp_r = Pp[br * 8 + r], Pq_r = Pq[br * 8 + r];
       const double *Prs = P + size_t(br * 8 + r) * npad + bs * 8;  // wave-uniform
       double apr = 0.0, aqr = 0.0;
 #pragma unroll
@@ -256,8 +262,8 @@ __global__ __launch_bounds__(256) void zq_jk_records(const E *__restrict__ eri, 
         aqr += Pp_s[s] * a;
         apr += Pq_s[s] * a;
       }
-      accpr[rr] = apr;
-      accqr[rr] = aqr;
+      accpr[rr] = apr * fI;
+      accqr[rr] = aqr * fI;
     }
     // J of the wave's 16 ket pairs (r, s), over the 64 bra pairs: lane l holds pair l >> 2
     const double tj = sum16_scatter(jt, lane);
@@ -269,6 +275,8 @@ __global__ __launch_bounds__(256) void zq_jk_records(const E *__restrict__ eri, 
     out += 192;
 
     if (run_end || k == k1 - 1) {
+#pragma unroll
+      for (int s = 0; s < 8; ++s) Kps[s] *= fI, Kqs[s] *= fI;
       // buffer rb was last read by wave 0 before the previous cross-wave barrier, so it is free
       red[rb][wave][0][lane] = sum8_scatter_low(Kps, lane);   // K[p, bs*8+s], s = q
       red[rb][wave][1][lane] = sum8_scatter_high(Kqs, lane);  // K[q, bs*8+s], s = p
@@ -286,26 +294,44 @@ __global__ __launch_bounds__(256) void zq_jk_records(const E *__restrict__ eri, 
       if (run_end && k + 1 < k1) {
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-          Pp_s[s] = Prow[nbs * 8 + s] * fI;
-          Pq_s[s] = Qrow[nbs * 8 + s] * fI;
+          Pp_s[s] = Pp[nbs * 8 + s];
+          Pq_s[s] = Pq[nbs * 8 + s];
         }
       }
     }
     bs = nbs, br = nbr;
+  };
+  for (int k = k0; k < k1; k += R)
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      cur[j] = double(pf[0][j]);
+    for (int u = 0; u < R; ++u) {
+      load(ring[(u + D) % R]);
+      if (k + u < k1) {
+        if constexpr (sizeof(E) == 8) {
+          contract(k + u, ring[u]);
+        } else {
+          double cur[16];
 #pragma unroll
-      for (int d = 0; d + 1 < D; ++d) pf[d][j] = pf[d + 1][j];
+          for (int j = 0; j < 16; ++j) cur[j] = double(ring[u][j]);
+          contract(k + u, cur);
+        }
+      }
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) Pr_cur[j] = Pr_nxt[j];
-  }
   red[rb][wave][0][lane] = Jbra * fI;
   __syncthreads();
   if (wave == 0)
     out[lane] = 2.0 * (((red[rb][0][0][lane] + red[rb][1][0][lane]) + red[rb][2][0][lane]) + red[rb][3][0][lane]);
 }
+
+// Dynamic LDS of zq_jk_records for leading dimension npad of P (npad <= 736: larger ERI sets fit no card).
+inline size_t jk_lds(int npad, bool lng) { return lng ? 16 * size_t(npad + 2) * sizeof(double) : 0; }
+
+// Quartets per work item, for nq quartets.  Long items read few quartets twice over (records, rows of P) and keep
+// loads in flight; short ones keep every compute unit busy.  Records and their sum, us, items of 1 / 4 / 8 / 16:
+// n = 56 (406 quartets) 14 / 18 / 21 / 28, n = 72 (1035) 22 / 24 / 23 / 31, n = 80 (1540) 27 / 25 / 24 / 33, n = 96 (3081)
+// - / 40 / 35 / 36, n = 128 (9316) - / 93 / 80 / 90, n = 144 (14706) - / 137 / 122 / 118, n = 192 (45150) records
+// alone - / 362 / 311 / 309.
+inline int jk_chunk(size_t nq) { return nq < 1536 ? 1 : nq < 14000 ? 8 : 16; }
+inline bool jk_long(int chunk) { return chunk >= 4; }
 
 // F block (x >= y) = H + sum of records aimed at (x,y) + transposed records aimed at (y,x).  kRedWaves
 // waves take contiguous shares of the block's record list with 8 loads in flight each; the shares are
@@ -394,7 +420,7 @@ __global__ __launch_bounds__(64 * kRedWaves) void zq_jk_reduce(const double *__r
 
 // Host-side work plan: work items, the exact record sequence each emits, and the per-output-block CSR.
 void zq_jk_plan(int Nb, size_t nq, int chunk, JKPlan &plan) {
-  const int CH = chunk > 0 ? chunk : int(std::max<size_t>(1, std::min<size_t>(16, nq / 3072)));
+  const int CH = chunk > 0 ? chunk : jk_chunk(nq);
   std::vector<JKItem> &items = plan.items;
   items.clear();
   std::vector<std::pair<int, int>> tgt;
@@ -531,15 +557,17 @@ int zq_build_jk_plan(zq_ctx *ctx) {
 namespace {
 int zq_jk_records_device(zq_ctx *ctx, const double *dP, double x_exch, const int *skip, bool f32) {
   if (f32 && !ctx->eri32) return zq_fail(ctx, ZQ_ERR_STATE, "zq_fock_jk_device: no FP32 ERI copy");
+  const bool lng = jk_long(jk_chunk(ctx->nquartets));
+  const size_t lds = jk_lds(ctx->npad, lng);
   zq_prof_begin(ctx, f32 ? "jk_records32" : "jk_records");
   if (f32)
-    hipLaunchKernelGGL((zq_jk_records<float, false>), dim3(unsigned(ctx->nitems)), dim3(256), 0, ctx->stream,
-                       ctx->eri32, ctx->d_items, ctx->nitems, dP, ctx->npad, x_exch, ctx->d_records, skip, nullptr,
-                       nullptr);
+    hipLaunchKernelGGL((lng ? zq_jk_records<float, false, false, true> : zq_jk_records<float, false, false, false>),
+                       dim3(unsigned(ctx->nitems)), dim3(256), lds, ctx->stream, ctx->eri32, ctx->d_items, ctx->nitems, dP, ctx->npad,
+                       x_exch, ctx->d_records, skip, nullptr, nullptr, 0LL, 0LL);
   else
-    hipLaunchKernelGGL((zq_jk_records<double, false>), dim3(unsigned(ctx->nitems)), dim3(256), 0, ctx->stream,
-                       ctx->eri, ctx->d_items, ctx->nitems, dP, ctx->npad, x_exch, ctx->d_records, skip, nullptr,
-                       nullptr);
+    hipLaunchKernelGGL((lng ? zq_jk_records<double, false, false, true> : zq_jk_records<double, false, false, false>),
+                       dim3(unsigned(ctx->nitems)), dim3(256), lds, ctx->stream, ctx->eri, ctx->d_items, ctx->nitems, dP, ctx->npad,
+                       x_exch, ctx->d_records, skip, nullptr, nullptr, 0LL, 0LL);
   zq_prof_end(ctx);
   ZQ_LAUNCH_CHECK(ctx, "zq_jk_records");
   return ZQ_OK;
@@ -565,9 +593,11 @@ int zq_fock_jk_device(zq_ctx *ctx, const double *dP, const double *dH, double x_
 
 hipError_t zq_jk_group(hipStream_t stream, const double *eri, const JKItem *items, int nitems, const double *P,
                        double x_exch, double *rec, const JKMol *mols, const int *done, const int *csr_ptr,
-                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F) {
-  hipLaunchKernelGGL((zq_jk_records<double, true>), dim3(unsigned(nitems)), dim3(256), 0, stream, eri, items, nitems, P,
-                     0, x_exch, rec, nullptr, mols, done);
+                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F, int ld_max, int chunk) {
+  const bool lng = jk_long(chunk);
+  hipLaunchKernelGGL((lng ? zq_jk_records<double, true, false, true> : zq_jk_records<double, true, false, false>),
+                     dim3(unsigned(nitems)), dim3(256), jk_lds(ld_max, lng), stream, eri, items, nitems, P, 0, x_exch, rec, nullptr,
+                     mols, done, 0LL, 0LL);
   hipLaunchKernelGGL(zq_jk_reduce<true>, dim3(unsigned(nblk)), dim3(64 * kRedWaves), 0, stream, rec, csr_ptr, csr_idx, H, 0, F,
                      nullptr, 0, mols, blk, done);
   return hipGetLastError();
@@ -645,10 +675,11 @@ extern "C" int zq_fock_jk_multi(zq_ctx *ctx, const double *H, const double *P, s
   zq_pad(ctx, src, ndens, n, np, dP);
   if (H) zq_pad(ctx, src + ndens * nn, 1, n, n, ctx->d_H);
   ZQ_LAUNCH_CHECK(ctx, "k_pad");
+  const bool lng = jk_long(jk_chunk(ctx->nquartets));
   zq_prof_begin(ctx, "jk_records");
-  hipLaunchKernelGGL((zq_jk_records<double, false, true>), dim3(unsigned(ndens), unsigned(ctx->nitems)), dim3(256), 0,
-                     ctx->stream, ctx->eri, ctx->d_items, ctx->nitems, dP, np, x_exch, dR, nullptr, nullptr, nullptr,
-                     (long long)pstride, (long long)rstride);
+  hipLaunchKernelGGL((lng ? zq_jk_records<double, false, true, true> : zq_jk_records<double, false, true, false>),
+                     dim3(unsigned(ndens), unsigned(ctx->nitems)), dim3(256), jk_lds(ctx->npad, lng), ctx->stream, ctx->eri, ctx->d_items,
+                     ctx->nitems, dP, np, x_exch, dR, nullptr, nullptr, nullptr, (long long)pstride, (long long)rstride);
   zq_prof_end(ctx);
   ZQ_LAUNCH_CHECK(ctx, "zq_jk_records (multi)");
   zq_prof_begin(ctx, "jk_reduce");
