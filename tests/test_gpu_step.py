@@ -61,3 +61,28 @@ def test_scf_step_ghf(ctx):
     ro = O.scf(H, S, g, VN, s.nel // 2)
     assert ctx.last_scf_driver() == "device"
     assert r["E"] == pytest.approx(ro["E"], abs=1e-10)
+
+
+@pytest.mark.parametrize("n,diis", [(80, 16), (81, 3), (81, 16)])
+def test_scf_launches(ctx, n, diis):
+    """The multi-launch iteration with n a multiple of 16 (wide tile loads) and one above it (a last tile of one row
+    and column), with short and full histories, on a positive two-electron part weak enough for SCF to settle."""
+    rng = np.random.default_rng(n)
+    o = n // 5
+    Q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+    H = (Q * np.concatenate([np.linspace(-20.0, -2.0, o), np.linspace(0.5, 4.0, n - o)])) @ Q.T
+    H = 0.5 * (H + H.T)
+    S = np.eye(n) + 0.002 * (lambda a: a + a.T)(rng.standard_normal((n, n)))
+    g = 0.0
+    for _ in range(3):
+        b = rng.standard_normal((n, n))
+        b = 0.025 * (b + b.T)
+        g = g + b[:, None, :, None] * b[:, None, :]
+    ro = O.scf(H, S, g, 1.5, o, diis=diis, threshold=1e-8)
+    ctx.eri_load(g)
+    for fock in ("fp64", "fp32"):
+        r = ctx.scf(H, S, 1.5, o, diis=diis, threshold=1e-8, device=True, fock_precision=fock)
+        print(f"n={n} diis={diis} {fock}: dE {r['E'] - ro['E']:+.1e} it {r['iterations']}/{ro['iterations']}", flush=True)
+        assert ctx.last_scf_driver() == "device"
+        assert abs(r["iterations"] - ro["iterations"]) <= 1
+        assert r["E"] == pytest.approx(ro["E"], abs=1e-10)

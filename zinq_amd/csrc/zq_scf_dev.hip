@@ -164,11 +164,13 @@ __global__ __launch_bounds__(256) void k_store_density(const double *__restrict_
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
+inline int tiles_of(int n) { return (n + 15) / 16; }
+
 struct Dev {
   zq_ctx *ctx;
   int n;
   size_t nn;
-  double *S, *X, *XT, *C, *T, *Fp, *W, *FP, *FPS, *Pn, *Fh, *Eh, *part, *scal, *coef, *eig, *offd;
+  double *S, *X, *XT, *C, *T, *Fp, *W, *FP, *FPS, *Pn, *Fh, *Eh, *part, *dots, *rms, *scal, *coef, *eig, *offd;
   double *dP = nullptr;     // P_k - P_(k-1), npad x npad zero padded (mixed Fock path only)
   double *epart = nullptr;  // energy partials of the J/K reduce, one per output block
   int *slots, *info;
@@ -179,14 +181,14 @@ struct Dev {
 
 int alloc(zq_ctx *ctx, Dev &d, int n, int maxh) {
   d.ctx = ctx, d.n = n, d.nn = size_t(n) * n;
-  const size_t nn = d.nn;
+  const size_t nn = d.nn, upper = size_t(tiles_of(n)) * (tiles_of(n) + 1) / 2;
   struct {
     const char *name;
     double **p;
     size_t cnt;
   } bufs[] = {{"scf_S", &d.S, nn},       {"scf_X", &d.X, nn},     {"scf_XT", &d.XT, nn},   {"scf_C", &d.C, nn},
               {"scf_T", &d.T, nn},       {"scf_Fp", &d.Fp, nn},   {"scf_W", &d.W, nn},     {"scf_FP", &d.FP, nn},
-              {"scf_FPS", &d.FPS, nn},   {"scf_Pn", &d.Pn, nn},   {"scf_Fh", &d.Fh, nn * maxh},
+              {"scf_FPS", &d.FPS, std::max(nn, upper * maxh)}, {"scf_Pn", &d.Pn, nn}, {"scf_Fh", &d.Fh, nn * maxh},
               {"scf_Eh", &d.Eh, nn * maxh}, {"scf_part", &d.part, size_t(kRedBlocks) * (2 + maxh)},
               {"scf_scal", &d.scal, size_t(2 + maxh)}, {"scf_coef", &d.coef, size_t(2 + maxh)}, {"scf_eig", &d.eig, size_t(n)},
               {"scf_offd", &d.offd, size_t(n)}};
@@ -194,6 +196,7 @@ int alloc(zq_ctx *ctx, Dev &d, int n, int maxh) {
     *b.p = (double *)zq_scratch(ctx, b.name, b.cnt * sizeof(double));
     if (!*b.p) return zq_fail(ctx, ZQ_ERR_OOM, std::string("device SCF buffer ") + b.name);
   }
+  d.dots = d.FPS, d.rms = d.Pn;  // the asynchronous driver's partials: it stores neither product
   d.slots = (int *)zq_scratch(ctx, "scf_slots", 64 * sizeof(int));
   d.info = (int *)zq_scratch(ctx, "scf_info", 4 * sizeof(int));
   if (!d.slots || !d.info) return zq_fail(ctx, ZQ_ERR_OOM, "device SCF buffers");
@@ -265,48 +268,109 @@ __global__ void k_state_init(ScfState *st, double VN, int diis) {
   if (diis > 0) diis_next_slot(st, diis);
 }
 
-// err = scale (FPS - (FPS)^T) into Eh[cur], F into Fh[cur].
-__global__ void k_antisym_store(const double *__restrict__ FPS, const double *__restrict__ F, int n, double scale,
-                                double *__restrict__ Eh, double *__restrict__ Fh, const ScfState *__restrict__ st) {
+// Tile pairs (ti, tj), ti <= tj, of an n x n matrix, row by row.
+__device__ inline void upper_tile_of(int t, int T, int &ti, int &tj) {
+  ti = 0;
+  while (t >= T - ti) t -= T - ti, ++ti;
+  tj = ti + t;
+}
+
+// err = scale (FP S - (FP S)^T) into Eh[cur], F into Fh[cur], and part[slot ntiles + t]: tile pair t's share of
+// dot(err, err_slot) for the slots of the history.  Workgroup t holds tiles (ti, tj), by wave 0, and (tj, ti), by
+// wave 1, of the product (S symmetric), which is all that its part of err needs, so the product, the history entry
+// and the dot products are one launch, not three.  What bounds it is the launch and one chain of load, 4 n / 16 MFMAs
+// and a butterfly.  With k_density_tile in place of a product and a store: 17 iterations at n = 144 6.91 -> 6.81 ms,
+// n = 96 from FP32 integrals 3.30 -> 3.25 ms (host round trip included).
+template <bool VEC>
+__global__ __launch_bounds__(128) void k_error(const double *__restrict__ FP, const double *__restrict__ S,
+                                               const double *__restrict__ F, int n, double scale, double *Eh,
+                                               double *__restrict__ Fh, double *__restrict__ part,
+                                               const ScfState *__restrict__ st) {
   if (st->done) return;
+  __shared__ double tile[2][16][17];
+  const int T = (n + 15) / 16, t = blockIdx.x, ntiles = T * (T + 1) / 2;
+  int ti, tj;
+  upper_tile_of(t, T, ti, tj);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int i0 = 16 * (wave ? tj : ti), j0 = 16 * (wave ? ti : tj), m = st->hist_n;
   const size_t nn = size_t(n) * n, off = size_t(st->cur) * nn;
-  for (size_t e = blockIdx.x * size_t(blockDim.x) + threadIdx.x; e < nn; e += size_t(gridDim.x) * blockDim.x) {
-    const int i = int(e / n), j = int(e % n);
-    Eh[off + e] = scale * (FPS[e] - FPS[size_t(j) * n + i]);
-    Fh[off + e] = F[e];
+  // tile (tj, ti) of every err is minus the other's transpose, so one of the two tiles gives both shares: the waves
+  // take the slots in turn, each on its own tile.  Their entries are loaded before the product (slots past the
+  // history's end repeat its last).
+  constexpr int kWaveSlots = kMaxHist / 2;
+  int slot[kWaveSlots];
+  double old[kWaveSlots][4];
+#pragma unroll
+  for (int k = 0; k < kWaveSlots; ++k) slot[k] = st->hist[min(2 * k + wave, m - 1)];
+#pragma unroll
+  for (int k = 0; k < kWaveSlots; ++k)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      old[k][j] = Eh[size_t(slot[k]) * nn + size_t(min(i0 + 4 * j + q, n - 1)) * n + min(j0 + r, n - 1)];
+  const zqt::d4 acc = zqt::tile_nt<VEC>(FP, n, S, n, i0, j0, n, n, n);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) tile[wave][4 * j + q][r] = acc[j];
+  __syncthreads();
+  double e[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = i0 + 4 * j + q, col = j0 + r;
+    const bool in = row < n && col < n;
+    e[j] = in ? scale * (acc[j] - tile[wave ^ 1][r][4 * j + q]) : 0.0;
+    if (in && (wave == 0 || ti != tj)) {
+      Eh[off + size_t(row) * n + col] = e[j];
+      Fh[off + size_t(row) * n + col] = F[size_t(row) * n + col];
+    }
+  }
+  const double both = ti == tj ? 1.0 : 2.0;
+#pragma unroll
+  for (int k = 0; k < kWaveSlots; ++k) {
+    if (2 * k + wave >= m) break;
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s = fma(e[j], slot[k] == st->cur ? e[j] : old[k][j], s);
+    s = zqt::wave_sum(s);
+    if (lane == 0) part[size_t(slot[k]) * ntiles + t] = both * s;
   }
 }
 
-// part[slot*kRedBlocks + b]: dot(err_cur, err_slot) over a strided subset (blockIdx.y = slot).
-__global__ __launch_bounds__(256) void k_dots_state(const double *__restrict__ hist, size_t nn, double *__restrict__ part,
-                                                    const ScfState *__restrict__ st) {
-  __shared__ double red[256];
-  if (st->done) return;
-  const double *enew = hist + size_t(st->cur) * nn, *ei = hist + size_t(blockIdx.y) * nn;
+// P (padded npad stride) = factor T X^T, with part[tile] = the tile's share of sum (P - P_old)^2 and dP (if
+// given) = P - P_old: the last product of the density and its store in one launch.
+template <bool VEC>
+__global__ __launch_bounds__(64) void k_density_tile(const double *__restrict__ T, const double *__restrict__ X, int n,
+                                                     double factor, double *__restrict__ P, int npad,
+                                                     double *__restrict__ part, const int *__restrict__ skip,
+                                                     double *__restrict__ dP) {
+  if (skip && *skip) return;
+  const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16, lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+  double old[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = i0 + 4 * j + q, col = j0 + r;
+    old[j] = row < n && col < n ? P[size_t(row) * npad + col] : 0.0;
+  }
+  const zqt::d4 acc = zqt::tile_nt<VEC>(T, n, X, n, i0, j0, n, n, n);
   double s = 0.0;
-  if (int(blockIdx.y) < kMaxHist) {
-    bool live = false;
-    for (int k = 0; k < st->hist_n; ++k) live |= st->hist[k] == int(blockIdx.y);
-    if (live)
-      for (size_t e = blockIdx.x * 256 + threadIdx.x; e < nn; e += size_t(gridDim.x) * 256) s += enew[e] * ei[e];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = i0 + 4 * j + q, col = j0 + r;
+    if (row >= n || col >= n) continue;
+    const double v = factor * acc[j], d = v - old[j];
+    s = fma(d, d, s);
+    P[size_t(row) * npad + col] = v;
+    if (dP) dP[size_t(row) * npad + col] = d;
   }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.y * kRedBlocks + blockIdx.x] = red[0];
+  s = zqt::wave_sum(s);
+  if (lane == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
 // E = sum of the energy partials + V_NN; DIIS: the new row of B, the bordered system, its LU solve
 // (src/hartree_fock.zig:176-227), or a reset to the current entry when it is singular (:821-845).
-// One wave: lane b holds partial b of every sum (kRedBlocks == 64), each sum a fixed-order butterfly;
-// the wave solves the <= 17 x 17 system, one row per lane.
+// One wave: lane b holds partials b, b + 64, ... of every sum (np of them a slot, k_error's), each sum a fixed-order
+// butterfly; the wave solves the <= 17 x 17 system, one row per lane.
 // epart: the nep energy partials the J/K reduce wrote (one per output block).
 __global__ __launch_bounds__(64) void k_diis_solve(const double *__restrict__ part, const double *__restrict__ epart,
-                                                   int nep, int diis, double VN, ScfState *__restrict__ st) {
-  static_assert(kRedBlocks == 64, "one partial per lane");
+                                                   int np, int nep, int diis, double VN, ScfState *__restrict__ st) {
   __shared__ double Bs[kMaxHist * kMaxHist];
   if (st->done) return;
   const int lane = threadIdx.x;
@@ -318,7 +382,11 @@ __global__ __launch_bounds__(64) void k_diis_solve(const double *__restrict__ pa
   for (int h = 0; h < kMaxHist; ++h) hist[h] = st->hist[h];
   const int hist_lane = st->hist[min(lane, kMaxHist - 1)];
 #pragma unroll
-  for (int k = 0; k < kMaxHist; ++k) dp[k] = part[(1 + k) * kRedBlocks + lane];
+  for (int k = 0; k < kMaxHist; ++k) dp[k] = lane < np && diis > k ? part[size_t(k) * np + lane] : 0.0;
+  for (int b = lane + 64; b < np; b += 64)
+#pragma unroll
+    for (int k = 0; k < kMaxHist; ++k)
+      if (diis > k) dp[k] += part[size_t(k) * np + b];
   double e = 0.0;
   for (int b = lane; b < nep; b += 64) e += epart[b];
   // the live slots as a mask, the history and the dot products in LDS (indexed at run time below)
@@ -406,7 +474,7 @@ __global__ void k_sp2_check(int parity, ScfState *__restrict__ st) {
 // The end of an iteration: the SP2 check of k_sp2_check (parity of its step budget), then rms(dP) and
 // the convergence test of src/hartree_fock.zig:853-870 (one wave, butterfly sum), and the report to the host,
 // which reads it one iteration late.
-__global__ __launch_bounds__(64) void k_converge(const double *__restrict__ part, int n, double thr, int maxit,
+__global__ __launch_bounds__(64) void k_converge(const double *__restrict__ part, int np, int n, double thr, int maxit,
                                                  ScfState *st, int parity, const double *est, ScfProgress *progress,
                                                  int diis) {
   if (st->done) {
@@ -414,7 +482,9 @@ __global__ __launch_bounds__(64) void k_converge(const double *__restrict__ part
     if (threadIdx.x == 0) report(st, est, progress);
     return;
   }
-  const double s = zqt::wave_sum(part[threadIdx.x]);
+  double s = 0.0;
+  for (int b = threadIdx.x; b < np; b += 64) s += part[b];
+  s = zqt::wave_sum(s);
   if (threadIdx.x != 0) return;
   const int *fin = st->sp2 + 2 * parity;
   st->sp2_steps = fin[1];
@@ -454,9 +524,11 @@ int density_async(Dev &d, const double *A, int nocc, double factor, int nsteps, 
   if (int rc = zq_sp2_enqueue(ctx, d.Fp, n, nocc, 1e-9, nsteps, skip, st->sp2, &D, &stride, &ld, check ? 1 : 2)) return rc;
   if (check) hipLaunchKernelGGL(k_sp2_check, dim3(1), dim3(64), 0, ctx->stream, nsteps & 1, st);
   if (int rc = zq_gemm_nt(ctx, d.X, n, D, ld, d.T, n, n, n, n, 1.0, "scf_gemm", skip, st->sp2 + 4, stride)) return rc;
-  if (int rc = zq_gemm_nt(ctx, d.T, n, d.X, n, d.Pn, n, n, n, n, factor, "scf_gemm", skip)) return rc;
-  hipLaunchKernelGGL(k_store_density, dim3(kRedBlocks), dim3(256), 0, ctx->stream, d.Pn, n, ctx->d_P, np, part_rms, skip,
-                     dP);
+  const dim3 tiles(unsigned(tiles_of(n)), unsigned(tiles_of(n)));
+  zq_prof_begin(ctx, "scf_gemm");
+  hipLaunchKernelGGL((n % 16 == 0 ? k_density_tile<true> : k_density_tile<false>), tiles, dim3(64), 0, ctx->stream, d.T, d.X, n,
+                     factor, ctx->d_P, np, part_rms, skip, dP);
+  zq_prof_end(ctx);
   ZQ_LAUNCH_CHECK(ctx, "density_async");
   return ZQ_OK;
 }
@@ -585,7 +657,7 @@ int step_args(const Dev &d, Run &r, ScfState *st) {
 // The kernels of one SCF iteration; every one of them returns at once while state.done != 0.
 int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *part_rms, ScfProgress *progress) {
   zq_ctx *ctx = d.ctx;
-  const int n = d.n, maxh = r.opt->diis > 0 ? r.opt->diis : 1;
+  const int n = d.n, upper = tiles_of(n) * (tiles_of(n) + 1) / 2;
   const size_t nn = d.nn;
   const int gblocks = int(std::min<size_t>(1024, (nn + 255) / 256));
   const int *skip = &st->done;
@@ -606,20 +678,20 @@ int enqueue_iteration(Dev &d, const Run &r, int budget, ScfState *st, double *pa
     return rc;
   }
   if (r.opt->diis > 0) {
-    // F P (P symmetric) and (F P) S (S symmetric) as A B^T products
+    // F P (P symmetric) as an A B^T product, then the error from (F P) S
     if (int rc = zq_gemm_nt(ctx, ctx->d_F, n, ctx->d_P, r.np, d.FP, n, n, n, n, 1.0, "scf_gemm", skip)) return rc;
-    if (int rc = zq_gemm_nt(ctx, d.FP, n, d.S, n, d.FPS, n, n, n, n, 1.0, "scf_gemm", skip)) return rc;
-    hipLaunchKernelGGL(k_antisym_store, dim3(gblocks), dim3(256), 0, ctx->stream, d.FPS, ctx->d_F, n, ctx->diis_err_scale,
-                       d.Eh, d.Fh, st);
-    hipLaunchKernelGGL(k_dots_state, dim3(kRedBlocks, maxh), dim3(256), 0, ctx->stream, d.Eh, nn, d.part + kRedBlocks, st);
+    zq_prof_begin(ctx, "scf_gemm");
+    hipLaunchKernelGGL((n % 16 == 0 ? k_error<true> : k_error<false>), dim3(unsigned(upper)), dim3(128), 0, ctx->stream, d.FP, d.S,
+                       ctx->d_F, n, ctx->diis_err_scale, d.Eh, d.Fh, d.dots, st);
+    zq_prof_end(ctx);
   }
-  hipLaunchKernelGGL(k_diis_solve, dim3(1), dim3(64), 0, ctx->stream, d.part, d.epart, ctx->Nb, r.opt->diis, r.VN, st);
+  hipLaunchKernelGGL(k_diis_solve, dim3(1), dim3(64), 0, ctx->stream, d.dots, d.epart, upper, ctx->Nb, r.opt->diis, r.VN, st);
   hipLaunchKernelGGL(k_combine_state, dim3(gblocks), dim3(256), 0, ctx->stream, d.Fh, ctx->d_F, n, d.W, st);
   if (int rc = density_async(d, d.W, r.nocc, r.factor, budget, st, part_rms, r.mixed ? d.dP : nullptr, false)) return rc;
   const double *est = zq_sp2_est(ctx);
   if (!est) return zq_fail(ctx, ZQ_ERR_OOM, "SP2 buffers");
-  hipLaunchKernelGGL(k_converge, dim3(1), dim3(64), 0, ctx->stream, part_rms, n, r.opt->threshold, r.opt->iterations, st,
-                     budget & 1, est, progress, r.opt->diis);
+  hipLaunchKernelGGL(k_converge, dim3(1), dim3(64), 0, ctx->stream, part_rms, tiles_of(n) * tiles_of(n), n, r.opt->threshold,
+                     r.opt->iterations, st, budget & 1, est, progress, r.opt->diis);
   ZQ_LAUNCH_CHECK(ctx, "scf iteration");
   return ZQ_OK;
 }
@@ -656,7 +728,7 @@ int scf_async(Dev &d, Run &r, int *status, double *energy, int *iterations) {
   if (!st || !hprog) return zq_fail(ctx, ZQ_ERR_OOM, "SCF state");
   ScfProgress *dprog = nullptr;  // the same host memory as the kernels address it
   ZQ_TRY(ctx, hipHostGetDevicePointer((void **)&dprog, hprog, 0));
-  double *part_rms = d.part + (1 + kMaxHist) * kRedBlocks;
+  double *part_rms = d.rms;
   d.epart = (double *)zq_scratch(ctx, "scf_epart", size_t(ctx->Nb) * sizeof(double));
   if (!d.epart) return zq_fail(ctx, ZQ_ERR_OOM, "SCF energy partials");
   if (r.mixed) {
