@@ -534,8 +534,8 @@ int density_async(Dev &d, const double *A, int nocc, double factor, int nsteps, 
 }
 
 // The one-workgroup form takes molecules up to n = 64.  A whole run, multi-launch / one workgroup, ms: n = 7
-// 1.24 / 0.66, n = 24 2.73 / 1.37, n = 48 3.27 / 2.20, n = 56 2.91 / 2.44.  Beyond that the FP64 matrix rate of
-// one compute unit costs what the launches did: n = 72 4.21 / 4.16, n = 96 5.27 / 6.76.
+// 0.94 / 0.50, n = 24 2.00 / 1.22, n = 48 2.41 / 1.94, n = 56 2.15 / 2.16.  Beyond that the FP64 matrix rate of
+// one compute unit costs more than the launches: n = 72 3.10 / 4.16, n = 96 3.94 / 6.76.
 constexpr int kStepMaxTiles = 4;
 bool step_fits(int n) { return n <= 16 * kStepMaxTiles; }
 
