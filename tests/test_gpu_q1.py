@@ -64,3 +64,24 @@ def test_group_takes_the_same_path(n, o):
         assert r["status"][0] == 0
         assert r["E_corr"][0] == c.mp2(C, e, o, precision=precision), precision
         c.close()
+
+
+@pytest.mark.parametrize("n,o", [(121, 8), (128, 17), (129, 8), (136, 17), (145, 18)])
+def test_last_quarters_both_forms(ctx, n, o):
+    """Q3 and Q4 of the 4-byte forms on both sides of the size (128 padded functions) where they go from registers to
+    tiles in LDS; integrals of rank 2, so that the reference needs no dense tensor."""
+    rng = np.random.default_rng(n + o)
+    B = rng.standard_normal((2, n, n))
+    B = B + B.transpose(0, 2, 1)
+    low = np.tril_indices(n)
+    b = B[:, low[0], low[1]]
+    pk = np.concatenate([b[:, t] @ b[:, :t + 1] for t in range(b.shape[1])])
+    C = rng.standard_normal((n, n)) / np.sqrt(n)
+    ctx.eri_load_packed(pk, n)
+
+    M, A = (np.einsum("mi,pmn,na->pia", c[:, :o], x, c[:, o:], optimize=True) for x, c in ((B, C), (np.abs(B), np.abs(C))))
+    ref, scale = np.einsum("pia,pjb->ijab", M, M), np.einsum("pia,pjb->ijab", A, A)
+    for precision in ("fp64", "fp32", "fp32c"):
+        out = ctx.ao2mo(C, o, "ovov", precision=precision)
+        eps = np.finfo(np.float64 if precision == "fp64" else np.float32).eps
+        assert np.all(np.abs(out - ref) <= (4 * n + 8) * eps * scale), (n, o, precision)

@@ -1158,29 +1158,41 @@ int upload(zq_ctx *ctx, const char *name, const std::vector<T> &h, T **d) {
   return ZQ_OK;
 }
 
+// Whether Q3 and Q4 run on the 64 x 64 tiles staged in LDS (zq_gemm) and not on zq_wide: FP64 always (Q3 231 us
+// against 291, Q4 219 against 278 at n = 192, o = 40); the 4-byte forms beyond np = 128, where a product has enough
+// tiles to hide the staging and its operands outgrow the L1 that zq_wide's waves share them through.  A whole MP2
+// energy, FP32 / FP32C, us, registers against tiles: n = 101 150 / 179 against 166 / 200, n = 120 236 / 279 against
+// 253 / 296, n = 128 331 / 375 against 334 / 370, n = 144 471 / 552 against 452 / 534, n = 192 1510 / 1828 against
+// 1427 / 1752, n = 240 3916 / 6075 against 3844 / 6021.
+constexpr int kWide34Max = 128;
+template <class T>
+__host__ __device__ constexpr bool q34_tiles(int np) {
+  return sizeof(T) == 8 || np > kWide34Max;
+}
+
 // The coefficient slices of run_chain built on the device from C (n x n, already on the device): the
 // same element conversions as the host staging, so the values are identical.
 template <class T>
 __device__ __forceinline__ void c_slices_body(const double *__restrict__ C, int n, int np, int m1, int m2, int m3,
-                                              int off3, T *__restrict__ c1, T *__restrict__ c2, bool plain,
-                                              T *__restrict__ c3, int mu) {
+                                              int off3, T *__restrict__ c1, T *__restrict__ c2, bool plain2,
+                                              bool plain3, T *__restrict__ c3, int mu) {
   for (int t = threadIdx.x; t < m1 + m2 + m3; t += blockDim.x) {
     if (t < m1) {
       c1[q1_c_index(mu, t, m1)] = mu < n ? T(C[size_t(mu) * n + t]) : T(0);
     } else if (t < m1 + m2) {
       const int j = t - m1;
-      c2[plain ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = mu < n ? T(C[size_t(mu) * n + j]) : T(0);
+      c2[plain2 ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = mu < n ? T(C[size_t(mu) * n + j]) : T(0);
     } else {
       const int a = t - m1 - m2;
-      c3[plain || sizeof(T) == 8 ? size_t(mu) * m3 + a : q1_c_index(mu, a, m3)] = mu < n ? T(C[size_t(mu) * n + off3 + a]) : T(0);
+      c3[plain3 ? size_t(mu) * m3 + a : q1_c_index(mu, a, m3)] = mu < n ? T(C[size_t(mu) * n + off3 + a]) : T(0);
     }
   }
 }
 
 template <class T>
 __global__ void zq_c_slices(const double *__restrict__ C, int n, int np, int m1, int m2, int m3, int off3,
-                            T *__restrict__ c1, T *__restrict__ c2, bool plain, T *__restrict__ c3) {
-  c_slices_body<T>(C, n, np, m1, m2, m3, off3, c1, c2, plain, c3, blockIdx.x);  // one workgroup per row mu < np
+                            T *__restrict__ c1, T *__restrict__ c2, bool plain2, bool plain3, T *__restrict__ c3) {
+  c_slices_body<T>(C, n, np, m1, m2, m3, off3, c1, c2, plain2, plain3, c3, blockIdx.x);  // one workgroup per row mu < np
 }
 
 // y = x (n doubles; x may be pinned host memory)
@@ -1247,8 +1259,9 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
   // BF16X3 Q1 takes C1 split and transposed: C1h/C1l[i][mu], mu padded to a multiple of 32
   const int ldt = ((nb + 3) / 4) * 32;
   T *d1, *d2, *d3, *d4 = nullptr;
-  // BF16X3 takes C2 transposed and C3, C4 as plain matrices, FP64 C3 and C4; the others as q1_c_index lays them out
-  const bool plain = precision == ZQ_PREC_BF16X3;
+  // BF16X3 takes C2 transposed, it and the tile forms of Q3 and Q4 C3 and C4 as plain matrices; the others as
+  // q1_c_index lays them out
+  const bool plain = precision == ZQ_PREC_BF16X3, plain3 = plain || q34_tiles<T>(np);
   bf16 *d1h = nullptr, *d1l = nullptr;
   if constexpr (sizeof(T) == 4) {
     if (precision != ZQ_PREC_BF16X3) {
@@ -1271,7 +1284,7 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
       return zq_fail(ctx, ZQ_ERR_INVALID, "zq_mp2_noalloc: static scratch too small");
     ZQ_TRY(ctx, hipMemcpyAsync(dC, C, size_t(n) * n * 8, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(zq_c_slices<T>, dim3(unsigned(np)), dim3(256), 0, ctx->stream, dC, n, np, m1, m2, m3, d.off3, d1,
-                       d2, plain, d3);
+                       d2, plain, plain3, d3);
     if (precision == ZQ_PREC_BF16X3)
       hipLaunchKernelGGL(zq_c1_split, dim3(unsigned(m1)), dim3(256), 0, ctx->stream, dC, n, m1, ldt, d1h, d1l);
     ZQ_LAUNCH_CHECK(ctx, "zq_c_slices");
@@ -1288,7 +1301,7 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     if (!d1 || !d2 || !d3 || (precision == ZQ_PREC_BF16X3 && (!d1h || !d1l)))
       return zq_fail(ctx, ZQ_ERR_OOM, "transform scratch C slices");
     hipLaunchKernelGGL(zq_c_slices<T>, dim3(unsigned(np)), dim3(256), 0, ctx->stream, C, n, np, m1, m2, m3, d.off3, d1,
-                       d2, plain, d3);
+                       d2, plain, plain3, d3);
     if (precision == ZQ_PREC_BF16X3)
       hipLaunchKernelGGL(zq_c1_split, dim3(unsigned(m1)), dim3(256), 0, ctx->stream, C, n, m1, ldt, d1h, d1l);
     ZQ_LAUNCH_CHECK(ctx, "zq_c_slices");
@@ -1300,9 +1313,9 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     for (int mu = 0; mu < n; ++mu) {
       for (int i = 0; i < m1; ++i) h1[q1_c_index(mu, i, m1)] = T(cf.q[0][size_t(mu) * n + i]);
       for (int j = 0; j < m2; ++j) h2[plain ? size_t(j) * np + mu : q1_c_index(mu, j, m2)] = T(cf.q[1][size_t(mu) * n + j]);
-      for (int a = 0; a < m3; ++a) h3[plain || sizeof(T) == 8 ? size_t(mu) * m3 + a : q1_c_index(mu, a, m3)] = T(cf.q[2][size_t(mu) * n + d.off3 + a]);
+      for (int a = 0; a < m3; ++a) h3[plain3 ? size_t(mu) * m3 + a : q1_c_index(mu, a, m3)] = T(cf.q[2][size_t(mu) * n + d.off3 + a]);
       if (own4)
-        for (int b = 0; b < m4; ++b) h4[plain || sizeof(T) == 8 ? size_t(mu) * m4 + b : q1_c_index(mu, b, m4)] = T(cf.q[3][size_t(mu) * n + d.off3 + b]);
+        for (int b = 0; b < m4; ++b) h4[plain3 ? size_t(mu) * m4 + b : q1_c_index(mu, b, m4)] = T(cf.q[3][size_t(mu) * n + d.off3 + b]);
     }
     if (int rc = upload(ctx, "C1", h1, &d1)) return rc;
     if (int rc = upload(ctx, "C2", h2, &d2)) return rc;
@@ -1392,9 +1405,11 @@ int run_chain(zq_ctx *ctx, const Coefs &cf, const Dims &d, int precision, T **d_
     }
   }
   if (int rc = launch_wide<MF, true, true>(ctx, g2, m1, "ao2mo_q2")) return rc;
-  if constexpr (sizeof(T) == 4) {
-    if (int rc = launch_wide<MF, false, false>(ctx, q3_args<T>(Y, d4, W, np, m2, m4, sym), nij, "ao2mo_q3")) return rc;
-    if (int rc = launch_wide<MF, false, true>(ctx, q4_args<T>(W, d3, O, np, m3, m4), nij, "ao2mo_q4")) return rc;
+  if (!plain3) {
+    if constexpr (sizeof(T) == 4) {
+      if (int rc = launch_wide<MF, false, false>(ctx, q3_args<T>(Y, d4, W, np, m2, m4, sym), nij, "ao2mo_q3")) return rc;
+      if (int rc = launch_wide<MF, false, true>(ctx, q4_args<T>(W, d3, O, np, m3, m4), nij, "ao2mo_q4")) return rc;
+    }
   } else {
     if (int rc = launch_gemm<MF>(ctx, q3_tile_args<T>(Y, d3, W, np, m2, m3, sym), nij, "ao2mo_q3")) return rc;
     if (int rc = launch_gemm<MF>(ctx, q4_tile_args<T>(W, d4, O, np, m3, m4), nij, "ao2mo_q4")) return rc;
@@ -1613,7 +1628,7 @@ __global__ __launch_bounds__(256) void zq_group_slices(const GJob<T, E> *__restr
                                                        int nmol) {
   const int m = group_find(start, nmol, blockIdx.x);
   const GJob<T, E> J = jobs[m];
-  c_slices_body<T>(J.C, J.n, J.np, J.o, J.o, J.v, J.o, J.c1, J.c2, false, J.c3, int(blockIdx.x) - start[m]);
+  c_slices_body<T>(J.C, J.n, J.np, J.o, J.o, J.v, J.o, J.c1, J.c2, false, q34_tiles<T>(J.np), J.c3, int(blockIdx.x) - start[m]);
 }
 
 template <class MF, class E>
@@ -1732,6 +1747,10 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
       J.out = d_out + k;
       const GemmArgs<T> &g2 = J.g[0] = q2_args(J.X, J.c2, Y, J.np, J.o, J.o, true);
       constexpr bool wide = sizeof(T) == 4;
+      if (wide && q34_tiles<T>(J.np)) {  // a molecule of a group takes the form it takes alone
+        err = "grouped MP2: molecule above the register forms' size";
+        return ZQ_ERR_INVALID;
+      }
       const GemmArgs<T> &g3 = J.g[1] = wide ? q3_args<T>(Y, J.c3, W, J.np, J.o, J.v, true) : q3_tile_args<T>(Y, J.c3, W, J.np, J.o, J.v, true);
       const GemmArgs<T> &g4 = J.g[2] = wide ? q4_args<T>(W, J.c3, J.O, J.np, J.v, J.v) : q4_tile_args<T>(W, J.c3, J.O, J.np, J.v, J.v);
       constexpr int cols = wide ? 128 : 64;
