@@ -62,6 +62,7 @@ void *zq_scratch(zq_ctx *ctx, const std::string &name, size_t bytes, bool *fresh
   DevBuf &b = ctx->scratch[name];
   if (fresh) *fresh = false;
   if (b.bytes >= bytes && b.ptr) return b.ptr;
+  if (tl_excl) return nullptr;  // capturing: nothing is freed or allocated, the buffer may be in use
   if (b.ptr) (void)hipFree(b.ptr);
   b.ptr = nullptr;
   b.bytes = 0;

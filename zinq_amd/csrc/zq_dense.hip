@@ -637,7 +637,8 @@ int zq_gemm_nt(zq_ctx *ctx, const double *A, int lda, const double *B, int ldb, 
 
 namespace {
 
-// X: two m x m buffers (nx for the one-XCD form: an X per step); part: the partials of X_0 .. X_kSp2MaxSteps
+// X: two m x m buffers (nx for the one-XCD form, an X per step whatever the budget: the guess density and the captured
+// iteration have budgets of their own, and a capture may not grow a buffer); part: the partials of X_0 .. X_kSp2MaxSteps
 // (ntiles each; the step-per-launch form ping-pongs between the first two); sync: the counters of the one-launch
 // forms.
 struct Sp2Bufs {
@@ -695,7 +696,7 @@ int zq_sp2_enqueue(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, i
   if (nsteps < 1 || nsteps > kSp2MaxSteps) return zq_fail(ctx, ZQ_ERR_INVALID, "SP2 step budget out of range");
   if (track < 0 || track > 2) return zq_fail(ctx, ZQ_ERR_INVALID, "SP2 fold tracking mode out of range");
   Sp2Bufs b;
-  if (int rc = sp2_bufs(ctx, n, n <= kSp2HomeMax ? nsteps + 1 : 2, b)) return rc;
+  if (int rc = sp2_bufs(ctx, n, n <= kSp2HomeMax ? kSp2MaxSteps + 1 : 2, b)) return rc;
   zq_prof_begin(ctx, "scf_sp2");
   sp2_start(ctx, b, dF, n, nocc, state6, skip, track);
   double *est = track ? b.est : nullptr;
