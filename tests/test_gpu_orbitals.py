@@ -54,3 +54,25 @@ def test_batch_orbitals_vs_scipy(degenerate):
         np.testing.assert_allclose(C.T @ S @ C, np.eye(n), rtol=0, atol=16 * n * EPS * np.linalg.cond(S), err_msg=str(n))
         np.testing.assert_allclose(H @ C, S @ C * e, rtol=0, atol=tol * np.abs(S).sum(1).max() * np.abs(C).max(), err_msg=str(n))
     b.close()
+
+
+@pytest.mark.parametrize("n", [6, 33, 70])
+def test_batch_orbitals_zero_levels(n):
+    """Levels at zero that couplings of 1e-20 to a low level split by 1e-41 of the largest element: a gap and a pivot
+    below the range of normal single-precision numbers.  The matrix is diagonal to working precision, so the
+    levels come back to n eps of the largest and the orbitals orthonormal to n eps."""
+    from zinq_amd.batch import Batch
+
+    nocc, zeros = 2, n // 2
+    w = np.concatenate([[-8.0, -4.0], np.zeros(zeros), np.linspace(1.0, 3.0, n - 2 - zeros)])
+    H = np.diag(w)
+    H[0, 2:2 + zeros] = H[2:2 + zeros, 0] = 1e-20 * np.arange(1, zeros + 1)
+    npair = n * (n + 1) // 2
+    b = Batch(0)
+    b.add(H, np.eye(n), 0.0, nocc, np.zeros(npair * (npair + 1) // 2))
+    r = b.run(iterations=50)
+    e, C = b.orbitals(0)
+    b.close()
+    assert r["status"][0] == 0
+    np.testing.assert_allclose(e, w, rtol=0, atol=16 * n * EPS * 8.0)
+    np.testing.assert_allclose(C.T @ C, np.eye(n), rtol=0, atol=16 * n * EPS)

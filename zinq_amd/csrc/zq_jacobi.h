@@ -144,7 +144,8 @@ struct Jacobi {
     const double gap = aqq - app;
     const float hf = float(0.5 * gap * inv), af = float(apq * inv);
     const float den = fabsf(hf) + __builtin_amdgcn_sqrtf(hf * hf + af * af);
-    const float t = den > 0.0f ? copysignf(1.0f, hf) * af * __builtin_amdgcn_rcpf(den) : 0.0f;
+    // below the normal numbers the reciprocal is infinite; gap and pivot are then 1e-19 of the largest at most
+    const float t = den >= 0x1p-126f ? copysignf(1.0f, hf) * af * __builtin_amdgcn_rcpf(den) : 0.0f;
     const double tau = double(t * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_sqrtf(1.0f + t * t)));
     const double x = fma(tau, tau, 1.0);
     double y = __builtin_amdgcn_rcp(x);
