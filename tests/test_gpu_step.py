@@ -86,3 +86,16 @@ def test_scf_launches(ctx, n, diis):
         assert ctx.last_scf_driver() == "device"
         assert abs(r["iterations"] - ro["iterations"]) <= 1
         assert r["E"] == pytest.approx(ro["E"], abs=1e-10)
+
+
+def test_scf_without_iterations_reports_its_guess(ctx):
+    """A run of no iterations makes the guess density alone: one SP2 density, not folded."""
+    from zinq_amd import hip
+    for k in (1, 10):  # one workgroup, multi-launch
+        s, H, S, g, VN = _water(k)
+        ctx.eri_load_packed(s.coulomb_packed(), s.nbf)
+        with pytest.raises(hip.ScfDidNotConverge):
+            ctx.scf(H, S, VN, s.nel // 2, iterations=0, device=True)
+        sp2 = ctx.last_scf_sp2()
+        assert ctx.last_scf_driver() == "device" and ctx.scf_replays() == 0
+        assert sp2["densities"] == 1 and sp2["folded"] == 0 and sp2["steps"] > 1, sp2

@@ -806,10 +806,15 @@ int scf_async(Dev &d, Run &r, int *status, double *energy, int *iterations) {
   }
   if (r.opt->iterations < 1) {  // no iteration, no report: the guess density's state
     ScfState hs;
+    double sp2[3];
+    const double *est = zq_sp2_est(ctx);
+    if (!est) return zq_fail(ctx, ZQ_ERR_OOM, "SP2 buffers");
     ZQ_TRY(ctx, hipMemcpyAsync(&hs, st, sizeof(ScfState), hipMemcpyDeviceToHost, ctx->stream));
+    ZQ_TRY(ctx, hipMemcpyAsync(sp2, est + kEstRuns, sizeof sp2, hipMemcpyDeviceToHost, ctx->stream));
     ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
     *status = hs.done == 0 ? 2 : hs.done;
     *energy = hs.e_new, *iterations = hs.it;
+    for (int x = 0; x < 3; ++x) ctx->scf_sp2[x] = *status == 3 ? 0 : int(sp2[x]);
     return ZQ_OK;
   }
   // a run that used its last iteration has not seen that one's report yet
