@@ -99,3 +99,14 @@ def test_scf_without_iterations_reports_its_guess(ctx):
         sp2 = ctx.last_scf_sp2()
         assert ctx.last_scf_driver() == "device" and ctx.scf_replays() == 0
         assert sp2["densities"] == 1 and sp2["folded"] == 0 and sp2["steps"] > 1, sp2
+
+
+def test_scf_history_beyond_the_device(ctx):
+    """A DIIS history above 16 goes to the host-synchronised driver at once, on the inputs set up before it."""
+    s, H, S, g, VN = _water(5)
+    o = s.nel // 2
+    ctx.eri_load_packed(s.coulomb_packed(), s.nbf)
+    ro = O.scf(H, S, g, VN, o, diis=20, threshold=1e-8)
+    r = ctx.scf(H, S, VN, o, diis=20, threshold=1e-8, device=True)
+    assert ctx.last_scf_driver() == "synced" and r["iterations"] == ro["iterations"]
+    assert r["E"] == pytest.approx(ro["E"], abs=1e-10)

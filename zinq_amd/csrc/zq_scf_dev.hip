@@ -616,8 +616,8 @@ __global__ __launch_bounds__(256) void k_scf_out(const double *__restrict__ C, c
 
 unsigned io_blocks(size_t cnt) { return unsigned(std::min<size_t>(1024, (cnt + 255) / 256)); }
 
-// Uploads S, X = L^-T, X^T, H; zeroes P.  (A second call, of the host-synchronised restart, finds the first one's
-// copies long done: iterations have run behind them.)
+// Uploads S, X = L^-T, X^T, H; zeroes P.  A second call refills the pinned copies, so it may only follow a read of
+// results behind the first one's kernel.
 int setup(Dev &d, const double *H, const double *S) {
   zq_ctx *ctx = d.ctx;
   const int n = d.n, np = ctx->npad;
@@ -976,8 +976,9 @@ extern "C" int zq_scf_run_device(zq_ctx *ctx, size_t n_, size_t nocc_, const dou
   ctx->scf_driver = (status == 0 || status == 3) ? 2 : 1;
   if (status == 0 || status == 3) {
     // DIIS history beyond the device bookkeeping, or an SP2 budget too small: synchronised driver
-    // (FP64 Fock builds throughout)
-    if (int rc = setup(d, H, S)) return rc;
+    // (FP64 Fock builds throughout), on fresh inputs where the device driver has run (its report has been read)
+    if (status == 3)
+      if (int rc = setup(d, H, S)) return rc;
     if (int rc = scf_synced(d, r, &status, &energy, &iterations)) return rc;
   } else if (r.mixed) {
     // mixed path: one full FP64 build from the last density; its energy is variational (error second
