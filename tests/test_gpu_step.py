@@ -110,3 +110,46 @@ def test_scf_history_beyond_the_device(ctx):
     r = ctx.scf(H, S, VN, o, diis=20, threshold=1e-8, device=True)
     assert ctx.last_scf_driver() == "synced" and r["iterations"] == ro["iterations"]
     assert r["E"] == pytest.approx(ro["E"], abs=1e-10)
+
+
+def test_batch_largest_molecules():
+    """Batch molecules on five and six tiles (n = 73 .. 96) with a two-electron part, in a batch that was not
+    autotuned, so that their Fock builds take long work items, beside a small molecule in the short form and alone in the
+    long one, and again after the autotuner chose: the oracle's SCF to the bars above, alone and mixed the same bits."""
+    from zinq_amd.batch import Batch
+    mols = []
+    for n in (7, 73, 80, 81, 96):
+        rng = np.random.default_rng(n)
+        o = max(1, n // 5)
+        Q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+        H = (Q * np.concatenate([np.linspace(-20.0, -2.0, o), np.linspace(0.5, 4.0, n - o)])) @ Q.T
+        S = np.eye(n) + 0.002 * (lambda a: a + a.T)(rng.standard_normal((n, n)))
+        tri = np.tril_indices(n)
+        m = 0.0
+        for _ in range(3):  # (pq|rs) = sum of b_pq b_rs
+            b = rng.standard_normal((n, n))
+            b = 0.025 * (b + b.T)[tri]
+            m = m + b[:, None] * b[None, :]
+        mols.append((0.5 * (H + H.T), S, 1.5, o, m[np.tril_indices(len(b))]))
+    ref = [O.scf(H, S, None, VN, o, threshold=1e-8, packed=pk) for H, S, VN, o, pk in mols]
+    mix = Batch(0)
+    for m in mols:
+        mix.add(*m)
+    for tuned in (False, True):
+        if tuned:
+            print("autotuned:", mix.autotune(), flush=True)
+        r = mix.run(threshold=1e-8)
+        assert (r["status"] == 0).all(), r["status"]
+        for k, ro in enumerate(ref):
+            print(f"n={len(mols[k][0])} tuned={tuned}: dE {r['E_rhf'][k] - ro['E']:+.1e} it {r['iterations'][k]}/"
+                  f"{ro['iterations']}", flush=True)
+            assert r["E_rhf"][k] == pytest.approx(ro["E"], abs=1e-10)
+            assert abs(r["iterations"][k] - ro["iterations"]) <= 1
+            if not tuned:
+                alone = Batch(0)
+                alone.add(*mols[k])
+                ra = alone.run(threshold=1e-8)
+                assert ra["E_rhf"][0] == r["E_rhf"][k] and ra["E_corr"][0] == r["E_corr"][k]
+                assert ra["iterations"][0] == r["iterations"][k]
+                alone.close()
+    mix.close()

@@ -216,6 +216,7 @@ struct zq_batch {
   JKMol *d_jkm = nullptr;
   int2 *d_blk = nullptr;
   int nitems = 0, nblk = 0;
+  bool jk_long = false;  // the J/K plan is run in the records kernel's long form
   std::vector<long long> eri_off, ws_off;
   size_t eri_count = 0;  // doubles in eri
   int mp_max = 16;       // largest padded size of the batch (the step's LDS)
@@ -328,18 +329,24 @@ void free_all(zq_batch *b) {
 int mp_of(int n) { return (n + 15) / 16 * 16; }
 int nb_of(int n) { return (n + ZQ_BLK - 1) / ZQ_BLK; }
 
-// The grouped J/K plan for item size `chunk`: items, records and CSR rows of all molecules concatenated.
+// The grouped J/K plan for item size `chunk` (0: each molecule's default): items, records and CSR rows of all molecules
+// concatenated.  With the defaults, long and short items mix; the long form is taken when all are long.  SCF of 6
+// iterations without autotune, ms, short / long form / each item in its own, in two launches: 32 molecules n = 96
+// 8.62 / 8.54 / 8.55, 8 n = 80 2.72 / 2.68 / 2.68, 40 n = 24 .. 96 6.36 / 6.77 / 6.34, 60 n <= 24 and one n = 96
+// 3.94 / 3.91 / 3.98 (items of one quartet throughout: 9.61, 2.78, 6.59, 4.00).
 int build_plan(zq_batch *b, int chunk) {
   free_plan(b);
   std::vector<JKItem> items;
   std::vector<int> ptr(1, 0), idx;
   std::vector<int2> blk;
   size_t rec_base = 0;
+  b->jk_long = true;
   for (size_t m = 0; m < b->mols.size(); ++m) {
     const int nb = nb_of(b->mols[m].n), Nb = nb * (nb + 1) / 2;
     const size_t nq = size_t(Nb) * (Nb + 1) / 2;
     JKPlan pl;
     zq_jk_plan(Nb, nq, chunk, pl);
+    b->jk_long = b->jk_long && zq_jk_long(nq, chunk);
     for (JKItem it : pl.items) {
       it.rec0 += int(rec_base);
       it.mol = int(m);
@@ -479,7 +486,7 @@ void launch_step(zq_batch *b, int mode, int diis, double thr, int maxit) {
 
 int enqueue_iteration(zq_batch *b, int diis, double thr, int maxit) {
   BTRY(b, zq_jk_group(b->stream, b->eri, b->d_items, b->nitems, b->ws, 0.5, b->rec, b->d_jkm, b->d_done, b->d_ptr,
-                      b->d_idx, b->d_blk, b->nblk, b->ws, b->ws, b->mp_max, b->chunk));
+                      b->d_idx, b->d_blk, b->nblk, b->ws, b->ws, b->mp_max, b->jk_long));
   launch_step(b, kStepIter, diis, thr, maxit);
   hipLaunchKernelGGL(k_batch_count, dim3(1), dim3(256), 0, b->stream, b->d_done, int(b->mols.size()), b->d_count);
   BTRY(b, hipGetLastError());
@@ -584,7 +591,7 @@ int zq_batch_autotune(zq_batch *b, int chosen[2]) {
     if (int rc = build_plan(b, ch)) return rc;
     const float ms = time_it([&] {
       (void)zq_jk_group(b->stream, b->eri, b->d_items, b->nitems, b->ws, 0.5, b->rec, b->d_jkm, b->d_done, b->d_ptr,
-                        b->d_idx, b->d_blk, b->nblk, b->ws, b->ws, b->mp_max, b->chunk);
+                        b->d_idx, b->d_blk, b->nblk, b->ws, b->ws, b->mp_max, b->jk_long);
     });
     if (ms < best) best = ms, best_chunk = ch;
   }

@@ -66,6 +66,8 @@ struct JKPlan {
 };
 // chunk = quartets per item (<= 0: the default for this size)
 void zq_jk_plan(int Nb, size_t nquartets, int chunk, JKPlan &plan);  // zq_jk.hip
+// Whether that plan's items are better off in the long form of the records kernel.
+bool zq_jk_long(size_t nquartets, int chunk);  // zq_jk.hip
 // The same plan on the device: it depends on the molecule's size only, so a resident ERI set keeps one
 // that every context attached to it reads.
 struct JKPlanDev {
@@ -260,10 +262,10 @@ constexpr int kZqMaxDevices = 64;
 void zq_noalloc_setup(int device);
 // Grouped J/K on `stream`: F = H + G(P) (x_exch) for every molecule of a grouped plan whose done flag
 // is 0.  blk[g] = (molecule, output block) for the nblk CSR rows; ld_max: the largest leading dimension of a P;
-// chunk: the plan's item size (0: each molecule's own).  Returns the launch status.
+// lng: the records kernel's long form (the same bits).  Returns the launch status.
 hipError_t zq_jk_group(hipStream_t stream, const double *eri, const JKItem *items, int nitems, const double *P,
                        double x_exch, double *rec, const JKMol *mols, const int *done, const int *csr_ptr,
-                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F, int ld_max, int chunk);
+                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F, int ld_max, bool lng);
 // Packs canonical chemist ERIs (zq_eri_load_packed layout) into 8x8 AO-block quartets (zq_context.hip).
 __global__ __launch_bounds__(256) void zq_pack_quartets(const double *__restrict__ canon, double *__restrict__ out, int n,
                                                         size_t nquartets);

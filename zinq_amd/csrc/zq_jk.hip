@@ -332,6 +332,11 @@ inline size_t jk_lds(int npad, bool lng) { return lng ? 16 * size_t(npad + 2) * 
 // alone - / 362 / 311 / 309.
 inline int jk_chunk(size_t nq) { return nq < 1536 ? 1 : nq < 14000 ? 8 : 16; }
 inline bool jk_long(int chunk) { return chunk >= 4; }
+}  // namespace
+
+bool zq_jk_long(size_t nq, int chunk) { return jk_long(chunk > 0 ? chunk : jk_chunk(nq)); }
+
+namespace {
 
 // F block (x >= y) = H + sum of records aimed at (x,y) + transposed records aimed at (y,x).  kRedWaves
 // waves take contiguous shares of the block's record list with 8 loads in flight each; the shares are
@@ -593,8 +598,7 @@ int zq_fock_jk_device(zq_ctx *ctx, const double *dP, const double *dH, double x_
 
 hipError_t zq_jk_group(hipStream_t stream, const double *eri, const JKItem *items, int nitems, const double *P,
                        double x_exch, double *rec, const JKMol *mols, const int *done, const int *csr_ptr,
-                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F, int ld_max, int chunk) {
-  const bool lng = jk_long(chunk);
+                       const int *csr_idx, const int2 *blk, int nblk, const double *H, double *F, int ld_max, bool lng) {
   hipLaunchKernelGGL((lng ? zq_jk_records<double, true, false, true> : zq_jk_records<double, true, false, false>),
                      dim3(unsigned(nitems)), dim3(256), jk_lds(ld_max, lng), stream, eri, items, nitems, P, 0, x_exch, rec, nullptr,
                      mols, done, 0LL, 0LL);
