@@ -194,10 +194,11 @@ __device__ inline void tile_partials(const double v[4], int ti, int tj, int i0, 
 }
 
 // X_0 on the m x m padded grid (zero outside n x n), its partials, the stop state, and the zeroed
-// counters of the one-launch form.
+// counters of the one-launch forms; for the one-XCD form, which polls them, the partials of the nunset steps it may
+// take are marked as not there.
 __global__ __launch_bounds__(64) void k_sp2_init(const double *__restrict__ F, int n, int m, const double *__restrict__ scal,
                                                  double *__restrict__ X, double2 *__restrict__ part, int *__restrict__ state,
-                                                 unsigned *__restrict__ sync, const int *__restrict__ skip) {
+                                                 unsigned *__restrict__ sync, int nunset, const int *__restrict__ skip) {
   if (skip && *skip) return;
   const int T = m / 16;
   int ti, tj;
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(64) void k_sp2_init(const double *__restrict__ F, i
   }
   tile_partials(v, ti, tj, i0, j0, part, blockIdx.x);
   const double unset = __longlong_as_double((long long)kSp2Unset);
-  for (int k = 1 + lane; k <= kSp2MaxSteps; k += 64) part[size_t(k) * gridDim.x + blockIdx.x] = make_double2(unset, unset);
+  for (int k = 1 + lane; k <= nunset; k += 64) part[size_t(k) * gridDim.x + blockIdx.x] = make_double2(unset, unset);
   if (blockIdx.x == 0) {
     for (int u = lane; u < kSp2Sync; u += 64) sync[u] = 0u;
     if (lane == 0) state[0] = -1, state[1] = 0, state[4] = 0, state[5] = 0;
@@ -668,12 +669,13 @@ int sp2_bufs(zq_ctx *ctx, int n, int nx, Sp2Bufs &b) {
 }
 
 // track: 0 plain SP2 outside the fold bookkeeping, 1 the first run of a device SCF, 2 a later run.
-void sp2_start(zq_ctx *ctx, const Sp2Bufs &b, const double *dF, int n, int nocc, int *state, const int *skip,
+// nunset: steps of the one-XCD form, 0 for the others.
+void sp2_start(zq_ctx *ctx, const Sp2Bufs &b, const double *dF, int n, int nocc, int *state, int nunset, const int *skip,
                int track) {
   hipLaunchKernelGGL(k_gershgorin, dim3(kGershBlocks), dim3(256), 0, ctx->stream, dF, n, b.scal, skip, track, nocc, b.est,
                      b.ref, b.gpart, b.gcount);
   hipLaunchKernelGGL(k_sp2_init, dim3(b.ntiles), dim3(64), 0, ctx->stream, dF, n, b.m, b.scal, b.X, b.part, state, b.sync,
-                     skip);
+                     nunset, skip);
 }
 
 void sp2_step(zq_ctx *ctx, const Sp2Bufs &b, int k, int nocc, double tol, int *state, const int *skip) {
@@ -696,14 +698,15 @@ int zq_sp2_enqueue(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, i
   if (nsteps < 1 || nsteps > kSp2MaxSteps) return zq_fail(ctx, ZQ_ERR_INVALID, "SP2 step budget out of range");
   if (track < 0 || track > 2) return zq_fail(ctx, ZQ_ERR_INVALID, "SP2 fold tracking mode out of range");
   Sp2Bufs b;
-  if (int rc = sp2_bufs(ctx, n, n <= kSp2HomeMax ? kSp2MaxSteps + 1 : 2, b)) return rc;
+  const bool home = n <= kSp2HomeMax;
+  if (int rc = sp2_bufs(ctx, n, home ? kSp2MaxSteps + 1 : 2, b)) return rc;
   zq_prof_begin(ctx, "scf_sp2");
-  sp2_start(ctx, b, dF, n, nocc, state6, skip, track);
+  sp2_start(ctx, b, dF, n, nocc, state6, home ? nsteps : 0, skip, track);
   double *est = track ? b.est : nullptr;
   // about kSp2TilesPerGroup tiles per workgroup and step: fewer workgroups hand each step over with fewer
   // release fences, at the cost of more tiles per workgroup on the step's critical path
   const int groups = std::max(1, (b.ntiles + kSp2TilesPerGroup - 1) / kSp2TilesPerGroup);
-  if (b.m <= kSp2HomeMax)
+  if (home)
     hipLaunchKernelGGL(k_sp2_home, dim3(8 * b.ntiles), dim3(256), 0, ctx->stream, b.X, b.mm, b.m, nocc, b.part, b.sync, state6,
                        nsteps, tol, skip, est, ctx->turn & 7);
   else if (b.m <= 256)
@@ -729,7 +732,7 @@ int zq_sp2_density(zq_ctx *ctx, const double *dF, int n, int nocc, double tol, i
   auto *state = (int *)zq_scratch(ctx, "sp2_state", 6 * sizeof(int));
   if (!state) return zq_fail(ctx, ZQ_ERR_OOM, "SP2 buffers");
   zq_prof_begin(ctx, "scf_sp2");
-  sp2_start(ctx, b, dF, n, nocc, state, nullptr, 0);
+  sp2_start(ctx, b, dF, n, nocc, state, 0, nullptr, 0);
   int launched = 0, h[2] = {0, 0}, fin = 0;
   int next_check = std::max(4, std::min(max_steps, *steps_hint + 3));
   while (true) {
