@@ -185,3 +185,25 @@ def test_serve_k1_to_10_under_the_hbm_budget():
         assert abs(r["E_mp2"] - ref[r["key"]]) < 1e-6, (r["key"], r["E_mp2"] - ref[r["key"]])
     worst = max(abs(r["E_mp2"] - ref[r["key"]]) for r in rec)
     print(f"served {len(rec)} requests, max |dE_MP2| vs oracle = {worst:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("n", [7, 64, 70, 104, 150, 168])
+def test_slot_reserve_covers_a_request(n):
+    """What the server reserves for a slot is at least what a context holds after a request of that size: a mixed SCF on
+    a shared set, then MP2 of its orbitals in every precision the server runs."""
+    from zinq_amd import hip, serve
+    o = max(1, n // 5)
+    rng = np.random.default_rng(n)
+    npair = n * (n + 1) // 2
+    Q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+    H = (Q * np.concatenate([np.linspace(-20.0, -2.0, o), np.linspace(0.5, 4.0, n - o)])) @ Q.T
+    s = hip.EriSet(np.zeros(npair * (npair + 1) // 2), n, 0, True)
+    for precision, size in (("fp32c", 4), ("fp64", 8)):
+        with hip.Context(0) as c:
+            c.attach(s)
+            c.scf(0.5 * (H + H.T), np.eye(n), 0.0, o, device=True, fock_precision="fp32", threshold=1e-6)
+            c.mp2_resident(o, precision)
+            held, reserve = c.device_bytes(), serve.scratch_bytes(n, o, size)
+            print(f"n={n} {precision}: held {held / 1e6:.2f} MB, reserved {reserve / 1e6:.2f} MB", flush=True)
+            assert held <= reserve
+    s.close()

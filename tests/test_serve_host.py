@@ -146,3 +146,15 @@ def test_budget_below_the_slot_reserve_is_refused(monkeypatch):
     monkeypatch.setattr(sv, "hip", _fake_hip([0], []))
     with pytest.raises(MemoryError):
         sv.Server(mols, slots=4, hbm_budget=sv.scratch_bytes(72, 9, 4))
+
+
+def test_slot_reserve_counts_the_sp2_iterates():
+    """Up to n = 160 a context keeps an SP2 iterate for each of the 128 steps and the start: beyond the records, the
+    transform and 64 n^2 doubles for the rest."""
+    from zinq_amd import hip
+    for n in (65, 96, 150, 160):
+        o, m, npd = n // 5, (n + 15) // 16 * 16, (n + 7) // 8 * 8
+        Nb, v = npd // 8 * (npd // 8 + 1) // 2, n - o
+        transform = 4 * (Nb * 64 * o * npd + o * o * npd * npd + o * o * npd * v + o * o * v * v)
+        rest = sv.scratch_bytes(n, o, 4) - hip.jk_record_count(n) * 512 - transform
+        assert rest >= 8 * (129 * m * m + 64 * n * n), n

@@ -29,14 +29,18 @@ def eri_set_bytes(n, with_fp32):
 
 
 def scratch_bytes(n, o, transform_bytes=4):
-    """Transient device memory of one request: the J/K records of the molecule's plan (64 doubles each)
-    and the OVOV intermediates X, Y, W, OUT of the transform (element size transform_bytes)."""
+    """Transient device memory of one request: the J/K records of the molecule's plan (64 doubles each), the
+    OVOV intermediates X, Y, W, OUT of the transform (element size transform_bytes), the SP2 iterates on the
+    padded grid (one for each of the 128 steps and the start at n = 65 .. 160, else two at most) and the SCF's matrices
+    and small buffers."""
     nb = (n + 7) // 8
     npd, Nb = nb * 8, nb * (nb + 1) // 2
     v = n - o
     records = hip.jk_record_count(n) * 64 * 8
     tr = (Nb * 64 * o * npd + o * o * npd * npd + o * o * npd * v + o * o * v * v) * transform_bytes
-    return records + tr + 64 * n * n * 8
+    m = (n + 15) // 16 * 16
+    sp2 = (129 if 64 < n <= 160 else 2) * m * m * 8
+    return records + tr + sp2 + 64 * n * n * 8 + (1 << 16)
 
 
 class Molecule:
