@@ -83,7 +83,7 @@ void *zq_pinned(zq_ctx *ctx, const std::string &name, size_t bytes) {
   if (b.ptr) (void)hipHostFree(b.ptr);
   b.ptr = nullptr;
   b.bytes = 0;
-  if (hipHostMalloc(&b.ptr, std::max<size_t>(bytes, 256), hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&b.ptr, std::max<size_t>(bytes, 256), hipHostMallocCoherent) != hipSuccess) {
     b.ptr = nullptr;
     (void)hipGetLastError();
     return nullptr;
@@ -135,7 +135,7 @@ int ZqStage::take(zq_ctx *c, size_t cnt) {
       p.kept -= want;
     }
   }
-  if (!ptr && hipHostMalloc(&ptr, want, hipHostMallocPortable) != hipSuccess) {
+  if (!ptr && hipHostMalloc(&ptr, want, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
     (void)hipGetLastError();
     return zq_fail(c, ZQ_ERR_OOM, "pinned host buffer");
   }

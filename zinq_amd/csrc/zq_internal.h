@@ -143,7 +143,7 @@ struct zq_ctx {
 
   // named scratch buffers (grow-only)
   std::map<std::string, DevBuf> scratch;
-  // named pinned host buffers (hipHostMalloc, grow-only) for asynchronous device-to-host reads
+  // named pinned host buffers (hipHostMalloc, coherent, grow-only) that kernels write and the host reads meanwhile
   std::map<std::string, DevBuf> pinned;
 
   // profiling
@@ -198,7 +198,9 @@ void *zq_pinned(zq_ctx *ctx, const std::string &name, size_t bytes);
 // staging and costs 20 us at 5 KB, 125 us at 300 KB, and 2-D copies one of these per few rows.  So they
 // are copied to or from pinned buffers here, which kernels read and write in place over the link (55 GB/s).
 //
-// ZqStage: a pinned buffer for the length of one call, and its device address.  The buffers come from a pool of
+// ZqStage: a pinned buffer for the length of one call, and its device address.  The memory is asked for as coherent,
+// not left to the runtime's default, and what the host writes while a kernel reads the buffer (zq_fock_jk) starts on a
+// cache line of its own.  The buffers come from a pool of
 // the process, because the host's first touch of pinned pages costs 0.4 ms per MB: a new context takes pages
 // that an earlier call has touched.  The pool keeps at most 64 MB and is emptied with the last context.  A
 // buffer goes back when its holder has waited for the stream (done()); without that (an error return) the

@@ -709,17 +709,18 @@ extern "C" int zq_fock_jk(zq_ctx *ctx, const double *H, const double *P, double 
   if (!ctx->eri) return zq_fail(ctx, ZQ_ERR_STATE, "zq_fock_jk: no ERIs loaded");
   ZQ_TRY(ctx, hipSetDevice(ctx->device));
   const int n = ctx->n, np = ctx->npad;
-  const size_t nn = size_t(n) * n;
+  const size_t nn = size_t(n) * n, line = 32;  // H is written while P is read: 256 bytes apart at least
+  const size_t h = (nn + line - 1) / line * line, f = 2 * h;
   ZqStage st;
-  if (int rc = st.take(ctx, 3 * nn)) return rc;
+  if (int rc = st.take(ctx, f + nn)) return rc;
   std::memcpy(st.host, P, nn * sizeof(double));
   zq_pad(ctx, st.dev, 1, n, np, ctx->d_P);
   if (int rc = zq_jk_records_device(ctx, ctx->d_P, x_exch, nullptr, false)) return rc;
-  std::memcpy(st.host + nn, H, nn * sizeof(double));
-  if (int rc = zq_jk_reduce_device(ctx, st.dev + nn, st.dev + 2 * nn, nullptr, nullptr)) return rc;
+  std::memcpy(st.host + h, H, nn * sizeof(double));
+  if (int rc = zq_jk_reduce_device(ctx, st.dev + h, st.dev + f, nullptr, nullptr)) return rc;
   ZQ_TRY(ctx, hipStreamSynchronize(ctx->stream));
   st.done();
-  std::memcpy(F_out, st.host + 2 * nn, nn * sizeof(double));
+  std::memcpy(F_out, st.host + f, nn * sizeof(double));
   return ZQ_OK;
 }
 
