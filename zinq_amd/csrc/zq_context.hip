@@ -150,11 +150,13 @@ ZqStage::~ZqStage() {
   PinPool &p = pin_pool();
   {
     std::lock_guard<std::mutex> lock(p.mu);
-    if (p.kept + bytes <= kPinKeep && p.users > 0) {
-      p.free.emplace(bytes, host);
-      p.kept += bytes;
-      return;
-    }
+    if (p.kept + bytes <= kPinKeep && p.users > 0) try {
+        p.free.emplace(bytes, host);
+        p.kept += bytes;
+        return;
+      } catch (...) {
+        // no memory for the pool's entry: given back instead
+      }
   }
   (void)hipHostFree(host);
 }
