@@ -38,10 +38,10 @@ using namespace zqs;
 
 namespace {
 
-constexpr int kMaxN = 96;
+constexpr int kMaxN = kZqBatchMaxN;
 constexpr int kHist = 8;
-constexpr int kMats = 10;
-enum { M_H, M_F, M_P, M_S, M_X, M_XT, M_W, M_T, M_FP, M_FPR };
+constexpr int kMats = 9;
+enum { M_H, M_F, M_P, M_S, M_X, M_XT, M_W, M_T, M_FPR };
 // matrices of mp x mp in a molecule's workspace: the above, the DIIS history of F and of the error, and the
 // two buffers of the SP2 fold reference
 constexpr int kWsMats = kMats + 2 * kHist + 2;

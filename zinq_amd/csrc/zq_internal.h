@@ -238,6 +238,8 @@ int zq_eri32(zq_ctx *ctx);  // zq_jk.hip: FP32 copy of the resident quartets, ma
 void zq_narrow_eri(hipStream_t stream, const double *eri, size_t cnt, float *out);  // zq_jk.hip
 // MP2 correlation energy of the resident ERIs (zq_transform.hip); C and e are host arrays.
 int zq_mp2_device(zq_ctx *ctx, const double *C, const double *e, int nocc, int precision, double *e_corr);
+// Largest molecule of a batch.
+constexpr int kZqBatchMaxN = 96;
 // One molecule of a grouped MP2: its resident quartets (and their FP32 copy, for the FP32 forms), size,
 // doubly occupied count, and device C (n x n, row-major, columns = MOs) and orbital energies e (n).
 struct ZqGroupMol {
@@ -246,7 +248,7 @@ struct ZqGroupMol {
   int n, nocc;
   const double *C, *e;
 };
-// Closed-shell MP2 correlation energies of many molecules, one launch per transform stage for all of
+// Closed-shell MP2 correlation energies of many molecules (n <= kZqBatchMaxN), one launch per transform stage for all of
 // them, each molecule's result bitwise that of zq_mp2 (zq_transform.hip).  precision: FP64, FP32 or
 // FP32C.  ws / ws_bytes: the caller's grow-only device workspace (allocated here when too small, under
 // the caller's gate).  e_corr: host array of mols.size().  On error the reason is in err.

@@ -1747,10 +1747,7 @@ int group_run(hipStream_t stream, const std::vector<ZqGroupMol> &mols, void **ws
       J.out = d_out + k;
       const GemmArgs<T> &g2 = J.g[0] = q2_args(J.X, J.c2, Y, J.np, J.o, J.o, true);
       constexpr bool wide = sizeof(T) == 4;
-      if (wide && q34_tiles<T>(J.np)) {  // a molecule of a group takes the form it takes alone
-        err = "grouped MP2: molecule above the register forms' size";
-        return ZQ_ERR_INVALID;
-      }
+      static_assert(!wide || !q34_tiles<T>(kZqBatchMaxN), "a molecule of a group takes the form it takes alone");
       const GemmArgs<T> &g3 = J.g[1] = wide ? q3_args<T>(Y, J.c3, W, J.np, J.o, J.v, true) : q3_tile_args<T>(Y, J.c3, W, J.np, J.o, J.v, true);
       const GemmArgs<T> &g4 = J.g[2] = wide ? q4_args<T>(W, J.c3, J.O, J.np, J.v, J.v) : q4_tile_args<T>(W, J.c3, J.O, J.np, J.v, J.v);
       constexpr int cols = wide ? 128 : 64;
