@@ -220,7 +220,9 @@ struct ZqStage {
   bool idle = false;
 };
 void zq_stage_pool_users(int change);  // contexts alive: +1 / -1
-// Largest array (doubles) that is staged whole: 8 MB.  Larger ones take the runtime's copies.
+// Largest array (doubles) that zq_fock_jk_multi, zq_eigh and zq_ao2mo_pp stage: 8 MB.  Larger ones take the runtime's
+// copies.  A Fock build's, an SCF's and a transform's matrices are staged at any size: three of the largest n whose
+// ERIs fit a card (736) are 13 MB.
 constexpr size_t kZqStageMax = size_t(1) << 20;
 // cnt doubles from the device into the caller's array, in order on ctx's stream, which is idle on return.
 int zq_read_back(zq_ctx *ctx, const double *src, double *out, size_t cnt);

@@ -131,7 +131,8 @@ __device__ inline double sum8_scatter_high(const double (&v)[8], int lane) {
 // bound makes them return 0 without a fetch.
 // Cross-wave sums (K[p,s], K[q,s] at the end of a bs run, J[p,q] at the end of the item) go through
 // LDS in a fixed order.
-// Bound by memory for long items.  Against loads of P in the loop, a conditional prefetch and sets copied along, which
+// Long items are bound by neither memory nor arithmetic alone but by how far the two overlap: n = 192 309 us, its loads
+// alone 220, its arithmetic alone 160, on two waves per SIMD (VALU 25 - 28 % busy).  Against loads of P in the loop, a conditional prefetch and sets copied along, which
 // together waited for every load of a step within it (n = 192: 4.2 TB/s): n = 192 322 -> 309 us, n = 144 104 -> 97, six
 // densities at n = 93 180 -> 131, 96 molecules n <= 72 197 -> 184, n = 96 in FP32 28.6 -> 18.8, n = 72 14.5 -> 12.6.
 // GROUP: the item's molecule selects the quartets, P and its leading dimension from mols[], and the

@@ -533,9 +533,11 @@ int density_async(Dev &d, const double *A, int nocc, double factor, int nsteps, 
   return ZQ_OK;
 }
 
-// The one-workgroup form takes molecules up to n = 64.  A whole run, multi-launch / one workgroup, ms: n = 7
-// 0.94 / 0.50, n = 24 2.00 / 1.22, n = 48 2.41 / 1.94, n = 56 2.15 / 2.16.  Beyond that the FP64 matrix rate of
-// one compute unit costs more than the launches: n = 72 3.10 / 4.16, n = 96 3.94 / 6.76.
+// The one-workgroup form takes molecules up to n = 64, where its form of four tiles a row ends.  A whole run of 5 to
+// 7 iterations, multi-launch / one workgroup, ms: n = 16 0.95 / 0.65, 24 1.03 / 0.71, 32 1.17 / 0.87, 40 1.28 / 1.04,
+// 48 1.39 / 1.16; at four tiles the two are even: 49 1.43 / 1.42, 56 1.47 / 1.46, 60 1.54 / 1.54, 64 1.66 / 1.69 (17
+// iterations at n = 63 3.20 / 3.29).  Five tiles lose, the FP64 matrix rate of one compute unit costing more than the
+// launches: n = 65 1.60 / 1.84, 72 1.78 / 2.05, 80 1.87 / 2.21.
 constexpr int kStepMaxTiles = 4;
 bool step_fits(int n) { return n <= 16 * kStepMaxTiles; }
 

@@ -371,9 +371,9 @@ __device__ inline bool lu_solve(int n, double *A, double &b) {
 // operands, then written over one of them.  SP2 ping-pongs between the buffers with one barrier per step and
 // forms the upper tiles only.
 //
-// Every sum is taken in the order of the multi-launch form (zq_scf_dev.hip, zq_dense.hip), so F', D, P and
-// the extrapolated Fock matrix are bitwise that form's: the signs of the orbitals of a symmetric molecule
-// hang on the last bits of F'.  Only rms(dP), which is compared with the threshold, is summed differently.
+// The sums of F', D and P are taken in the order of the multi-launch form (zq_scf_dev.hip, zq_dense.hip).  The DIIS
+// dot products and rms(dP) are not (that form sums both tile by tile), so the two forms agree to rounding, not to the
+// bit.  The order here stays as it is: the signs of the orbitals of a symmetric molecule hang on the last bits of F'.
 //
 // Matrices in global memory are n x n with a leading dimension each, or n n contiguous (history, reference).
 constexpr int kStepTiles = 6;  // largest T that fits: 2 x 96 x 98 doubles of LDS
@@ -577,7 +577,7 @@ struct StepBody {
   // as a halving tree, the nb (at most 36) trees by wave_sum.  er: err_new, n n contiguous in LDS; tree: nb m
   // doubles of LDS.  A wave takes (tree, entry) pairs, four of them in flight.
   static __device__ void diis_dots(StepShared &sh, const double *er, double *tree, const double *Eh, int nn, int m) {
-#pragma clang fp contract(off)  // each product is rounded before its tree, as the multi-launch form stores it
+#pragma clang fp contract(off)  // the trees sum rounded products, whatever is inlined around them
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nb = (nn + 255) / 256, tot = nb * m;
     for (int i0 = wave; i0 < tot; i0 += 4 * NW) {
       double e[4][4];

@@ -168,7 +168,8 @@ __device__ inline E q1_val(const E *__restrict__ eri, const Q1Src &s, int K, int
 // block.  Loads are unconditional (indices past the last block are clamped: their copies land in the buffer no
 // later step reads, and the A operands past m1 take column m1 - 1, which only reaches output rows that are never
 // stored).  n = 192, o = 40, FP64: 1607 -> 1470 us (MFMA peak of the executed tiles 940); n = 101, o = 20, FP32C:
-// 106 -> 94; a group of 96 molecules n <= 72: 636 -> 546.
+// 106 -> 94; a group of 96 molecules n <= 72: 636 -> 546.  FP32C with three row tiles a wave loses by it: n = 192, o = 40
+// 1200 -> 1223 (its whole MP2 gains through the later quarters).
 // The body takes the workgroup's coordinates (bx, by, bz) as arguments, so that a grouped launch over
 // many molecules can run it for each molecule's share of the grid.
 struct Q1Slots {
